@@ -97,7 +97,7 @@ int lookup(const char* name, hipFunction_t* fn) {
     return fail(AOTO_ERR_NO_CODE_OBJECT, "no gfx950 code object loaded on device %d", device);
   auto& fns = it->second.functions;
   auto found = fns.find(name);
-  if (found != fns.end()) {
+  if (found != fns.end() && found->second != nullptr) {
     *fn = found->second;
     return AOTO_OK;
   }
@@ -106,9 +106,34 @@ int lookup(const char* name, hipFunction_t* fn) {
   if (err != hipSuccess)
     return fail(AOTO_ERR_NO_CODE_OBJECT, "kernel %s not found in the code object: %s", name,
                 hipGetErrorString(err));
-  fns.emplace(name, f);
+  fns[name] = f;
   *fn = f;
   return AOTO_OK;
+}
+
+// Whether the code object installed on the current device has a kernel. A code
+// object stored in an artifact by an earlier build holds that build's kernels
+// only: a launcher whose fast path is a newer symbol asks first and otherwise
+// launches what the stored plan was built with.
+bool has_kernel(const char* name) {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) {
+    hipGetLastError();
+    return false;
+  }
+  std::lock_guard<std::mutex> lock(g_mutex);
+  auto it = g_modules.find(device);
+  if (it == g_modules.end() || it->second.module == nullptr) return false;
+  auto& fns = it->second.functions;
+  auto found = fns.find(name);
+  if (found != fns.end()) return found->second != nullptr;
+  hipFunction_t f = nullptr;
+  if (hipModuleGetFunction(&f, it->second.module, name) != hipSuccess) {
+    hipGetLastError();  // an absent optional kernel is not an error to report later
+    f = nullptr;
+  }
+  fns.emplace(name, f);
+  return f != nullptr;
 }
 
 // Kernel symbols launched by this thread while recording is on (aoto_hip_trace_launches),
@@ -431,6 +456,34 @@ int aoto_hip_code_object_loaded(void) {
   return (it != g_modules.end() && it->second.module != nullptr) ? 1 : 0;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The packers' kernel: the coalesced form where a group is a power-of-two count of
+// 8-weight units that fits one wave (groups of 8 to 512) and the base allows 16-byte
+// loads and whole-word stores; other groups and bases keep one thread per group.
+int launch_quantize(int bits, const void* weight, int weight_is_f32, int rows, int inner, int group,
+                    int32_t* packed, void* scales_bf16, float* scales_f32, void* stream) {
+  const char* wide = bits == 4 ? "aoto_w4_quantize_units" : "aoto_w8_quantize_units";
+  const int lanes = group / 8;
+  if (group % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && aligned16(weight) && aligned8(packed) &&
+      has_kernel(wide)) {
+    const long long units = (long long)rows * (inner / 8);
+    int shift = 0;
+    while ((1 << shift) < lanes) ++shift;
+    return launch(wide, dim3(blocks_for(units, 1024)), dim3(256), 0, stream, weight, weight_is_f32, shift, units,
+                  packed, scales_bf16, scales_f32);
+  }
+  const long long tasks = (long long)rows * (inner / group);
+  return launch(bits == 4 ? "aoto_w4_quantize" : "aoto_w8_quantize", dim3(blocks_for(tasks, 256)), dim3(256), 0,
+                stream, weight, weight_is_f32, rows, inner, group, packed, scales_bf16, scales_f32);
+}
+
+}  // namespace
+
+extern "C" {
+
 int aoto_hip_w4_quantize(const void* weight, int weight_is_f32, int rows, int inner, int group,
                          int32_t* packed, void* scales_bf16, float* scales_f32, void* stream) {
   if (!weight || !packed || !scales_bf16) return fail(AOTO_ERR_ARGUMENT, "w4_quantize: null pointer");
@@ -438,10 +491,7 @@ int aoto_hip_w4_quantize(const void* weight, int weight_is_f32, int rows, int in
   if (group <= 0 || group % 8 != 0 || inner % group != 0)
     return fail(AOTO_ERR_ARGUMENT, "w4_quantize: group %d must be a positive multiple of 8 dividing %d",
                 group, inner);
-  long long tasks = (long long)rows * (inner / group);
-  unsigned blocks = (unsigned)((tasks + 255) / 256);
-  return launch("aoto_w4_quantize", dim3(blocks), dim3(256), 0, stream, weight, weight_is_f32, rows, inner,
-                group, packed, scales_bf16, scales_f32);
+  return launch_quantize(4, weight, weight_is_f32, rows, inner, group, packed, scales_bf16, scales_f32, stream);
 }
 
 int aoto_hip_w4_dequantize(const int32_t* packed, const void* scales, int rows, int inner, int group,
@@ -1066,9 +1116,7 @@ int aoto_hip_w8_quantize(const void* weight, int weight_is_f32, int rows, int in
   if (group <= 0 || group % 4 != 0 || inner % group != 0)
     return fail(AOTO_ERR_ARGUMENT, "w8_quantize: group %d must be a positive multiple of 4 dividing %d",
                 group, inner);
-  const long long tasks = (long long)rows * (inner / group);
-  return launch("aoto_w8_quantize", dim3(blocks_for(tasks, 256)), dim3(256), 0, stream, weight, weight_is_f32,
-                rows, inner, group, packed, scales_bf16, scales_f32);
+  return launch_quantize(8, weight, weight_is_f32, rows, inner, group, packed, scales_bf16, scales_f32, stream);
 }
 
 int aoto_hip_w8_dequantize(const int32_t* packed, const void* scales, int rows, int inner, int group,

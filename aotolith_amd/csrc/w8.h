@@ -16,7 +16,8 @@
 
 namespace aoto {
 
-// One thread per (row, group). `src_f32` selects an f32 source, else bf16.
+// One thread per (row, group), for groups or bases the coalesced packer does not take.
+// `src_f32` selects an f32 source, else bf16.
 extern "C" __global__ __launch_bounds__(256) void aoto_w8_quantize(
     const void* __restrict__ src, int src_f32, int rows, int inner, int group,
     int32_t* __restrict__ packed, uint16_t* __restrict__ scales_bf16, float* __restrict__ scales_f32) {

@@ -363,3 +363,30 @@ def test_gemv_finish_refuses_other_shapes():
                            out=torch.empty(20000, dtype=torch.bfloat16, device="cuda"),
                            token_out=torch.zeros((1,), dtype=torch.int64, device="cuda"),
                            hidden_out=torch.empty(896, dtype=torch.bfloat16, device="cuda"))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("source", ["bf16", "f32"])
+@pytest.mark.parametrize("n,k,group", [(1, 8, 8), (257, 8, 8), (129, 64, 16), (33, 96, 32), (17, 1024, 64),
+                                       (9, 1280, 256), (5, 1536, 512), (2, 4096, 1024), (7, 240, 24)])
+def test_packers_at_the_edges_of_their_units(n, k, group, source, bits):
+    """Unit counts around a block's 1024, one to 64 lanes a group, groups the coalesced form leaves out
+    (over 512, not a power of two), zero, infinite and NaN groups, and a base that is not 16-byte aligned."""
+
+    from oracle.quant import pack_weight_bits_bf16
+
+    rng = np.random.default_rng(n + k + group)
+    weight = bf16_normal(rng, (n, k), 0.02)
+    weight[0, :group] = 0.0
+    ref_packed, ref_scales = pack_weight_bits_bf16(weight, group, bits)
+    tensor = to_gpu_bf16(weight) if source == "bf16" else torch.from_numpy(weight).cuda()
+    shifted = torch.empty(n * k + 1, dtype=tensor.dtype, device="cuda")[1:].view(n, k).copy_(tensor)
+    for given in (tensor, shifted):
+        packed, scales = _ops().quantize(given, group, bits)
+        np.testing.assert_array_equal(packed.cpu().numpy(), ref_packed)
+        np.testing.assert_array_equal(bf16_bits_of(scales), ref_scales)
+    # values no weight should hold: both forms still agree, bit for bit
+    tensor.view(-1)[-1], tensor.view(-1)[-2] = float("nan"), float("inf")
+    shifted.copy_(tensor)
+    for got, want in zip(_ops().quantize(tensor, group, bits), _ops().quantize(shifted, group, bits)):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
