@@ -42,6 +42,7 @@ SIGNATURES: dict[str, tuple] = {
     "aoto_hip_hold_graphs": (_c_int,),
     "aoto_hip_graph_holds": (),
     "aoto_hip_code_object_loaded": (),
+    "aoto_hip_has_kernel": (ctypes.c_char_p,),
     "aoto_hip_w4_quantize": (_p, _c_int, _c_int, _c_int, _c_int, _p, _p, _p, _p),
     "aoto_hip_w4_dequantize": (_p, _p, _c_int, _c_int, _c_int, _p, _p),
     "aoto_hip_w4_gemv": (

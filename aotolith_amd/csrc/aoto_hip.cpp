@@ -484,6 +484,8 @@ int launch_quantize(int bits, const void* weight, int weight_is_f32, int rows, i
 
 extern "C" {
 
+int aoto_hip_has_kernel(const char* name) { return name != nullptr && has_kernel(name) ? 1 : 0; }
+
 int aoto_hip_w4_quantize(const void* weight, int weight_is_f32, int rows, int inner, int group,
                          int32_t* packed, void* scales_bf16, float* scales_f32, void* stream) {
   if (!weight || !packed || !scales_bf16) return fail(AOTO_ERR_ARGUMENT, "w4_quantize: null pointer");
@@ -1584,6 +1586,28 @@ int broadcast_operand(const char* what, const char* name, const aoto_tensor* t, 
   return AOTO_OK;
 }
 
+// The matrix product's instance: how its operands can be read, its tile and its k-groups.
+// 128 x 128 tiles where they fill the chip (256 blocks: twice the products per LDS byte);
+// else 64 x 64, with four k-groups a block up to 256 tiles and two up to 512, where a
+// step's latency and not the MFMA pipe is the bound - a k-group needs a k-step or two.
+void generic_gemm_plan(const aoto::GemmArgs& g, char* name, size_t size, int* tiles, int* kgroups) {
+  const bool bf16 = g.a_dtype == AOTO_DT_BF16 && g.b_dtype == AOTO_DT_BF16;
+  const int elem = bf16 ? 2 : 4, chunk = 16 / elem;
+  const bool one_type = bf16 || (g.a_dtype == AOTO_DT_F32 && g.b_dtype == AOTO_DT_F32);
+  auto whole = [&](long long stride, long long extent) { return extent <= 1 || stride % chunk == 0; };
+  const bool a_rows = one_type && g.k > 0 && g.k % chunk == 0 && g.sa_k == 1 && aligned16(g.a) && whole(g.sa_m, g.m) &&
+                      whole(g.sa_b, g.batch);
+  const bool b_rows = g.sb_k == 1 && aligned16(g.b) && whole(g.sb_n, g.n) && whole(g.sb_b, g.batch);
+  const bool b_cols = g.sb_n == 1 && (bf16 ? g.n % 2 == 0 && g.sb_k % 2 == 0 && g.sb_b % 2 == 0 && aligned4(g.b)
+                                           : aligned4(g.b));
+  const char mode = a_rows && b_rows ? 'v' : a_rows && b_cols ? 'c' : 'a';
+  auto blocks = [&](long long side) { return (g.n + side - 1) / side * ((g.m + side - 1) / side) * g.batch; };
+  const long long steps = (g.k + 8 * chunk - 1) / (8 * chunk), small = blocks(64);
+  *tiles = blocks(128) >= 256 ? 2 : 1;
+  *kgroups = *tiles == 2 ? 1 : small <= 256 && steps >= 4 ? 4 : small <= 512 && steps >= 2 ? 2 : 1;
+  snprintf(name, size, "aoto_generic_gemm_%s_%c_t%dk%d", bf16 ? "bf16" : "f32", mode, *tiles, *kgroups);
+}
+
 unsigned grid_for(long long total) {
   long long blocks = (total + 255) / 256;
   if (blocks < 1) blocks = 1;
@@ -1749,6 +1773,15 @@ int aoto_hip_generic_matmul(const aoto_tensor* out, const aoto_tensor* a, const 
     g.sbias_n = o.strides[2];
   }
   if (B == 0 || M == 0 || N == 0) return AOTO_OK;
+  if (has_kernel("aoto_generic_gemm_f32_a_t1k1")) {
+    int tiles = 1, kgroups = 1;
+    char name[64];
+    generic_gemm_plan(g, name, sizeof(name), &tiles, &kgroups);
+    const unsigned side = 64u * tiles;
+    return launch(name, dim3((unsigned)((N + side - 1) / side), (unsigned)((M + side - 1) / side), (unsigned)B),
+                  dim3(256 * kgroups), 0, stream, g);
+  }
+  // (a code object stored by an earlier build: its one f32 FMA kernel)
   return launch("aoto_generic_gemm", dim3((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)B),
                 dim3(256), 0, stream, g);
 }

@@ -462,68 +462,6 @@ extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_reduce(Re
   }
 }
 
-// Batched strided GEMM: 64x64 output tile per block, k-steps of 16 staged in
-// LDS as f32, 4x4 outputs per thread, f32 FMA accumulation.
-extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_gemm(GemmArgs g) {
-  __shared__ float as[16][64 + 4];
-  __shared__ float bs[16][64 + 4];
-  const long long batch = blockIdx.z;
-  const long long m0 = (long long)blockIdx.y * 64, n0 = (long long)blockIdx.x * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float acc[4][4] = {};
-  for (long long k0 = 0; k0 < g.k; k0 += 16) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int e = threadIdx.x + t * kGenThreads;  // 0..1023
-      // A tile: 64 rows x 16 k (element e -> row e / 16, k e % 16)
-      const int ar = e >> 4, ak = e & 15;
-      const long long gm = m0 + ar, gk = k0 + ak;
-      float av = 0.f;
-      if (gm < g.m && gk < g.k)
-        av = (float)load_value(g.a, g.a_dtype, batch * g.sa_b + gm * g.sa_m + gk * g.sa_k);
-      as[ak][ar] = av;
-      // B tile: 16 k x 64 cols (element e -> k e / 64, col e % 64)
-      const int bk = e >> 6, bn = e & 63;
-      const long long gk2 = k0 + bk, gn = n0 + bn;
-      float bv = 0.f;
-      if (gk2 < g.k && gn < g.n)
-        bv = (float)load_value(g.b, g.b_dtype, batch * g.sb_b + gk2 * g.sb_k + gn * g.sb_n);
-      bs[bk][bn] = bv;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float av[4], bv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = as[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long long gm = m0 + ty * 4 + i;
-    if (gm >= g.m) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const long long gn = n0 + tx * 4 + j;
-      if (gn >= g.n) continue;
-      float v = acc[i][j];
-      if (g.alpha != 1.f) v *= g.alpha;
-      if (g.bias) {
-        const float b = (float)load_value(g.bias, g.bias_dtype, batch * g.sbias_b + gm * g.sbias_m + gn * g.sbias_n);
-        v = g.beta == 1.f ? v + b : v + g.beta * b;
-      }
-      store_float(g.c, g.c_dtype, batch * g.sc_b + gm * g.sc_m + gn * g.sc_n, v);
-    }
-  }
-}
-
 // Advanced indexing over the leading dims of a contiguous source; an index out
 // of [-size, size) sets *error and writes zeros.
 extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_index(IndexArgs a) {

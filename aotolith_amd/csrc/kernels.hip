@@ -10,6 +10,7 @@
 #include "w4_gemm_lds.h"
 #include "w8.h"
 #include "generic.h"
+#include "generic_gemm.h"
 #include "decode.h"
 #include "prefill.h"
 #include "flash_attention.h"
@@ -155,3 +156,11 @@ AOTO_FLASH_INSTANCE(128)
 AOTO_FLASH_INSTANCE_KG(64, 2, false, _k2_q64, 1, 2)
 AOTO_FLASH_INSTANCE_KG(64, 2, false, _k2_q32, 1, 1)
 AOTO_FLASH_INSTANCE_KG(128, 2, false, _k2_q64, 1, 2)
+
+// The graph plans' matrix products: {element type} x {operand loads} x {tile, k-groups}.
+AOTO_GENERIC_GEMM_MODE(bf16, uint16_t, v, aoto::kVec)
+AOTO_GENERIC_GEMM_MODE(bf16, uint16_t, c, aoto::kCols)
+AOTO_GENERIC_GEMM_MODE(bf16, uint16_t, a, aoto::kAny)
+AOTO_GENERIC_GEMM_MODE(f32, float, v, aoto::kVec)
+AOTO_GENERIC_GEMM_MODE(f32, float, c, aoto::kCols)
+AOTO_GENERIC_GEMM_MODE(f32, float, a, aoto::kAny)

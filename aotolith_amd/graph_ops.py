@@ -219,6 +219,10 @@ FAMILIES[RMS_NORM] = "rms_norm"
 KERNELS = {"elementwise": "aoto_generic_elementwise", "reduction": "aoto_generic_reduce",
            "matmul": "aoto_generic_gemm", "gather": "aoto_generic_index", "copy": "aoto_generic_copy",
            "fill": "aoto_generic_fill", "rms_norm": "aoto_generic_rms_norm", "attention": "aoto_generic_attention"}
+#: Families whose kernel an earlier build's code object does not have: the symbol that tells, and the
+#: names this build's selections record (a family prefix: the instance follows the operands' strides).
+NEWER = {"matmul": ("aoto_generic_gemm_f32_a_t1k1", "aoto_generic_gemm_*",
+                    "strided batched GEMM on the matrix cores, LDS-staged tiles, f32 accumulation")}
 REASONS = {
     "elementwise": "strided broadcasting elementwise kernel, f32 compute, one rounding to the output type",
     "reduction": "row reduction / scan over the (permuted) last dim, f32 or int64 accumulation",
@@ -276,14 +280,18 @@ class GraphRunner:
     # -- selection records --------------------------------------------------------
     def selections(self, device_name: str | None) -> tuple[KernelSelection, ...]:
         out = []
+        kernels, reasons = dict(KERNELS), dict(REASONS)
+        for family, (symbol, name, reason) in NEWER.items():
+            if _lib.library().aoto_hip_has_kernel(symbol.encode()):
+                kernels[family], reasons[family] = name, reason
         for node in self.graph.nodes:
             if node.is_view:
                 continue
             family = FAMILIES[node.op]
             out.append(KernelSelection(
                 op_index=len(out), op=node.op.split(".")[1] if node.op.startswith("aten.") else node.op,
-                output_id=node.name, implementation="hip_kernel", kind=family, reason=REASONS[family],
-                artifact_name=KERNELS[family], device_name=device_name, device_architecture=ARCHITECTURE,
+                output_id=node.name, implementation="hip_kernel", kind=family, reason=reasons[family],
+                artifact_name=kernels[family], device_name=device_name, device_architecture=ARCHITECTURE,
             ))
         return tuple(out)
 

@@ -81,6 +81,10 @@ int aoto_hip_unload_code_object(void);
 /* 1 when a module is installed on the current device, else 0. */
 int aoto_hip_code_object_loaded(void);
 
+/* 1 when the code object installed on the current device has this kernel. Plans loaded
+ * with an earlier build's code object launch the kernels it holds. */
+int aoto_hip_has_kernel(const char* name);
+
 /* Symmetric int4 group quantizer + packer, bit-exact with quantize.py:95-152 and
  * the bf16 scale cast of models/quantized.py:133-163 (pack_weight).
  * weight: [rows, inner] bf16 (weight_is_f32 == 0) or f32; group % 8 == 0 and

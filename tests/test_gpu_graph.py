@@ -196,3 +196,51 @@ def test_callable_artifact_round_trip(tmp_path):
     loaded = load_compiled_module(result.save(tmp_path / "indexing.aoto"))
     got = loaded.plan(*inputs)
     assert all(torch.equal(a.cpu(), b.cpu()) for a, b in zip(got, want))
+
+
+def _matmul_operand(gen, batch, rows, cols, dtype, layout):
+    """A [batch, rows, cols] operand: row-major, column-major, padded rows, or every other element."""
+
+    if layout == "rows":
+        return torch.randn(batch, rows, cols, generator=gen).to(dtype).cuda()
+    if layout == "cols":
+        return torch.randn(batch, cols, rows, generator=gen).to(dtype).cuda().transpose(1, 2)
+    if layout == "padded":
+        return torch.randn(batch, rows, cols + 3, generator=gen).to(dtype).cuda()[:, :, 1:cols + 1]
+    return torch.randn(batch, rows, 2 * cols, generator=gen).to(dtype).cuda()[:, :, ::2]
+
+
+@pytest.mark.parametrize("types", ["bf16", "f32", "mixed"])
+@pytest.mark.parametrize("layouts", [("rows", "cols"), ("rows", "rows"), ("cols", "rows"), ("padded", "cols"),
+                                     ("strided", "strided")])
+@pytest.mark.parametrize("batch,m,n,k", [(1, 1, 1, 1), (1, 4, 128, 64), (3, 65, 66, 40), (2, 63, 64, 512),
+                                         (1, 130, 192, 136), (1, 100, 77, 33), (1, 1030, 2050, 72), (5, 257, 130, 264)])
+def test_matmul_over_its_tiles_layouts_and_types(batch, m, n, k, layouts, types):
+    """Every operand loader, tile and k-group count of the matrix-core product, at their remainders, against 64-bit
+    products. Bound: K f32 additions of the absolute products, then one rounding to the output type."""
+
+    from aotolith_amd.graph_ops import launch_matmul
+
+    gen = torch.Generator().manual_seed(m * 7 + n * 3 + k)
+    a_type, b_type = {"bf16": (torch.bfloat16,) * 2, "f32": (torch.float32,) * 2,
+                      "mixed": (torch.float32, torch.bfloat16)}[types]
+    a = _matmul_operand(gen, batch, m, k, a_type, layouts[0])
+    b = _matmul_operand(gen, batch, k, n, b_type, layouts[1])
+    bias = torch.randn(n, generator=gen).to(b_type).cuda()
+    exact = a.double() @ b.double()
+    room = (k + 4) * 2.0 ** -24 * (a.double().abs() @ b.double().abs() + 1.0)
+    for out_type, eps in ((torch.float32, 2.0 ** -24), (torch.bfloat16, 2.0 ** -8)):
+        out = torch.full((batch, m, n), 7.0, dtype=out_type, device="cuda")
+        launch_matmul(out, a, b)
+        assert bool(((out.double() - exact).abs() <= room + eps * exact.abs()).all())
+        launch_matmul(out, a, b, bias, 0.5, 2.0)
+        want = 0.5 * exact + 2.0 * bias.double()
+        assert bool(((out.double() - want).abs() <= 2 * room + 2 ** -20 * want.abs() + eps * want.abs()).all())
+
+
+def test_matmul_with_no_reduction_is_its_bias():
+    from aotolith_amd.graph_ops import launch_matmul
+
+    out = torch.full((2, 3, 5), 7.0, device="cuda")
+    launch_matmul(out, torch.empty(2, 3, 0, device="cuda"), torch.empty(2, 0, 5, device="cuda"))
+    assert bool((out == 0).all())
