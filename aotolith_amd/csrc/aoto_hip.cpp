@@ -1608,6 +1608,22 @@ void generic_gemm_plan(const aoto::GemmArgs& g, char* name, size_t size, int* ti
   snprintf(name, size, "aoto_generic_gemm_%s_%c_t%dk%d", bf16 ? "bf16" : "f32", mode, *tiles, *kgroups);
 }
 
+// The matrix-core attention's instance for head sizes up to 128: bf16 products where q, k and v are all
+// bf16, f32 ones otherwise; 16-byte operand loads where every row is whole 16-byte chunks.
+void generic_attention_plan(const aoto::AttnArgs& a, char* name, size_t size) {
+  const bool bf16 = a.q_dtype == AOTO_DT_BF16 && a.k_dtype == AOTO_DT_BF16 && a.v_dtype == AOTO_DT_BF16;
+  const int chunk = bf16 ? 8 : 4;
+  auto rows = [&](const void* p, int dtype, const long long* strides, int dim) {
+    return dtype == (bf16 ? AOTO_DT_BF16 : AOTO_DT_F32) && aligned16(p) && strides[3] == 1 && dim % chunk == 0 &&
+           strides[0] % chunk == 0 && strides[1] % chunk == 0 && strides[2] % chunk == 0;
+  };
+  // (f32 values are read element by element in operand order whatever their layout)
+  const bool vec = rows(a.q, a.q_dtype, a.qs, a.d) && rows(a.k, a.k_dtype, a.ks, a.d) &&
+                   (!bf16 || rows(a.v, a.v_dtype, a.vs, a.dv));
+  snprintf(name, size, "aoto_generic_attention_%s_d%d_%c", bf16 ? "bf16" : "f32", a.d > 64 || a.dv > 64 ? 128 : 64,
+           vec ? 'v' : 'a');
+}
+
 unsigned grid_for(long long total) {
   long long blocks = (total + 255) / 256;
   if (blocks < 1) blocks = 1;
@@ -1972,6 +1988,11 @@ int aoto_hip_generic_attention(const aoto_tensor* out, const aoto_tensor* q, con
   }
   args.scale = scale;
   if (B == 0 || H == 0 || Lq == 0) return AOTO_OK;
+  if (D <= 128 && Dv <= 128 && has_kernel("aoto_generic_attention_f32_d64_a")) {
+    char name[64];
+    generic_attention_plan(args, name, sizeof(name));
+    return launch(name, dim3((unsigned)((Lq + 31) / 32), (unsigned)(B * H)), dim3(256), 0, stream, args);
+  }
   return launch("aoto_generic_attention", dim3((unsigned)Lq, (unsigned)(B * H)), dim3(256), 0, stream, args);
 }
 

@@ -50,6 +50,17 @@ AOTO_DEVICE long long load_int(const void* p, int dtype, long long off) {
   }
 }
 
+// A float element where the host has checked that the type is one of the two.
+AOTO_DEVICE float load_float(const void* p, int dtype, long long off) {
+  return dtype == AOTO_DT_F32 ? static_cast<const float*>(p)[off] : bf16_to_f32(static_cast<const uint16_t*>(p)[off]);
+}
+AOTO_DEVICE void store_float_type(void* p, int dtype, long long off, float v) {
+  if (dtype == AOTO_DT_F32)
+    static_cast<float*>(p)[off] = v;
+  else
+    static_cast<uint16_t*>(p)[off] = (uint16_t)f32_to_bf16(v);
+}
+
 // Store a float result (rounded once to the element type; float -> int truncates).
 AOTO_DEVICE void store_float(void* p, int dtype, long long off, float v) {
   switch (dtype) {
@@ -537,7 +548,7 @@ extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_rms_norm(
   }
 }
 
-// Scaled dot-product attention, one (batch, head, query row) per block:
+// Scaled dot-product attention for head sizes over 128, one (batch, head, query row) per block:
 // scores into LDS, f32 softmax, then each thread owns output columns. A bool
 // mask keeps True entries, a float mask is added; is_causal keeps j <= i
 // (aligned to the top-left, as torch's is_causal). A row with every key

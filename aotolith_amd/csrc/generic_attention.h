@@ -1,0 +1,374 @@
+// The graph plans' scaled-dot-product attention on the matrix cores.
+//
+// out[b][h][i] = softmax_j(scale * q_i . k_j + mask) v_j, f32 scores and softmax: a bool mask keeps
+// True entries, a float mask is added, is_causal keeps j <= i (aligned to the top-left, as torch's), a
+// row with every key masked gives zeros, and a key whose probability is zero contributes nothing,
+// whatever its value holds - the semantics of aoto_generic_attention, which keeps head sizes over 128.
+//
+// A block owns 32 queries of one head; its four waves take the key tiles in turn, each with its own
+// running softmax (no barrier inside the loop), and combine through LDS at the end. Per wave and tile:
+//   S^T [keys x 32 queries] = K . Q^T    K straight from global memory in operand order, Q in registers
+//   O^T [d x 32 queries] += V^T . P^T    P from S^T's accumulators, lane l holding query l % 32
+// bf16 operands: 64-key tiles on v_mfma_f32_32x32x16_bf16, V staged row-major in the wave's LDS and read
+// with the transposing LDS reads; P stays at f32 precision: it enters as three bf16 terms (8 + 8 + 8
+// bits: p = hi + mid + lo exactly, short of the f32's underflow), three products into the one f32 sum.
+// f32 (and mixed) operands: 32-key tiles on v_mfma_f32_32x32x2_f32, V read in operand order.
+//
+// Values that are not finite: 0 * inf would poison every query through the product, so they enter it as
+// zeros, and a tile that holds any runs a second pass (special_values) that gives +-inf / NaN to the
+// queries whose probability of such a key is not zero.
+//
+// Bound: latency (two tiles a wave at 512 keys), then the MFMA pipe. 14 heads of 64, 512 tokens,
+// causal, bf16: 881 us with one block per query row and scalar dots (every score a 64-step chain of
+// typed loads) -> MEAS us.
+#pragma once
+
+#include "aoto_hip.h"
+#include "common.h"
+#include "flash_attention.h"
+#include "generic.h"
+#include "generic_args.h"
+
+namespace aoto {
+
+constexpr int kGenAttnQueries = 32;
+constexpr int kGenAttnWaves = 4;
+
+// Order of one wave's own LDS writes and reads (the hardware keeps it; this keeps the compiler to it).
+AOTO_DEVICE void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+AOTO_DEVICE bool not_finite_bf16(uint32_t bits16) { return (bits16 & 0x7F80u) == 0x7F80u; }
+AOTO_DEVICE bool not_finite_f32(float v) { return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u; }
+// The class of a value that is not finite: 0 +inf, 1 -inf, 2 NaN.
+AOTO_DEVICE int special_class(float v) { return v != v ? 2 : v < 0.f ? 1 : 0; }
+
+// One 16-byte operand chunk (8 bf16 or 4 f32) at `off` along stride `step`, elements from `count` on zero.
+template <bool F32, bool VEC>
+AOTO_DEVICE uint4 attn_chunk(const void* p, int dtype, long long off, long long step, int count) {
+  if (VEC) {
+    // whole chunks only (the host checks the head sizes): past the row's end nothing is read
+    if (count <= 0) return make_uint4(0u, 0u, 0u, 0u);
+    return F32 ? *reinterpret_cast<const uint4*>(static_cast<const float*>(p) + off)
+               : *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + off);
+  }
+  uint32_t w[4] = {0u, 0u, 0u, 0u};
+  constexpr int E = F32 ? 4 : 8;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (e < count) {
+      if (F32)
+        w[e & 3] = __float_as_uint(load_float(p, dtype, off + e * step));
+      else
+        w[e >> 1] |= (uint32_t) static_cast<const uint16_t*>(p)[off + e * step] << (16 * (e & 1));
+    }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+template <bool F32, int D, bool VEC>
+__device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
+  constexpr int E = F32 ? 4 : 8;          // elements of a 16-byte chunk
+  constexpr int KT = F32 ? 1 : 2;         // 32-key parts of a tile
+  constexpr int BK = 32 * KT;
+  constexpr int S = D / (2 * E);          // operand chunks of a row and half
+  constexpr int DT = D / 32;
+  constexpr int STRV = D + 32;            // bf16 of a staged V row (transpose reads touch all banks)
+  constexpr int RC = D / E;               // chunks of a V row
+  constexpr int VL = F32 ? 1 : BK * RC / 64;  // V chunks a lane stages
+  constexpr int REC = 2 + 16 * DT;        // a lane's softmax state: max, sum, O
+  constexpr int kWaveBytes = 64 * REC * 4 > (F32 ? 0 : BK * STRV * 2) ? 64 * REC * 4 : BK * STRV * 2;
+  __shared__ __attribute__((aligned(16))) char lds[kGenAttnWaves][kWaveBytes];
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const int h = blockIdx.y % a.heads, b = blockIdx.y / a.heads;
+  const int kvh = h / (a.heads / a.kv_heads);
+  // the last query tile first: a causal one has the most keys
+  const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kGenAttnQueries;
+  const int qi = q0 + col, qrow = min(qi, a.lq - 1);
+  const long long kbase = b * a.ks[0] + kvh * a.ks[1], vbase = b * a.vs[0] + kvh * a.vs[1];
+  uint16_t* vs = reinterpret_cast<uint16_t*>(lds[wave]);
+
+  uint4 qf[S];
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int d0 = (2 * s + half) * E;
+    qf[s] = attn_chunk<F32, VEC>(a.q, a.q_dtype,
+                                 b * a.qs[0] + h * a.qs[1] + qrow * a.qs[2] + d0 * a.qs[3], a.qs[3], a.d - d0);
+  }
+
+  const int last_key = a.causal ? min(a.lk, q0 + kGenAttnQueries) : a.lk;
+  const int tiles = (last_key + BK - 1) / BK;
+
+  uint4 kf[KT][S], vf[VL];
+  auto load_keys = [&](int j0) {
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub) {
+      const long long off = kbase + (long long)min(j0 + 32 * sub + col, a.lk - 1) * a.ks[2];
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const int d0 = (2 * s + half) * E;
+        kf[sub][s] = attn_chunk<F32, VEC>(a.k, a.k_dtype, off + d0 * a.ks[3], a.ks[3], a.d - d0);
+      }
+    }
+  };
+  auto load_values = [&](int j0) {
+    if constexpr (!F32) {
+#pragma unroll
+      for (int i = 0; i < VL; ++i) {
+        const int c = lane + 64 * i, row = c / RC, d0 = (c % RC) * E;
+        vf[i] = attn_chunk<F32, VEC>(a.v, a.v_dtype, vbase + (long long)min(j0 + row, a.lk - 1) * a.vs[2] + d0 * a.vs[3],
+                                     a.vs[3], a.dv - d0);
+      }
+    }
+  };
+  // f32 V in operand order: key (e, half) of a tile, column 32 t + col
+  auto value_f32 = [&](int j0, int e, int t) -> float {
+    const int j = j0 + 8 * (e >> 2) + 4 * half + (e & 3), d = 32 * t + col;
+    if (j >= a.lk || d >= a.dv) return 0.f;
+    return load_float(a.v, a.v_dtype, vbase + (long long)j * a.vs[2] + (long long)d * a.vs[3]);
+  };
+
+  f32x16_t o[DT] = {}, p[KT];
+  float run_max = -INFINITY, run_sum = 0.f;
+
+  // +-inf and NaN of a tile's values, for the queries whose p of their key is not zero: per class, the
+  // product of the class's indicator with [p != 0], and the special value where it is not zero. The
+  // values are read again (the staged ones are gone); the pass is as rare as such values.
+  auto special_values = [&](int j0) {
+    for (int cls = 0; cls < 3; ++cls) {
+      f32x16_t hits[DT] = {};
+      if constexpr (F32) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float pe = p[0][e] != 0.f ? 1.f : 0.f;
+#pragma unroll
+          for (int t = 0; t < DT; ++t) {
+            const float v = value_f32(j0, e, t);
+            const float ind = not_finite_f32(v) && special_class(v) == cls ? 1.f : 0.f;
+            hits[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(ind, pe, hits[t], 0, 0, 0);
+          }
+        }
+      } else {
+        wave_lds_order();
+        for (int c = lane; c < BK * RC; c += 64) {
+          const int row = c / RC, d0 = (c % RC) * E;
+          const uint4 r = attn_chunk<F32, VEC>(
+              a.v, a.v_dtype, vbase + (long long)min(j0 + row, a.lk - 1) * a.vs[2] + d0 * a.vs[3], a.vs[3], a.dv - d0);
+          const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const uint32_t bits = (w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
+            const bool hit = not_finite_bf16(bits) && special_class(bf16_to_f32(bits)) == cls;
+            vs[row * STRV + d0 + i] = hit ? (uint16_t)0x3F80u : (uint16_t)0u;
+          }
+        }
+        wave_lds_order();
+#pragma unroll
+        for (int kt = 0; kt < 2 * KT; ++kt) {
+          uint32_t w[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float p0 = p[kt >> 1][8 * (kt & 1) + 2 * i], p1 = p[kt >> 1][8 * (kt & 1) + 2 * i + 1];
+            w[i] = (p0 != 0.f ? 0x3F80u : 0u) | (p1 != 0.f ? 0x3F800000u : 0u);
+          }
+          const fa_bf16x8 pb = __builtin_bit_cast(fa_bf16x8, w);
+#pragma unroll
+          for (int t = 0; t < DT; ++t)
+            hits[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(flash_v_operand<STRV>(vs, kt, 32 * t, lane), pb, hits[t],
+                                                              0, 0, 0);
+        }
+      }
+      const float value = cls == 0 ? INFINITY : cls == 1 ? -INFINITY : NAN;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (hits[t][e] > 0.f) o[t][e] += value;
+    }
+  };
+
+  if (wave < tiles) {
+    load_keys(wave * BK);
+    load_values(wave * BK);
+  }
+  for (int tile = wave; tile < tiles; tile += kGenAttnWaves) {
+    const int j0 = tile * BK;
+    const int next = min(tile + kGenAttnWaves, tiles - 1) * BK;
+
+    bool odd = false;  // a value that is not finite
+    if constexpr (!F32) {
+      wave_lds_order();
+#pragma unroll
+      for (int i = 0; i < VL; ++i) {
+        const int c = lane + 64 * i, row = c / RC, cc = c % RC;
+        uint32_t w[4] = {vf[i].x, vf[i].y, vf[i].z, vf[i].w};
+        bool mine = false;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          mine = mine || (w[u] & 0x7F80u) == 0x7F80u || (w[u] & 0x7F800000u) == 0x7F800000u;
+        if (mine) {
+          odd = true;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if ((w[u] & 0x7F80u) == 0x7F80u) w[u] &= 0xFFFF0000u;
+            if ((w[u] & 0x7F800000u) == 0x7F800000u) w[u] &= 0xFFFFu;
+          }
+        }
+        *reinterpret_cast<uint4*>(vs + row * STRV + cc * E) = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+      wave_lds_order();
+    }
+
+    f32x16_t sc[KT];
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub) {
+      sc[sub] = f32x16_t{};
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if constexpr (F32) {
+          const uint32_t kw[4] = {kf[sub][s].x, kf[sub][s].y, kf[sub][s].z, kf[sub][s].w};
+          const uint32_t qw[4] = {qf[s].x, qf[s].y, qf[s].z, qf[s].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sc[sub] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kw[e]), __uint_as_float(qw[e]), sc[sub], 0,
+                                                           0, 0);
+        } else {
+          sc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[sub][s]),
+                                                            __builtin_bit_cast(bf16x8_t, qf[s]), sc[sub], 0, 0, 0);
+        }
+      }
+    }
+    // the next tile's loads work under this one's softmax and products (the last trip reads its own again)
+    load_keys(next);
+    load_values(next);
+
+    float tile_max = -INFINITY;
+    const long long mrow = b * a.ms[0] + h * a.ms[1] + (long long)qrow * a.ms[2];
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int j = j0 + 32 * sub + 8 * (e >> 2) + 4 * half + (e & 3);
+        bool keep = j < a.lk && !(a.causal && j > qi);
+        float add = 0.f;
+        if (a.mask != nullptr && keep) {
+          const long long mo = mrow + (long long)j * a.ms[3];
+          if (a.mask_dtype == AOTO_DT_BOOL)
+            keep = static_cast<const uint8_t*>(a.mask)[mo] != 0;
+          else
+            add = load_float(a.mask, a.mask_dtype, mo);
+        }
+        const float v = keep ? sc[sub][e] * a.scale + add : -INFINITY;
+        p[sub][e] = v;
+        tile_max = fmaxf(tile_max, v);
+      }
+    tile_max = xor32_max(tile_max);
+    const float moved = fmaxf(run_max, tile_max);
+    // (a maximum of -inf has only zeros, or a NaN score's NaN, behind it: kept as they are)
+    const float correction = run_max == moved || run_max == -INFINITY ? 1.f : expf(run_max - moved);
+    run_max = moved;
+    if (__any(correction != 1.f)) {
+      // a correction of zero drops what was summed, infinities too
+      run_sum = correction == 0.f ? 0.f : run_sum * correction;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] = correction == 0.f ? 0.f : o[t][e] * correction;
+    }
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        p[sub][e] = p[sub][e] == -INFINITY ? 0.f : expf(p[sub][e] - moved);
+        run_sum += p[sub][e];
+      }
+
+    if constexpr (F32) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+          float v = value_f32(j0, e, t);
+          if (not_finite_f32(v)) {
+            odd = true;
+            v = 0.f;
+          }
+          o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, p[0][e], o[t], 0, 0, 0);
+        }
+    } else {
+#pragma unroll
+      for (int kt = 0; kt < 2 * KT; ++kt) {
+        uint32_t hi[4], mid[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p0 = p[kt >> 1][8 * (kt & 1) + 2 * i], p1 = p[kt >> 1][8 * (kt & 1) + 2 * i + 1];
+          hi[i] = cvt_pk_bf16(p0, p1);
+          const float r0 = p0 - bf16_lo(hi[i]), r1 = p1 - bf16_hi(hi[i]);
+          mid[i] = cvt_pk_bf16(r0, r1);
+          lo[i] = cvt_pk_bf16(r0 - bf16_lo(mid[i]), r1 - bf16_hi(mid[i]));
+        }
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+          const fa_bf16x8 va = flash_v_operand<STRV>(vs, kt, 32 * t, lane);
+          o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(fa_bf16x8, hi), o[t], 0, 0, 0);
+          o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(fa_bf16x8, mid), o[t], 0, 0, 0);
+          o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(fa_bf16x8, lo), o[t], 0, 0, 0);
+        }
+      }
+    }
+    if (__any(odd)) special_values(j0);
+  }
+
+  // The waves' states (the V stages are dead: a wave's records lie in its own), combined by all four:
+  // wave w takes every fourth run of 4 output columns.
+  wave_lds_order();
+  float* rec = reinterpret_cast<float*>(lds[wave]);
+  rec[lane] = run_max;
+  rec[64 + lane] = run_sum;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) rec[(2 + 16 * t + e) * 64 + lane] = o[t][e];
+  __syncthreads();
+  float big = -INFINITY, sum = 0.f, factor[kGenAttnWaves];
+#pragma unroll
+  for (int w = 0; w < kGenAttnWaves; ++w) big = fmaxf(big, reinterpret_cast<const float*>(lds[w])[lane]);
+#pragma unroll
+  for (int w = 0; w < kGenAttnWaves; ++w) {
+    const float* other = reinterpret_cast<const float*>(lds[w]);
+    factor[w] = other[lane] == -INFINITY ? 1.f : expf(other[lane] - big);
+    // both halves' keys
+    const float l = other[64 + col] + other[64 + 32 + col];
+    if (factor[w] != 0.f) sum += l * factor[w];
+  }
+  if (qi >= a.lq) return;
+  const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+  const long long ob = ((long long)(b * a.heads + h) * a.lq + qi) * a.dv;
+#pragma unroll
+  for (int g = wave; g < 4 * DT; g += kGenAttnWaves) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = 8 * g + 4 * half + i;
+      if (d >= a.dv) continue;
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < kGenAttnWaves; ++w) {
+        const float x = reinterpret_cast<const float*>(lds[w])[(2 + 4 * g + i) * 64 + lane];
+        if (factor[w] != 0.f) v += x * factor[w];
+      }
+      // a row with no kept key (and one whose scores are all NaN) gives zeros
+      store_float_type(a.out, a.out_dtype, ob + d, big == -INFINITY ? 0.f : v * inv);
+    }
+  }
+}
+
+}  // namespace aoto
+
+#define AOTO_GENERIC_ATTENTION(TYPE, F32, D, LETTER, VEC)                                             \
+  extern "C" __global__ __launch_bounds__(64 * aoto::kGenAttnWaves) void                              \
+      aoto_generic_attention_##TYPE##_d##D##_##LETTER(aoto::AttnArgs a) {                             \
+    aoto::generic_attention_body<F32, D, VEC>(a);                                                     \
+  }

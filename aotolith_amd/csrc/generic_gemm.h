@@ -44,7 +44,7 @@ AOTO_DEVICE uint4 gemm_chunk_any(const void* p, int dtype, long long off, long l
       if (sizeof(T) == 2)
         w[e >> 1] |= (uint32_t) static_cast<const uint16_t*>(p)[off + e * step] << (16 * (e & 1));
       else
-        w[e & 3] = __float_as_uint((float)load_value(p, dtype, off + e * step));
+        w[e & 3] = __float_as_uint(load_float(p, dtype, off + e * step));
     }
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
@@ -265,7 +265,7 @@ __device__ __forceinline__ void generic_gemm_body(const GemmArgs& g) {
           const float b = (float)load_value(g.bias, g.bias_dtype, batch * g.sbias_b + m * g.sbias_m + n * g.sbias_n);
           v = g.beta == 1.f ? v + b : v + g.beta * b;
         }
-        store_float(g.c, g.c_dtype, batch * g.sc_b + m * g.sc_m + n * g.sc_n, v);
+        store_float_type(g.c, g.c_dtype, batch * g.sc_b + m * g.sc_m + n * g.sc_n, v);
       }
   }
 }

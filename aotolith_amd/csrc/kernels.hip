@@ -14,6 +14,7 @@
 #include "decode.h"
 #include "prefill.h"
 #include "flash_attention.h"
+#include "generic_attention.h"
 
 // W4 decode GEMV: {lanes per row} x {norm prologue} x {paired} x {bias epilogue}.
 AOTO_GEMV_LPR(0, 0, 0)
@@ -164,3 +165,13 @@ AOTO_GENERIC_GEMM_MODE(bf16, uint16_t, a, aoto::kAny)
 AOTO_GENERIC_GEMM_MODE(f32, float, v, aoto::kVec)
 AOTO_GENERIC_GEMM_MODE(f32, float, c, aoto::kCols)
 AOTO_GENERIC_GEMM_MODE(f32, float, a, aoto::kAny)
+
+// The graph plans' attention: {operand type} x {head size up to} x {operand loads}.
+AOTO_GENERIC_ATTENTION(bf16, false, 64, v, true)
+AOTO_GENERIC_ATTENTION(bf16, false, 64, a, false)
+AOTO_GENERIC_ATTENTION(bf16, false, 128, v, true)
+AOTO_GENERIC_ATTENTION(bf16, false, 128, a, false)
+AOTO_GENERIC_ATTENTION(f32, true, 64, v, true)
+AOTO_GENERIC_ATTENTION(f32, true, 64, a, false)
+AOTO_GENERIC_ATTENTION(f32, true, 128, v, true)
+AOTO_GENERIC_ATTENTION(f32, true, 128, a, false)

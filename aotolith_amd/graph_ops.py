@@ -222,7 +222,10 @@ KERNELS = {"elementwise": "aoto_generic_elementwise", "reduction": "aoto_generic
 #: Families whose kernel an earlier build's code object does not have: the symbol that tells, and the
 #: names this build's selections record (a family prefix: the instance follows the operands' strides).
 NEWER = {"matmul": ("aoto_generic_gemm_f32_a_t1k1", "aoto_generic_gemm_*",
-                    "strided batched GEMM on the matrix cores, LDS-staged tiles, f32 accumulation")}
+                    "strided batched GEMM on the matrix cores, LDS-staged tiles, f32 accumulation"),
+         "attention": ("aoto_generic_attention_f32_d64_a", "aoto_generic_attention*",
+                       "legalized scaled-dot-product attention (bool/float mask, causal, GQA) on the matrix cores, "
+                       "f32 softmax")}
 REASONS = {
     "elementwise": "strided broadcasting elementwise kernel, f32 compute, one rounding to the output type",
     "reduction": "row reduction / scan over the (permuted) last dim, f32 or int64 accumulation",

@@ -244,3 +244,80 @@ def test_matmul_with_no_reduction_is_its_bias():
     out = torch.full((2, 3, 5), 7.0, device="cuda")
     launch_matmul(out, torch.empty(2, 3, 0, device="cuda"), torch.empty(2, 0, 5, device="cuda"))
     assert bool((out == 0).all())
+
+
+def _attention_reference(q, k, v, mask, causal, scale):
+    """(out, sum of p |v|, largest |q| . |k| scaled) in 64 bits; a key of probability zero contributes nothing."""
+
+    group = q.shape[1] // k.shape[1]
+    k, v = (t.double().repeat_interleave(group, 1) for t in (k, v))
+    q = q.double()
+    s = q @ k.transpose(-1, -2) * scale
+    room = (q.abs() @ k.abs().transpose(-1, -2) * scale).amax()
+    if causal:
+        s = s.masked_fill(~torch.ones(s.shape[-2:], dtype=torch.bool, device=s.device).tril(), float("-inf"))
+    if mask is not None:
+        s = s.masked_fill(~mask, float("-inf")) if mask.dtype == torch.bool else s + mask.double()
+    s = torch.exp(s - s.amax(-1, keepdim=True).clamp_min(torch.finfo(torch.float64).min))
+    s = torch.where(s < 2.0 ** -149, torch.zeros_like(s), s)
+    p = s / s.sum(-1, keepdim=True).clamp_min(1e-300)
+    finite = torch.where(torch.isfinite(v), v, torch.zeros_like(v))
+    out, size = p @ finite, p @ finite.abs()
+    live = (p > 0).double()
+    for value in (float("inf"), float("-inf")):
+        out = torch.where(live @ (v == value).double() > 0, out + value, out)
+    return torch.where(live @ v.isnan().double() > 0, torch.full_like(out, float("nan")), out), size, room
+
+
+@pytest.mark.parametrize("types", ["bf16", "f32", "mixed"])
+@pytest.mark.parametrize("masked", ["none", "causal", "bool", "float", "lowest"])
+@pytest.mark.parametrize("batch,heads,kv_heads,lq,lk,d,dv,layout", [
+    (1, 1, 1, 1, 1, 64, 64, "plain"), (2, 4, 2, 33, 65, 64, 64, "heads_last"), (1, 3, 1, 31, 300, 128, 128, "plain"),
+    (1, 2, 2, 70, 70, 80, 48, "plain"), (1, 2, 1, 40, 257, 24, 24, "heads_last"), (1, 2, 1, 9, 130, 33, 7, "strided"),
+    (1, 2, 1, 5, 40, 160, 136, "plain")])
+def test_attention_over_its_tiles_layouts_masks_and_types(batch, heads, kv_heads, lq, lk, d, dv, layout, masked, types):
+    """Every instance at tile remainders, against 64-bit attention. Bound: the scores' f32 sums move an exponent by at
+    most (d + 4) 2^-24 of the absolute products, the exponentials, sums and products add (lk + 16) 2^-24, and the
+    result is rounded once to the output type. Values that are not finite sit at masked keys and at one that is not."""
+
+    from aotolith_amd.graph_ops import launch_attention
+
+    gen = torch.Generator().manual_seed(lq * 5 + lk + d)
+    kinds = {"bf16": (torch.bfloat16,) * 3, "f32": (torch.float32,) * 3,
+             "mixed": (torch.bfloat16, torch.float32, torch.bfloat16)}[types]
+
+    def operand(h, rows, dim, dtype):
+        shape = {"plain": (batch, h, rows, dim), "heads_last": (batch, rows, h, dim),
+                 "strided": (batch, h, rows, 2 * dim)}[layout]
+        t = torch.randn(*shape, generator=gen).to(dtype).cuda()
+        return t.transpose(1, 2) if layout == "heads_last" else t[..., ::2] if layout == "strided" else t
+
+    q, k, v = operand(heads, lq, d, kinds[0]), operand(kv_heads, lk, d, kinds[1]), operand(kv_heads, lk, dv, kinds[2])
+    mask = None
+    if masked in ("bool", "lowest"):
+        mask = torch.rand(1, heads, lq, lk, generator=gen).cuda() > 0.4
+        mask[:, :, 0] = False  # a row with no key
+        mask[..., lk // 2] = False
+        v[:, :, lk // 2] = float("nan")  # a key no query keeps
+    if masked == "lowest":
+        mask[:, :, 0] = True  # (every key at the lowest value would weigh them evenly, the NaN one too)
+        mask[:, :, 0, lk // 2] = lk == 1
+        if lk == 1:
+            v[:, :, 0] = 1.0
+        mask = torch.zeros(mask.shape, device="cuda").masked_fill(~mask, torch.finfo(torch.float32).min)
+    if masked == "float":
+        mask = torch.randn(lq, lk, generator=gen).cuda()
+    if masked in ("none", "causal"):
+        v[:, :, lk - 1, 0] = float("inf")  # one column: inf for the queries that see the last key
+    scale = d ** -0.5
+    want, size, room = _attention_reference(q, k, v, mask, masked == "causal", scale)
+    exponent = (d + 4) * 2.0 ** -24 * float(room) + (2.0 ** -22 * 8 if mask is not None else 0.0)
+    for out_type, eps in ((torch.float32, 2.0 ** -24), (torch.bfloat16, 2.0 ** -8)):
+        out = torch.full((batch, heads, lq, dv), 7.0, dtype=out_type, device="cuda")
+        launch_attention(out, q, k, v, mask, masked == "causal", scale)
+        got = out.double()
+        fine = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), fine) and torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got[got.isinf()], want[want.isinf()])
+        bound = (4 * exponent + (lk + 16) * 2.0 ** -24) * size + eps * want.abs()
+        assert bool(((got - want).abs() <= bound)[fine].all())
