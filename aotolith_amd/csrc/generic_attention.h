@@ -20,7 +20,7 @@
 //
 // Bound: latency (two tiles a wave at 512 keys), then the MFMA pipe. 14 heads of 64, 512 tokens,
 // causal, bf16: 881 us with one block per query row and scalar dots (every score a 64-step chain of
-// typed loads) -> MEAS us.
+// typed loads) -> 19.7 us.
 #pragma once
 
 #include "aoto_hip.h"
