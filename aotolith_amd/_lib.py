@@ -232,14 +232,14 @@ def hold_graph(graph) -> None:
 def ensure_code_object(device: int | None = None) -> str:
     """Install the packaged code object on ``device`` unless one is installed."""
 
+    digest = None if device is None else _loaded_devices.get(device)
+    if digest is not None:
+        return digest
     import torch
 
     if not torch.cuda.is_available():
         raise HipBackendUnavailable("no ROCm GPU visible: the hip-gfx950 target needs an MI355X")
     device = torch.cuda.current_device() if device is None else device
-    digest = _loaded_devices.get(device)
-    if digest is not None:
-        return digest
     with _lock:
         digest = _loaded_devices.get(device)
         if digest is None:

@@ -981,27 +981,30 @@ class _Engine:
         ops.embedding(self.state.embed, ids.reshape(-1), out=x)
         layers = self.state.layers
         fuse = _prefill_fuses_norms(s)
+        positions, qkv, attn_rows = positions.reshape(-1), qkv.view(m, -1), attn.view(m, -1)
+        if rec is not None:
+            qkv_kernel = (
+                f"dequant-once W{bits} GEMM (packed tiles expanded once per 256-row block into LDS) on "
+                "32x32x16 bf16 MFMA"
+                if ops.lds_plan(m, s.qkv_width, s.hidden, group_size=layers[0].qkv.group, bits=bits, rope=True)
+                is not None
+                else f"wide-tile fused-dequant W{bits} GEMM on 32x32x16 bf16 MFMA"
+                if ops.wide_plan(m, s.qkv_width, s.hidden) is not None
+                else f"fused-dequant W{bits} GEMM on bf16 MFMA") + (" with q/k/v bias" if s.qkv_bias else "")
         for index, layer in enumerate(layers):
             if index == 0 or not fuse:
                 _mark(rec, "rms_norm", f"norm_{index}a", "rms_norm", "row RMSNorm")
                 ops.rms_norm(x, layer.input_norm, s.eps, out=xn)
             pair = pair_of(index)
-            _mark(rec, "addmm" if s.qkv_bias else "matmul", f"qkv_{index}", gemm,
-                  (f"dequant-once W{bits} GEMM (packed tiles expanded once per 256-row block into LDS) on "
-                   "32x32x16 bf16 MFMA"
-                   if ops.lds_plan(m, s.qkv_width, s.hidden, group_size=layer.qkv.group, bits=bits, rope=True)
-                   is not None
-                   else f"wide-tile fused-dequant W{bits} GEMM on 32x32x16 bf16 MFMA"
-                   if ops.wide_plan(m, s.qkv_width, s.hidden) is not None
-                   else f"fused-dequant W{bits} GEMM on bf16 MFMA") + (" with q/k/v bias" if s.qkv_bias else "")
-                  + ", RoPE of q/k and the layer's cache fill (with the split-K sum when the plan splits)")
+            if rec is not None:
+                _mark(rec, "addmm" if s.qkv_bias else "matmul", f"qkv_{index}", gemm,
+                      qkv_kernel + ", RoPE of q/k and the layer's cache fill (with the split-K sum when the plan splits)")
             # q/k/v projection, RoPE and the cache fill (one launch fewer when the plan splits K)
-            ops.matmul_qkv_rope(xn, layer.qkv.packed, layer.qkv.scales, layer.qkv.group, positions.reshape(-1),
+            ops.matmul_qkv_rope(xn, layer.qkv.packed, layer.qkv.scales, layer.qkv.group, positions,
                                 self.cos, self.sin, pair, query_heads=s.heads, kv_heads=s.kv_heads,
                                 head_dim=s.head_dim, slot0=slot0, bias=layer.qkv_bias, bits=layer.qkv.bits,
-                                out=qkv.view(m, -1), q_out=q)
-            keys = pair[0][:, :, slot0:slot0 + m]
-            values = pair[1][:, :, slot0:slot0 + m]
+                                out=qkv, q_out=q)
+            keys, values = pair.narrow(3, slot0, m).unbind(0)
             _mark(rec, "attention", f"attention_{index}", "flash_attention",
                   "masked GQA flash attention on MFMA" if mask is not None
                   else "causal + left-pad masked GQA flash attention on MFMA")
@@ -1013,11 +1016,11 @@ class _Engine:
                 _mark(rec, "addmm", f"hidden_{index}a", gemm,
                       f"W{bits} GEMM with residual epilogue, then the next RMSNorm (one launch with the split-K sum "
                       "when the plan splits)")
-                ops.matmul_residual_norm(attn.view(m, -1), layer.o.packed, layer.o.scales, layer.o.group, x,
+                ops.matmul_residual_norm(attn_rows, layer.o.packed, layer.o.scales, layer.o.group, x,
                                          layer.post_norm, s.eps, bits=layer.o.bits, out=x, norm_out=xn)
             else:
                 _mark(rec, "addmm", f"hidden_{index}a", gemm, f"W{bits} GEMM with residual epilogue")
-                self._matmul(attn.view(m, -1), layer.o, residual=x, out=x)
+                self._matmul(attn_rows, layer.o, residual=x, out=x)
                 _mark(rec, "rms_norm", f"norm_{index}b", "rms_norm", "row RMSNorm")
                 ops.rms_norm(x, layer.post_norm, s.eps, out=xn)
             if paired:
@@ -1161,7 +1164,7 @@ class DecoderStaticCacheRuntime:
         if tuple(ids.shape) != (1, self.prompt_length):
             raise PlanInputError(f"expected prompt shape (1, {self.prompt_length}), got {tuple(ids.shape)}")
         positions = torch.arange(self.prompt_length, dtype=torch.int64, device=ids.device)[None, :]
-        return self.prefill(ids, positions, None)
+        return self.prefill(ids, positions, None, verify_positions=False)
 
     def prefill_padded(self, input_ids):
         ids = _as_ids(input_ids, self.engine.device)
@@ -1178,7 +1181,7 @@ class DecoderStaticCacheRuntime:
         zeros = torch.zeros((1, padding), dtype=torch.int64, device=ids.device)
         padded_ids = torch.cat((zeros, ids), dim=1)
         positions = torch.cat((zeros, torch.arange(length, dtype=torch.int64, device=ids.device)[None, :]), dim=1)
-        return self.prefill(padded_ids, positions, length)
+        return self.prefill(padded_ids, positions, length, verify_positions=False)
 
     def pad_cache(self, compact_cache: torch.Tensor) -> torch.Tensor:
         expected = (self.num_layers, 2, 1, self.num_key_value_heads, self.prompt_length, self.head_dim)
@@ -1200,13 +1203,23 @@ class DecoderStaticCacheRuntime:
         if valid_length < 1 or valid_length >= self.cache_capacity:
             raise PlanInputError(f"valid_length must be in [1, {self.cache_capacity}), got {valid_length}")
         token = _as_ids(token, self.engine.device).reshape(-1)[:1]
-        if verify_token:
-            value = int(token.item())
-            if not 0 <= value < self.spec.vocab:
-                from .errors import IndexBoundsError
+        if not verify_token:
+            return self.decode(token, cache, valid_length)
+        # The token is read back while the step is being launched (an id outside the table embeds as zeros,
+        # so the launches are safe before it is known): the copy waits for whatever made the token, and
+        # waiting for that first would leave the GPU idle until the step's first launch.
+        host = torch.empty((1,), dtype=torch.int64, pin_memory=True)
+        host.copy_(token, non_blocking=True)
+        arrived = torch.cuda.Event()
+        arrived.record()
+        result = self.decode(token, cache, valid_length)
+        arrived.synchronize()
+        value = int(host.item())
+        if not 0 <= value < self.spec.vocab:
+            from .errors import IndexBoundsError
 
-                raise IndexBoundsError(f"token {value} is outside the vocabulary [0, {self.spec.vocab})")
-        return self.decode(token, cache, valid_length)
+            raise IndexBoundsError(f"token {value} is outside the vocabulary [0, {self.spec.vocab})")
+        return result
 
     def greedy_generate(self, input_ids, *, max_new_tokens: int | None = None, sync_each_step: bool = False,
                         use_graph: bool = True, events: dict | None = None) -> torch.Tensor:
@@ -1299,14 +1312,18 @@ class DecoderStaticCacheRuntime:
 def _build_plans(spec: DecoderSpec, engine: _Engine, prompt_length: int):
     capacity = engine.capacity
 
-    def run_prefill(ids, positions, mask_or_length=None):
-        """(ids [1,P], positions [1,P], mask [1,1,P,P] | real length | None) -> (logits, compact cache)."""
+    def run_prefill(ids, positions, mask_or_length=None, *, verify_positions: bool = True):
+        """(ids [1,P], positions [1,P], mask [1,1,P,P] | real length | None) -> (logits, compact cache).
+
+        ``verify_positions=False`` leaves out the range check (two reductions read back to the host), for
+        positions the caller has just counted itself.
+        """
 
         ids = _as_ids(ids, engine.device)
         if tuple(ids.shape) != (1, prompt_length):
             raise PlanInputError(f"expected ids of shape (1, {prompt_length}), got {tuple(ids.shape)}")
         positions = _as_ids(positions, engine.device)
-        if int(positions.max()) >= capacity or int(positions.min()) < 0:
+        if verify_positions and (int(positions.max()) >= capacity or int(positions.min()) < 0):
             raise PlanInputError(f"positions must lie in [0, {capacity})")
         compact = torch.empty((spec.layers, 2, 1, spec.kv_heads, prompt_length, spec.head_dim), dtype=BF16,
                               device=engine.device)

@@ -22,7 +22,7 @@ from collections.abc import Callable
 
 import torch
 
-from . import _lib
+from . import _lib, ops
 from .errors import CompilationError, PlanInputError
 from .graph import RMS_NORM, LoweredGraph, Node, Ref
 from .plan import ARCHITECTURE, CompiledPlan, PlanNode
@@ -47,8 +47,31 @@ class AotoTensor(ctypes.Structure):
     ]
 
 
+#: Filled descriptors by (dtype, shape, strides): a plan's calls meet the same few dozen again and again,
+#: and filling one field by field costs more than the launch. Copied before use, so safe to share;
+#: bounded, so a program with ever new shapes keeps none of them for long.
+_DESCRIPTORS: dict[tuple, AotoTensor] = {}
+_MAX_DESCRIPTORS = 4096
+
+
 def describe(value) -> AotoTensor:
     """The descriptor of a device tensor, or of a Python scalar (data NULL, ndim 0)."""
+
+    if isinstance(value, torch.Tensor):
+        key = (value.dtype, value.shape, value.stride())
+        known = _DESCRIPTORS.get(key)
+        if known is None:
+            if len(_DESCRIPTORS) >= _MAX_DESCRIPTORS:
+                _DESCRIPTORS.clear()
+            known = _DESCRIPTORS[key] = _describe_layout(value)
+        d = AotoTensor.from_buffer_copy(known)
+        d.data = value.data_ptr() if value.numel() else 1  # a non-null pointer for empty tensors
+        return d
+    return _describe_layout(value)
+
+
+def _describe_layout(value) -> AotoTensor:
+    """A descriptor without its address."""
 
     d = AotoTensor()
     if isinstance(value, torch.Tensor):
@@ -56,7 +79,6 @@ def describe(value) -> AotoTensor:
             raise CompilationError(f"element type {value.dtype} has no gfx950 kernel here")
         if value.dim() > MAX_DIMS:
             raise CompilationError(f"tensors of rank {value.dim()} exceed the kernels' {MAX_DIMS} dims")
-        d.data = value.data_ptr() if value.numel() else 1  # a non-null pointer for empty tensors
         d.dtype = DTYPE_CODES[value.dtype]
         d.ndim = value.dim()
         for i, (n, s) in enumerate(zip(value.shape, value.stride())):
@@ -69,14 +91,16 @@ def describe(value) -> AotoTensor:
     return d
 
 
+_addressof = ctypes.addressof
+
+
 def _p(desc: AotoTensor | None):
     """The address of a descriptor (kept alive by the caller for the call)."""
 
-    return None if desc is None else ctypes.addressof(desc)
+    return None if desc is None else _addressof(desc)
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+_stream = ops._stream
 
 
 # ----------------------------------------------------------------------------- launches
@@ -279,6 +303,9 @@ class GraphRunner:
         for node in graph.nodes:
             self.handlers.append((node, self._handler(node)))
         self.error = None
+        # only gathers can meet an index out of range: a graph without one has no flag to set or read back
+        self.gathers = any(node.op in INDEX_OPS for node in graph.nodes)
+        self.state_ptrs = {t.data_ptr() for t in self.state.values() if isinstance(t, torch.Tensor)}
 
     # -- selection records --------------------------------------------------------
     def selections(self, device_name: str | None) -> tuple[KernelSelection, ...]:
@@ -302,19 +329,19 @@ class GraphRunner:
     def run(self, inputs: dict[str, torch.Tensor], *, verify_index_bounds: bool = True):
         env: dict = dict(self.state)
         env.update(inputs)
-        self.error = torch.empty((1,), dtype=torch.int32, device=self.device)
-        launch_fill(self.error, 0)
+        if self.gathers:
+            self.error = torch.empty((1,), dtype=torch.int32, device=self.device)
+            launch_fill(self.error, 0)
         for node, handler in self.handlers:
             env[node.name] = handler(env, node)
         outputs = []
-        state_ptrs = {t.data_ptr() for t in self.state.values() if isinstance(t, torch.Tensor)}
         for out in self.graph.outputs:
             value = _value(env, out)
             aliased = isinstance(out, Ref) and out.name in inputs
-            if isinstance(value, torch.Tensor) and (value.data_ptr() in state_ptrs or aliased):
+            if isinstance(value, torch.Tensor) and (value.data_ptr() in self.state_ptrs or aliased):
                 value = launch_copy(_empty(value.shape, value.dtype, self.device), value)
             outputs.append(value)
-        if verify_index_bounds and int(self.error.item()) != 0:
+        if self.gathers and verify_index_bounds and int(self.error.item()) != 0:
             raise PlanInputError("an index input is out of range for the tensor it indexes",
                                  hint="embedding ids / gather indices must lie in [-size, size)")
         return tuple(outputs)

