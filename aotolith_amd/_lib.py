@@ -111,6 +111,7 @@ SIGNATURES: dict[str, tuple] = {
         _p, _p, _p, _p, _c_int, _p, _p, _c_int, _p, _p, _p, _p,
     ),
     "aoto_hip_generic_elementwise": (_c_int, _p, _p, _p, _p, ctypes.c_double, _p),
+    "aoto_hip_generic_fused": (_p, _p, _c_int, _p, _p, _c_int, _p),
     "aoto_hip_generic_reduce": (_c_int, _p, _p, _p),
     "aoto_hip_generic_matmul": (_p, _p, _p, _p, _c_float, _c_float, _p),
     "aoto_hip_generic_index": (_p, _p, _c_int, _p, _p, _p),

@@ -1624,6 +1624,108 @@ void generic_attention_plan(const aoto::AttnArgs& a, char* name, size_t size) {
            vec ? 'v' : 'a');
 }
 
+// Dims of extent 1 dropped, and neighbouring dims that every operand walks as one merged; `walks` are the
+// operands' element strides, rewritten in place. Returns the number of dims left (at least 1).
+int collapse_dims(int ndim, long long* shape, long long* const* walks, int count) {
+  int n = 0;
+  for (int d = 0; d < ndim; ++d) {
+    if (shape[d] == 1) continue;
+    bool merge = n > 0;
+    for (int w = 0; w < count && merge; ++w) merge = walks[w][n - 1] == walks[w][d] * shape[d];
+    if (merge) {
+      shape[n - 1] *= shape[d];
+      for (int w = 0; w < count; ++w) walks[w][n - 1] = walks[w][d];
+    } else {
+      shape[n] = shape[d];
+      for (int w = 0; w < count; ++w) walks[w][n] = walks[w][d];
+      ++n;
+    }
+  }
+  if (n == 0) {
+    shape[0] = 1;
+    for (int w = 0; w < count; ++w) walks[w][0] = 0;
+    n = 1;
+  }
+  return n;
+}
+
+bool fused_op(int op) {
+  switch (op) {
+    case AOTO_EW_CAST: case AOTO_EW_NEG: case AOTO_EW_ABS: case AOTO_EW_RSQRT: case AOTO_EW_EXP: case AOTO_EW_SIGMOID:
+    case AOTO_EW_SILU: case AOTO_EW_RELU: case AOTO_EW_TANH: case AOTO_EW_GELU: case AOTO_EW_GELU_TANH: case AOTO_EW_ADD:
+    case AOTO_EW_SUB: case AOTO_EW_MUL: case AOTO_EW_DIV: case AOTO_EW_MAXIMUM: case AOTO_EW_MINIMUM: return true;
+    default: return false;
+  }
+}
+
+// Collapses the operands' walks and says whether they are whole 8-element vectors: float operands with
+// stride 1 or 0 along the rows, 16-byte aligned row starts, row lengths in eights.
+bool fused_layout(aoto::FusedArgs& f, long long total) {
+  long long* walks[aoto::kFusedInputs];
+  for (int k = 0; k < f.inputs; ++k) walks[k] = f.in[k].strides;
+  f.ndim = collapse_dims(f.ndim, f.shape, walks, f.inputs);
+  const int last = f.ndim - 1;
+  if (!float_dtype(f.out_dtype) || !aligned16(f.out) || total >= (1ll << 31) || f.shape[last] % 8 != 0) return false;
+  for (int k = 0; k < f.inputs; ++k) {
+    const aoto::Operand& o = f.in[k];
+    if (o.data == nullptr) continue;
+    if (!float_dtype(o.dtype)) return false;
+    if (o.strides[last] == 0) continue;
+    if (o.strides[last] != 1 || !aligned16(o.data)) return false;
+    for (int d = 0; d < last; ++d)
+      if (o.strides[d] % 8 != 0) return false;
+  }
+  f.vectors = (unsigned)(total / 8);
+  f.per_row = (unsigned)(f.shape[last] / 8);
+  return true;
+}
+
+unsigned grid_for(long long total);
+
+int launch_elementwise(aoto::EwArgs& args, void* stream) {
+  if (args.domain == 0 && fused_op(args.op) && has_kernel("aoto_generic_fused")) {
+    aoto::FusedArgs f;
+    memset(&f, 0, sizeof(f));
+    f.inputs = args.op >= AOTO_EW_ADD ? 2 : 1;
+    f.count = 1;
+    f.ndim = args.ndim;
+    f.out = args.out;
+    f.out_dtype = args.out_dtype;
+    memcpy(f.in, args.in, f.inputs * sizeof(aoto::Operand));
+    memcpy(f.shape, args.shape, sizeof(f.shape));
+    f.steps[0] = {(uint8_t)args.op, 0, 4, 5, 0, (float)args.alpha};
+    if (fused_layout(f, args.total))
+      return launch("aoto_generic_fused", dim3(grid_for(f.vectors)), dim3(256), 0, stream, f);
+  }
+  long long* walks[3] = {args.in[0].strides, args.in[1].strides, args.in[2].strides};
+  args.ndim = collapse_dims(args.ndim, args.shape, walks, 3);
+  return launch("aoto_generic_elementwise", dim3(grid_for(args.total)), dim3(256), 0, stream, args);
+}
+
+int element_bytes(int dtype) {
+  switch (dtype) {
+    case AOTO_DT_F32: case AOTO_DT_I32: return 4;
+    case AOTO_DT_BF16: return 2;
+    case AOTO_DT_I64: return 8;
+    default: return 1;
+  }
+}
+
+// A collapsed copy of one element type with contiguous rows: its unit (16 bytes or the largest power of
+// two that divides every row's start and length), 0 where the rows are not contiguous.
+int copy_unit(const aoto::CopyArgs& a) {
+  if (a.src_dtype != a.dst_dtype || a.total >= (1ll << 31)) return 0;
+  const int last = a.ndim - 1;
+  if (a.shape[last] > 1 && (a.src_strides[last] != 1 || a.dst_strides[last] != 1)) return 0;
+  const long long es = element_bytes(a.src_dtype);
+  unsigned long long bits = 16ull | (unsigned long long)(a.shape[last] * es) | reinterpret_cast<uintptr_t>(a.src) |
+                            reinterpret_cast<uintptr_t>(a.dst);
+  for (int d = 0; d < last; ++d)
+    bits |= (unsigned long long)(a.src_strides[d] * es) | (unsigned long long)(a.dst_strides[d] * es);
+  const unsigned long long unit = bits & (~bits + 1);
+  return unit < (unsigned long long)es ? 0 : (int)unit;
+}
+
 unsigned grid_for(long long total) {
   long long blocks = (total + 255) / 256;
   if (blocks < 1) blocks = 1;
@@ -1679,7 +1781,44 @@ int aoto_hip_generic_elementwise(int op, const aoto_tensor* out, const aoto_tens
   args.out = out->data;
   args.alpha = alpha;
   if (args.total == 0) return AOTO_OK;
-  return launch("aoto_generic_elementwise", dim3(grid_for(args.total)), dim3(256), 0, stream, args);
+  return launch_elementwise(args, stream);
+}
+
+int aoto_hip_generic_fused(const aoto_tensor* out, const aoto_tensor* const* inputs, int input_count,
+                           const int32_t* program, const double* alphas, int count, void* stream) {
+  const char* what = "generic_fused";
+  if (int s = check_tensor(what, "out", out, false)) return s;
+  if (!contiguous(out)) return fail(AOTO_ERR_ARGUMENT, "%s: out must be contiguous", what);
+  if (!inputs || !program || !alphas || input_count < 1 || input_count > aoto::kFusedInputs || count < 1 ||
+      count > aoto::kFusedSteps)
+    return fail(AOTO_ERR_ARGUMENT, "%s: 1..%d operands and 1..%d steps", what, aoto::kFusedInputs, aoto::kFusedSteps);
+  aoto::FusedArgs f;
+  memset(&f, 0, sizeof(f));
+  bool written[4] = {false, false, false, false};
+  auto readable = [&](int s) { return s >= 0 && (s < 4 ? written[s] : s < 4 + input_count); };
+  for (int i = 0; i < count; ++i) {
+    const int32_t* p = program + 5 * i;
+    const bool binary = p[0] >= AOTO_EW_ADD;
+    if (!fused_op(p[0])) return fail(AOTO_ERR_ARGUMENT, "%s: step %d: op %d has no fused form", what, i, p[0]);
+    if (p[1] < 0 || p[1] > 3 || !readable(p[2]) || (binary && !readable(p[3])))
+      return fail(AOTO_ERR_ARGUMENT, "%s: step %d reads or writes a register it does not have", what, i);
+    written[p[1]] = true;
+    f.steps[i] = {(uint8_t)p[0], (uint8_t)p[1], (uint8_t)p[2], (uint8_t)(binary ? p[3] : 0), p[4] == AOTO_DT_BF16,
+                  (float)alphas[i]};
+  }
+  for (int k = 0; k < input_count; ++k)
+    if (int s = broadcast_operand(what, "operand", inputs[k], out, &f.in[k])) return s;
+  f.inputs = input_count;
+  f.count = count;
+  f.ndim = out->ndim;
+  f.out = out->data;
+  f.out_dtype = out->dtype;
+  for (int d = 0; d < out->ndim; ++d) f.shape[d] = out->shape[d];
+  const long long total = numel(out);
+  if (total == 0) return AOTO_OK;
+  if (!fused_layout(f, total))
+    return fail(AOTO_ERR_UNSUPPORTED, "%s: float operands whose rows are whole, aligned 8-element vectors", what);
+  return launch("aoto_generic_fused", dim3(grid_for(f.vectors)), dim3(256), 0, stream, f);
 }
 
 int aoto_hip_generic_reduce(int op, const aoto_tensor* out, const aoto_tensor* in, void* stream) {
@@ -1871,6 +2010,45 @@ int aoto_hip_generic_copy(const aoto_tensor* dst, const aoto_tensor* src, void* 
   args.ndim = dst->ndim;
   args.total = numel(dst);
   if (args.total == 0) return AOTO_OK;
+  if (args.src_dtype != args.dst_dtype && float_dtype(src->dtype) && float_dtype(dst->dtype) && contiguous(dst)) {
+    // a conversion between the float types into a contiguous tensor: the elementwise cast
+    aoto::EwArgs cast;
+    memset(&cast, 0, sizeof(cast));
+    cast.op = AOTO_EW_CAST;
+    cast.ndim = args.ndim;
+    cast.out_dtype = args.dst_dtype;
+    cast.total = args.total;
+    cast.out = args.dst;
+    cast.alpha = 1.0;
+    cast.in[0].data = args.src;
+    cast.in[0].dtype = args.src_dtype;
+    for (int d = 0; d < args.ndim; ++d) {
+      cast.shape[d] = args.shape[d];
+      cast.in[0].strides[d] = args.src_strides[d];
+    }
+    return launch_elementwise(cast, stream);
+  }
+  long long* walks[2] = {args.src_strides, args.dst_strides};
+  args.ndim = collapse_dims(args.ndim, args.shape, walks, 2);
+  const int unit = copy_unit(args);
+  char name[64];
+  snprintf(name, sizeof(name), "aoto_generic_copy_rows%d", unit);
+  if (unit > 0 && has_kernel(name)) {
+    const int es = element_bytes(args.src_dtype), last = args.ndim - 1;
+    aoto::CopyRowsArgs r;
+    memset(&r, 0, sizeof(r));
+    r.src = args.src;
+    r.dst = args.dst;
+    r.ndim = args.ndim;
+    r.units = (unsigned)(args.total * es / unit);
+    r.per_row = (unsigned)(args.shape[last] * es / unit);
+    for (int d = 0; d < last; ++d) {
+      r.shape[d] = (unsigned)args.shape[d];
+      r.src_strides[d] = args.src_strides[d] * es / unit;
+      r.dst_strides[d] = args.dst_strides[d] * es / unit;
+    }
+    return launch(name, dim3(grid_for(r.units)), dim3(256), 0, stream, r);
+  }
   return launch("aoto_generic_copy", dim3(grid_for(args.total)), dim3(256), 0, stream, args);
 }
 

@@ -220,13 +220,26 @@ AOTO_DEVICE bool compare_op(int op, double a, double b) {
   }
 }
 
+// The index along a dim of `extent`, taken off `rem` (below 2^31 elements in 32 bits: a 64-bit divide
+// is several times the instructions, once per dim and element).
+AOTO_DEVICE long long take_index(long long& rem, long long extent, bool small) {
+  if (small) {
+    const uint32_t r = (uint32_t)rem, q = r / (uint32_t)extent;
+    rem = q;
+    return r - q * (uint32_t)extent;
+  }
+  const long long c = rem % extent;
+  rem /= extent;
+  return c;
+}
+
 extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_elementwise(EwArgs a) {
   const long long stride = (long long)gridDim.x * kGenThreads;
+  const bool small = a.total < (1ll << 31);
   for (long long i = (long long)blockIdx.x * kGenThreads + threadIdx.x; i < a.total; i += stride) {
     long long rem = i, off0 = 0, off1 = 0, off2 = 0;
     for (int d = a.ndim - 1; d >= 0; --d) {
-      const long long c = rem % a.shape[d];
-      rem /= a.shape[d];
+      const long long c = take_index(rem, a.shape[d], small);
       off0 += c * a.in[0].strides[d];
       off1 += c * a.in[1].strides[d];
       off2 += c * a.in[2].strides[d];
@@ -252,6 +265,129 @@ extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_elementwi
       // where(cond, x, y): the selected value is copied exactly
       const bool c = operand_value(a.in[0], off0) != 0.0;
       store_double(a.out, a.out_dtype, i, c ? operand_value(a.in[1], off1) : operand_value(a.in[2], off2));
+    }
+  }
+}
+
+// Eight consecutive elements of an operand: stride 1 along the row (16-byte loads, two for f32), or one
+// value for all eight (stride 0, a scalar).
+AOTO_DEVICE void load_eight(const Operand& o, long long off, bool splat, float (&v)[8]) {
+  if (o.data == nullptr || splat) {
+    const float x = o.data == nullptr ? (float)o.value : load_float(o.data, o.dtype, off);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = x;
+  } else if (o.dtype == AOTO_DT_F32) {
+    const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(o.data) + off);
+    const float4 x = p[0], y = p[1];
+    v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w, v[4] = y.x, v[5] = y.y, v[6] = y.z, v[7] = y.w;
+  } else {
+    const uint4 r = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(o.data) + off);
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = bf16_lo(w[i]);
+      v[2 * i + 1] = bf16_hi(w[i]);
+    }
+  }
+}
+
+// f32 elementwise nodes, one or a chain of them, whose rows are whole 8-element vectors. Bound by memory:
+// the general kernel spends its time on per-element index divisions and typed 2-byte loads, and a chain
+// of nodes on writing and reading every intermediate (the bf16 gated MLP's silu(gate) * up, 2.5M elements,
+// captures as five nodes through f32: 80 us in five general launches, 15.6 us here). Every step's value
+// is rounded to its node's element type, so a chain's result has the bits of its nodes run one by one.
+extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_fused(FusedArgs a) {
+  const int last = a.ndim - 1;
+  for (unsigned c = blockIdx.x * kGenThreads + threadIdx.x; c < a.vectors; c += gridDim.x * kGenThreads) {
+    float in[kFusedInputs][8], reg[4][8];
+    const uint32_t row0 = c / a.per_row, col = (c - row0 * a.per_row) * 8u;
+#pragma unroll
+    for (int k = 0; k < kFusedInputs; ++k) {
+      if (k < a.inputs) {
+        const bool splat = a.in[k].strides[last] == 0;
+        long long off = splat ? 0 : col;
+        uint32_t row = row0;
+        for (int d = last - 1; d >= 0; --d) {
+          const uint32_t n = (uint32_t)a.shape[d], q = row / n;
+          off += (row - q * n) * a.in[k].strides[d];
+          row = q;
+        }
+        load_eight(a.in[k], off, splat, in[k]);
+      }
+    }
+    // (sources and destinations are the same for all lanes: the copies are scalar branches around eight moves)
+    auto source = [&](int s, float (&v)[8]) {
+#pragma unroll
+      for (int r = 0; r < 4 + kFusedInputs; ++r)
+        if (s == r) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[i] = r < 4 ? reg[r & 3][i] : in[r < 4 ? 0 : r - 4][i];
+        }
+    };
+    float r[8];
+    for (int s = 0; s < a.count; ++s) {
+      const FusedStep& step = a.steps[s];
+      float x[8], y[8];
+      source(step.a, x);
+      if (step.op < AOTO_EW_ADD) {
+        switch (step.op) {
+#define AOTO_FUSED_UNARY(OP)                                                  \
+  case OP:                                                                    \
+    _Pragma("unroll") for (int i = 0; i < 8; ++i) r[i] = unary_f32(OP, x[i]); \
+    break;
+          AOTO_FUSED_UNARY(AOTO_EW_NEG)
+          AOTO_FUSED_UNARY(AOTO_EW_ABS)
+          AOTO_FUSED_UNARY(AOTO_EW_RSQRT)
+          AOTO_FUSED_UNARY(AOTO_EW_EXP)
+          AOTO_FUSED_UNARY(AOTO_EW_SIGMOID)
+          AOTO_FUSED_UNARY(AOTO_EW_SILU)
+          AOTO_FUSED_UNARY(AOTO_EW_RELU)
+          AOTO_FUSED_UNARY(AOTO_EW_TANH)
+          AOTO_FUSED_UNARY(AOTO_EW_GELU_TANH)
+          AOTO_FUSED_UNARY(AOTO_EW_GELU)
+#undef AOTO_FUSED_UNARY
+          default:  // AOTO_EW_CAST
+#pragma unroll
+            for (int i = 0; i < 8; ++i) r[i] = x[i];
+        }
+      } else {
+        source(step.b, y);
+        switch (step.op) {
+#define AOTO_FUSED_BINARY(OP)                                                             \
+  case OP:                                                                                \
+    _Pragma("unroll") for (int i = 0; i < 8; ++i) r[i] = binary_f32(OP, x[i], y[i], step.alpha); \
+    break;
+          AOTO_FUSED_BINARY(AOTO_EW_ADD)
+          AOTO_FUSED_BINARY(AOTO_EW_SUB)
+          AOTO_FUSED_BINARY(AOTO_EW_DIV)
+          AOTO_FUSED_BINARY(AOTO_EW_MAXIMUM)
+          AOTO_FUSED_BINARY(AOTO_EW_MINIMUM)
+#undef AOTO_FUSED_BINARY
+          default:  // AOTO_EW_MUL
+#pragma unroll
+            for (int i = 0; i < 8; ++i) r[i] = x[i] * y[i];
+        }
+      }
+      if (step.round_bf16) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = round_bf16(r[i]);
+      }
+      if (s + 1 < a.count) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          if (step.dst == d) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) reg[d][i] = r[i];
+          }
+      }
+    }
+    if (a.out_dtype == AOTO_DT_F32) {
+      float4* p = reinterpret_cast<float4*>(static_cast<float*>(a.out) + 8ll * c);
+      p[0] = make_float4(r[0], r[1], r[2], r[3]);
+      p[1] = make_float4(r[4], r[5], r[6], r[7]);
+    } else {
+      reinterpret_cast<uint4*>(a.out)[c] = make_uint4(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]),
+                                                      pack_bf16x2(r[4], r[5]), pack_bf16x2(r[6], r[7]));
     }
   }
 }
@@ -504,17 +640,50 @@ extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_index(Ind
 
 extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_copy(CopyArgs a) {
   const long long stride = (long long)gridDim.x * kGenThreads;
+  const bool small = a.total < (1ll << 31);
+  // whole numbers stay whole (an f64 holds 53 of an int64's bits)
+  const bool whole = a.src_dtype >= AOTO_DT_I64 && a.dst_dtype >= AOTO_DT_I64;
   for (long long i = (long long)blockIdx.x * kGenThreads + threadIdx.x; i < a.total; i += stride) {
     long long rem = i, so = 0, dof = 0;
     for (int d = a.ndim - 1; d >= 0; --d) {
-      const long long c = rem % a.shape[d];
-      rem /= a.shape[d];
+      const long long c = take_index(rem, a.shape[d], small);
       so += c * a.src_strides[d];
       dof += c * a.dst_strides[d];
     }
-    store_double(a.dst, a.dst_dtype, dof, load_value(a.src, a.src_dtype, so));
+    if (whole)
+      store_int(a.dst, a.dst_dtype, dof, load_int(a.src, a.src_dtype, so));
+    else
+      store_double(a.dst, a.dst_dtype, dof, load_value(a.src, a.src_dtype, so));
   }
 }
+
+// A copy of one element type whose rows are contiguous on both sides, in the widest units that every
+// row start and length allow (clone, contiguous, cat and the transposes around attention heads).
+template <typename U>
+__device__ __forceinline__ void copy_rows_body(const CopyRowsArgs& a) {
+  const int last = a.ndim - 1;
+  for (unsigned c = blockIdx.x * kGenThreads + threadIdx.x; c < a.units; c += gridDim.x * kGenThreads) {
+    uint32_t row = c / a.per_row;
+    long long so = c - row * a.per_row, dof = so;
+    for (int d = last - 1; d >= 0; --d) {
+      const uint32_t q = row / a.shape[d], at = row - q * a.shape[d];
+      row = q;
+      so += at * a.src_strides[d];
+      dof += at * a.dst_strides[d];
+    }
+    static_cast<U*>(a.dst)[dof] = static_cast<const U*>(a.src)[so];
+  }
+}
+#define AOTO_COPY_ROWS(BYTES, U)                                                                             \
+  extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_copy_rows##BYTES(CopyRowsArgs a) { \
+    copy_rows_body<U>(a);                                                                                    \
+  }
+AOTO_COPY_ROWS(1, uint8_t)
+AOTO_COPY_ROWS(2, uint16_t)
+AOTO_COPY_ROWS(4, uint32_t)
+AOTO_COPY_ROWS(8, uint2)
+AOTO_COPY_ROWS(16, uint4)
+#undef AOTO_COPY_ROWS
 
 extern "C" __global__ __launch_bounds__(kGenThreads) void aoto_generic_fill(FillArgs a) {
   const long long stride = (long long)gridDim.x * kGenThreads;

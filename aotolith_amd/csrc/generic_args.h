@@ -31,6 +31,33 @@ struct EwArgs {
   Operand in[3];
 };
 
+// A chain of f32 elementwise nodes in one launch: a program over four registers and up to six operands.
+// Sources 0..3 are registers, 4..9 operands; the last instruction's value is the output.
+constexpr int kFusedInputs = 6, kFusedSteps = 16;
+struct FusedStep {
+  uint8_t op, dst, a, b;
+  int round_bf16;  // the node's own element type is bf16: its value is rounded as its store would be
+  float alpha;
+};
+struct FusedArgs {
+  Operand in[kFusedInputs];
+  FusedStep steps[kFusedSteps];
+  long long shape[kMaxDims];  // collapsed: dims that every operand walks as one are one
+  void* out;                  // contiguous
+  int inputs, count, ndim, out_dtype;
+  unsigned vectors, per_row;  // of eight elements, in all and along the last dim
+};
+
+// A copy of one element type in whole units of 1 to 16 bytes; strides and the row length in units.
+struct CopyRowsArgs {
+  const void* src;
+  void* dst;
+  int ndim;
+  unsigned units, per_row;
+  unsigned shape[kMaxDims];
+  long long src_strides[kMaxDims], dst_strides[kMaxDims];
+};
+
 // Row reduction / scan over a [rows, len] view.
 struct ReduceArgs {
   int op;

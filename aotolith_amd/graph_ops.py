@@ -115,6 +115,19 @@ def launch_elementwise(op: int, out: torch.Tensor, a, b=None, c=None, alpha: flo
     return out
 
 
+def launch_fused(out: torch.Tensor, inputs: list, program, alphas, count: int) -> bool:
+    """A chain of elementwise steps; False where the operands' rows are not whole vectors (nothing is launched)."""
+
+    do, descs = describe(out), [describe(x) for x in inputs]
+    array = (ctypes.c_void_p * len(descs))(*[_addressof(d) for d in descs])
+    status = _lib.library().aoto_hip_generic_fused(_p(do), _addressof(array), len(descs), _addressof(program),
+                                                   _addressof(alphas), count, _stream())
+    if status == _lib.AOTO_ERR_UNSUPPORTED:
+        return False
+    _lib.check(status)
+    return True
+
+
 def launch_copy(dst: torch.Tensor, src: torch.Tensor) -> torch.Tensor:
     dd, ds = describe(dst), describe(src)
     _lib.check(_lib.library().aoto_hip_generic_copy(_p(dd), _p(ds), _stream()))
@@ -249,7 +262,12 @@ NEWER = {"matmul": ("aoto_generic_gemm_f32_a_t1k1", "aoto_generic_gemm_*",
                     "strided batched GEMM on the matrix cores, LDS-staged tiles, f32 accumulation"),
          "attention": ("aoto_generic_attention_f32_d64_a", "aoto_generic_attention*",
                        "legalized scaled-dot-product attention (bool/float mask, causal, GQA) on the matrix cores, "
-                       "f32 softmax")}
+                       "f32 softmax"),
+         "elementwise": ("aoto_generic_fused", "aoto_generic_{fused,elementwise}",
+                         "strided broadcasting elementwise kernel (eight elements a thread where rows allow), f32 "
+                         "compute, one rounding to the output type"),
+         "copy": ("aoto_generic_fused", "aoto_generic_{copy,copy_rows*,fused}",
+                  "strided copy with element-type conversion (whole 1- to 16-byte units where rows allow)")}
 REASONS = {
     "elementwise": "strided broadcasting elementwise kernel, f32 compute, one rounding to the output type",
     "reduction": "row reduction / scan over the (permuted) last dim, f32 or int64 accumulation",
@@ -291,6 +309,142 @@ def _value(env, arg):
     return arg
 
 
+#: Elementwise node ops with a step in the fused kernel.
+_FUSED_UNARY = {op: name for op, name in UNARY_OPS.items()
+                if name in ("neg", "abs", "rsqrt", "exp", "sigmoid", "silu", "relu", "tanh")}
+_FUSED_BINARY = {op: name for op, name in BINARY_OPS.items() if name in ("add", "sub", "mul", "div", "maximum")}
+_FUSED_BINARY["aten.minimum.default"] = "minimum"
+_FLOATS = (torch.float32, torch.bfloat16)
+_MAX_FUSED_INPUTS, _MAX_FUSED_STEPS, _FUSED_REGISTERS = 6, 16, 4
+
+
+class FusedChain:
+    """Elementwise nodes that run as one launch: every member but the last feeds members only.
+
+    Members have one shape; each step rounds to its node's element type, so the chain's bits are those of
+    its nodes run one by one (which is what happens where a layout has no whole vectors).
+    """
+
+    def __init__(self, members: list[Node], inputs: list, steps: list[tuple], alphas: list[float]):
+        self.members, self.root = members, members[-1]
+        self.inputs = inputs
+        self.count = len(steps)
+        self.program = (ctypes.c_int32 * (5 * len(steps)))(*[field for step in steps for field in step])
+        self.alphas = (ctypes.c_double * len(steps))(*alphas)
+
+
+def _fused_step(node: Node, meta) -> tuple[int, list, float] | None:
+    """``(op code, operands, alpha)`` of a node the fused kernel has a step for, else None."""
+
+    if node.shape is None or node.dtype not in _FLOATS:
+        return None
+    alpha = 1.0
+    if node.op in _FUSED_UNARY:
+        code, operands = EW[_FUSED_UNARY[node.op]], list(node.args[:1])
+    elif node.op == "aten._to_copy.default":
+        code, operands = EW["cast"], list(node.args[:1])
+    elif node.op == "aten.gelu.default":
+        approximate = node.kwargs.get("approximate", node.args[1] if len(node.args) > 1 else "none")
+        code, operands = EW["gelu_tanh" if approximate == "tanh" else "gelu"], list(node.args[:1])
+    elif node.op in _FUSED_BINARY:
+        name = _FUSED_BINARY[node.op]
+        code, operands = EW[name], list(node.args[:2])
+        if name in ("add", "sub"):
+            alpha = float(node.args[2] if len(node.args) > 2 else node.kwargs.get("alpha", 1))
+    else:
+        return None
+    for operand in operands:
+        if isinstance(operand, Ref):
+            shape, dtype = meta.get(operand.name, (None, None))
+            if dtype not in _FLOATS:
+                return None
+            if len(operands) == 1 and tuple(shape) != tuple(node.shape):
+                return None
+        elif isinstance(operand, bool) or not isinstance(operand, (int, float)):
+            return None
+    return code, operands, alpha
+
+
+def _chain(members: list[Node], steps: dict) -> FusedChain | None:
+    """The members (in graph order, the root last) as a program, or None past its operands, steps or registers."""
+
+    names = {node.name for node in members}
+    inputs: list = []
+    last_use: dict[str, int] = {}
+    for index, node in enumerate(members):
+        for operand in steps[node.name][1]:
+            if isinstance(operand, Ref) and operand.name in names:
+                last_use[operand.name] = index
+            elif operand not in inputs:
+                inputs.append(operand)
+    if len(inputs) > _MAX_FUSED_INPUTS or len(members) > _MAX_FUSED_STEPS:
+        return None
+    register: dict[str, int] = {}
+    free = list(range(_FUSED_REGISTERS))
+    program, alphas = [], []
+    for index, node in enumerate(members):
+        code, operands, alpha = steps[node.name]
+        sources = [register[o.name] if isinstance(o, Ref) and o.name in names else 4 + inputs.index(o) for o in operands]
+        for name in {o.name for o in operands if isinstance(o, Ref) and o.name in names}:
+            if last_use[name] == index:
+                free.append(register[name])
+        if not free:
+            return None
+        register[node.name] = free.pop()
+        program.append((code, register[node.name], sources[0], sources[-1], DTYPE_CODES[node.dtype]))
+        alphas.append(alpha)
+    return FusedChain(members, inputs, program, alphas)
+
+
+def fuse_elementwise(graph: LoweredGraph) -> list[FusedChain]:
+    """Chains of two or more elementwise nodes of one shape whose inner values nothing else reads."""
+
+    meta = {name: (tuple(t.shape), t.dtype) for name, t in graph.state.items() if isinstance(t, torch.Tensor)}
+    meta.update(graph.input_meta)
+    meta.update({node.name: (node.shape, node.dtype) for node in graph.nodes})
+    steps = {node.name: step for node in graph.nodes if (step := _fused_step(node, meta)) is not None}
+    order = {node.name: i for i, node in enumerate(graph.nodes)}
+    readers: dict[str, set] = {}
+
+    def note(value, reader):
+        if isinstance(value, Ref):
+            readers.setdefault(value.name, set()).add(reader)
+        elif isinstance(value, (list, tuple)):
+            for item in value:
+                note(item, reader)
+        elif isinstance(value, dict):
+            note(list(value.values()), reader)
+
+    for node in graph.nodes:
+        note(node.args, node.name)
+        note(node.kwargs, node.name)
+    note(graph.outputs, None)
+    taken: set[str] = set()
+    chains = []
+    for root in reversed(graph.nodes):
+        if root.name not in steps or root.name in taken:
+            continue
+        members, chain = [root], None
+        rejected: set[str] = set()
+        while True:
+            names = {node.name for node in members}
+            candidates = [o.name for node in members for o in steps[node.name][1]
+                          if isinstance(o, Ref) and o.name in steps and o.name not in names | taken | rejected
+                          and tuple(meta[o.name][0]) == tuple(root.shape) and readers[o.name] <= names]
+            if not candidates:
+                break
+            grown = sorted(members + [graph.nodes[order[candidates[0]]]], key=lambda node: order[node.name])
+            attempt = _chain(grown, steps)
+            if attempt is None:
+                rejected.add(candidates[0])
+            else:
+                members, chain = grown, attempt
+        if chain is not None:
+            taken.update(node.name for node in members)
+            chains.append(chain)
+    return chains
+
+
 class GraphRunner:
     """Runs a lowered graph's nodes on the current GPU, one generic kernel per compute node."""
 
@@ -299,9 +453,17 @@ class GraphRunner:
         self.device = device
         self.state = {name: tensor.detach().to(device).contiguous() if isinstance(tensor, torch.Tensor) else tensor
                       for name, tensor in graph.state.items()}
+        chains = (fuse_elementwise(graph) if _lib.library().aoto_hip_has_kernel(b"aoto_generic_fused") else [])
+        #: node name -> its chain; a chain runs where its last member stands
+        self.chains = {node.name: chain for chain in chains for node in chain.members}
         self.handlers: list[tuple[Node, Callable]] = []
         for node in graph.nodes:
-            self.handlers.append((node, self._handler(node)))
+            handler = self._handler(node)
+            chain = self.chains.get(node.name)
+            if chain is None:
+                self.handlers.append((node, handler))
+            elif chain.root is node:
+                self.handlers.append((node, lambda env, node, chain=chain: self._fused(env, chain)))
         self.error = None
         # only gathers can meet an index out of range: a graph without one has no flag to set or read back
         self.gathers = any(node.op in INDEX_OPS for node in graph.nodes)
@@ -318,6 +480,14 @@ class GraphRunner:
             if node.is_view:
                 continue
             family = FAMILIES[node.op]
+            if node.name in self.chains:
+                out.append(KernelSelection(
+                    op_index=len(out), op=node.op.split(".")[1], output_id=node.name, implementation="hip_kernel",
+                    kind=family, reason="a step of the elementwise chain launched for "
+                                        f"{self.chains[node.name].root.name} (f32 compute, rounded to its own type)",
+                    artifact_name="aoto_generic_fused", device_name=device_name, device_architecture=ARCHITECTURE,
+                ))
+                continue
             out.append(KernelSelection(
                 op_index=len(out), op=node.op.split(".")[1] if node.op.startswith("aten.") else node.op,
                 output_id=node.name, implementation="hip_kernel", kind=family, reason=reasons[family],
@@ -369,6 +539,15 @@ class GraphRunner:
             return getattr(self, "_" + OTHER_OPS[op])
         raise CompilationError(f"node {node.name}: {op} has no gfx950 kernel in this backend",
                                hint="compile_callable/compile_module lower core-ATen graphs of the supported op set")
+
+    def _fused(self, env, chain: FusedChain):
+        out = self._out(chain.root)
+        inputs = [_value(env, x) for x in chain.inputs]
+        if launch_fused(out, inputs, chain.program, chain.alphas, chain.count):
+            return out
+        for node in chain.members:  # no whole vectors here: node by node
+            env[node.name] = self._handler(node)(env, node)
+        return env[chain.root.name]
 
     def _out(self, node: Node) -> torch.Tensor:
         if node.shape is None or node.dtype is None:

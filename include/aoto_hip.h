@@ -521,6 +521,14 @@ typedef struct aoto_tensor {
 int aoto_hip_generic_elementwise(int op, const aoto_tensor* out, const aoto_tensor* a, const aoto_tensor* b,
                                  const aoto_tensor* c, double alpha, void* stream);
 
+/* A chain of f32 elementwise ops in one launch. `program` holds count x {op, register written (0..3),
+ * first source, second source (binary ops), element type the step's value is rounded to}; sources
+ * 0..3 are registers already written, 4.. the operands (each broadcast to out, or a scalar). The last
+ * step's value goes to the contiguous `out`. AOTO_ERR_UNSUPPORTED where the operands' rows are not whole,
+ * 16-byte aligned vectors of eight elements: run the nodes one by one. */
+int aoto_hip_generic_fused(const aoto_tensor* out, const aoto_tensor* const* inputs, int input_count,
+                           const int32_t* program, const double* alphas, int count, void* stream);
+
 /* Row reductions and scans over the last dim of `in` (its leading dims must
  * collapse to one stride): SUM, MEAN, AMAX, AMIN, ANY, ALL, ARGMAX, ARGMIN
  * write out[rows]; SOFTMAX, LOG_SOFTMAX, CUMSUM write out[rows, len].

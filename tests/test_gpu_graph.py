@@ -321,3 +321,102 @@ def test_attention_over_its_tiles_layouts_masks_and_types(batch, heads, kv_heads
         assert torch.equal(got[got.isinf()], want[want.isinf()])
         bound = (4 * exponent + (lk + 16) * 2.0 ** -24) * size + eps * want.abs()
         assert bool(((got - want).abs() <= bound)[fine].all())
+
+
+def _views(gen, dtype):
+    """Pairs of operands of one broadcast shape: collapsible, broadcast, permuted, offset and odd-sized."""
+
+    def t(*shape):
+        return (torch.randn(*shape, generator=gen) * 3).to(dtype).cuda()
+
+    yield t(1, 7, 64), t(1, 7, 64)
+    yield t(3, 5, 16), t(16)
+    yield t(3, 5, 16), t(5, 1)
+    yield t(2, 3, 4, 24), t(1, 1, 4, 24)
+    yield t(2, 4, 3, 24).transpose(1, 2), t(2, 3, 4, 24)
+    yield t(6, 40)[:, 8:32], t(6, 24)
+    yield t(6, 40)[:, 3:27], t(6, 24)
+    yield t(24, 6).t(), t(6, 24)
+    yield t(5, 9), t(5, 9)
+    yield t(1), t(1)
+    yield t(300, 1024), t(300, 1024)
+    yield t(2, 8).unsqueeze(1).expand(2, 3, 8), t(3, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_elementwise_and_copies_over_strides_and_sizes(dtype):
+    """The vector kernels and the general ones give torch's values, bit for bit, on every kind of view."""
+
+    from aotolith_amd.graph_ops import EW, launch_copy, launch_elementwise
+
+    gen = torch.Generator().manual_seed(5)
+    other = torch.bfloat16 if dtype == torch.float32 else torch.float32
+    for x, y in _views(gen, dtype):
+        shape = torch.broadcast_shapes(x.shape, y.shape)
+        for name, fn in (("add", torch.add), ("mul", torch.mul), ("sub", torch.sub), ("div", torch.div),
+                         ("maximum", torch.maximum)):
+            for out_type in (dtype, other):
+                out = torch.empty(shape, dtype=out_type, device="cuda")
+                launch_elementwise(EW[name], out, x, y)
+                want = fn(x.float(), y.float()).to(out_type)
+                assert torch.equal(out, want), (name, tuple(x.shape), x.stride(), out_type)
+        for name, fn in (("neg", torch.neg), ("relu", torch.relu), ("abs", torch.abs)):
+            out = torch.empty(x.shape, dtype=dtype, device="cuda")
+            assert torch.equal(launch_elementwise(EW[name], out, x), fn(x)), (name, x.stride())
+        scaled = launch_elementwise(EW["mul"], torch.empty(x.shape, dtype=dtype, device="cuda"), x, 0.5)
+        assert torch.equal(scaled, x * 0.5)
+        for out_type in (dtype, other):
+            assert torch.equal(launch_copy(torch.empty(x.shape, dtype=out_type, device="cuda"), x), x.to(out_type))
+        wide = torch.zeros(*x.shape[:-1], x.shape[-1] + 9, dtype=dtype, device="cuda")
+        for start in (8, 1):
+            launch_copy(wide[..., start:start + x.shape[-1]], x)
+            assert torch.equal(wide[..., start:start + x.shape[-1]], x) and bool((wide[..., 0] == 0).all())
+            wide.zero_()
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32, torch.bool, torch.uint8, torch.int8])
+def test_copies_of_whole_numbers_keep_their_bits(dtype):
+    from aotolith_amd.graph_ops import launch_copy
+
+    gen = torch.Generator().manual_seed(6)
+    x = torch.randint(0, 2 if dtype == torch.bool else 100, (3, 5, 16), generator=gen).to(dtype).cuda()
+    if dtype == torch.int64:
+        x += (1 << 60) + 1
+    for view in (x, x.transpose(0, 1), x[..., 1:14], x[..., ::3], x.permute(2, 0, 1)):
+        assert torch.equal(launch_copy(torch.empty(view.shape, dtype=dtype, device="cuda"), view), view)
+
+
+@pytest.mark.parametrize("width", [64, 60])
+def test_fused_chains_keep_the_bits_of_their_nodes(width):
+    """Chains (gated MLP through f32, rotary mix, broadcast, scalars, a value read twice) against the same nodes run
+    one by one: equal bits, on whole vectors and on rows that have none."""
+
+    import aotolith_amd as aoto
+    from aotolith_amd.graph_ops import GraphRunner
+
+    def fn(gate, up, cos, sin, x):
+        act = torch.nn.functional.silu(gate) * up
+        mix = x * cos + torch.sigmoid(x) * sin
+        tail = torch.tanh((act - mix) * 0.5) / (mix.abs() + 1.0)
+        return act, torch.maximum(tail + act, -x)
+
+    gen = torch.Generator().manual_seed(11)
+
+    def t(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, generator=gen).to(dtype)
+
+    inputs = (t(3, 50, width), t(3, 50, width), t(50, width), t(50, width), t(3, 50, width))
+    result = aoto.compile_callable(fn, inputs, target="hip-gfx950")
+    device = torch.device("cuda", torch.cuda.current_device())
+    runner = GraphRunner(result.lowered_graph, device)
+    plain = GraphRunner(result.lowered_graph, device)
+    assert runner.chains
+    plain.chains = {}
+    plain.handlers = [(node, plain._handler(node)) for node in result.lowered_graph.nodes]
+    bound = dict(zip(result.lowered_graph.inputs, (x.cuda() for x in inputs)))
+    for got, want in zip(runner.run(bound), plain.run(bound)):
+        assert torch.equal(got, want)
+    for got, want in zip(result.plan(*inputs), fn(*(x.float() for x in inputs))):
+        assert torch.allclose(got.cpu().float(), want, atol=0.06, rtol=0.03)  # a handful of bf16 roundings
+    names = {s.artifact_name for s in result.plan.selections}
+    assert "aoto_generic_fused" in names
