@@ -20,6 +20,15 @@ from tests.test_graph_capture import _compare, _flat
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def _code_object():
+    """The launchers below are called on their own, without a compile that would install the kernels."""
+
+    from aotolith_amd import _lib
+
+    _lib.ensure_code_object()
+
+
 def _host(values):
     out = []
     for v in values:
