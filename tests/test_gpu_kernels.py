@@ -604,3 +604,29 @@ def test_matmul_qkv_rope_equals_matmul_then_rope(m, hq, hkv, dim, k, splits, bia
     assert_bf16_parity(got_pair[0, :, :, slot0:slot0 + m], oracle.rope(heads[:, hq:hq + hkv], c, s_), max_ulp=1.0)
     np.testing.assert_array_equal(got_pair[1, :, :, slot0:slot0 + m], from_gpu_bf16(y).reshape(
         m, hq + 2 * hkv, dim).transpose(1, 0, 2)[None, hq + hkv:])
+
+
+@pytest.mark.parametrize("n", [8, 56, 8192, 32768, 32776, 151936])
+def test_argmax_at_chunk_edges_with_ties_signs_and_nans(n):
+    """Rows around the loop's 8, 8192 and 32768 elements: ties go to the first index, +0 beats -0, NaN never wins,
+    an all-NaN row gives index 0; a row start that is not 16-byte aligned gives the same indices."""
+
+    gen = torch.Generator().manual_seed(n)
+    rows = torch.randn(8, n, generator=gen).to(torch.bfloat16)
+    rows[1] = -rows[1].abs() - 1
+    rows[2] = 0.0
+    rows[2, ::2] = -0.0  # +0 first at index 1
+    rows[3] = float("nan")
+    rows[4, : n // 2] = float("nan")
+    rows[5] = float("-inf")
+    rows[6, n - 1] = rows[6, n // 3] = 100.0
+    rows[7] = float("-inf")
+    rows[7, n // 2:] = float("nan")
+    bits = rows.view(torch.int16).to(torch.int64) & 0xFFFF
+    key = torch.where(bits >= 0x8000, 0xFFFF - bits, bits + 0x8000)
+    key[rows.isnan()] = 0
+    want = torch.tensor([int((row == row.max()).nonzero()[0]) for row in key])
+    logits = rows.cuda()
+    assert torch.equal(_ops().argmax(logits).cpu(), want)
+    shifted = torch.empty(8 * n + 1, dtype=torch.bfloat16, device="cuda")[1:].view(8, n).copy_(logits)
+    assert torch.equal(_ops().argmax(shifted).cpu(), want)
