@@ -368,6 +368,8 @@ def w8_matmul(
 
 #: From this many rows (with K % 256 == 0) the prefill GEMMs' automatic plan
 #: (tile = splits = 0) takes the wide-tile 32x32x16-MFMA kernel (the C ABI's kWideRows).
+#: Where neither this rule nor :func:`lds_plan` applies, the C ABI picks among all instances
+#: with a cost model (``modelled_plan`` in ``csrc/aoto_hip.cpp``).
 WIDE_ROWS = 512
 
 

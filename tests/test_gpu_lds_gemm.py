@@ -375,3 +375,77 @@ def test_lds_tiles_refuse_what_they_cannot_run():
     packed8, scales8 = pack_weight_bits_bf16(bf16_normal(rng, (256, 512), 0.02), 64, 8)
     with pytest.raises(HipKernelError, match="tile 822"):
         ops.w8_matmul(x, torch.from_numpy(packed8).cuda(), to_gpu_bits(scales8), 64, tile=822)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k,group", [(1, 896, 896, 64), (17, 896, 4864, 64), (33, 400, 1024, 64), (129, 1152, 896, 64),
+                                         (255, 2048, 5504, 32), (257, 896, 896, 64), (300, 1008, 1088, 64),
+                                         (333, 4096, 4096, 128), (511, 2560, 2048, 64), (700, 528, 960, 64),
+                                         (1030, 1152, 896, 64), (300, 896, 960, 192)])
+def test_modelled_plans_match_one_fixed_plan_and_fit_their_workspace(m, n, k, group, bits):
+    """Row counts and reductions outside the fixed rules, at tile and slice remainders, odd group counts and a group
+    that is not a power of two: every form under automatic codes against unsplit 64 x 64 tiles (the same f32
+    products in another order: one bf16 ulp), writing nothing past the queried workspace."""
+
+    from aotolith_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(*shape, generator=gen, device="cuda") * std).bfloat16()
+
+    packed, scales = ops.quantize(normal(n, k, std=0.02), group, bits)
+    up = ops.quantize(normal(n, k, std=0.02), group, bits)
+    x, residual, weight, bias = normal(m, k), normal(m, n), normal(n), normal(n)
+    matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
+    gate_up = ops.w4_matmul_gate_up if bits == 4 else ops.w8_matmul_gate_up
+
+    def workspace(size):
+        whole = torch.full((size // 4 + 4096,), 7.25, device="cuda")
+        return whole, whole[:size // 4]
+
+    # Two orders of one f32 sum: K / 8 roundings each of partial sums below six deviations of the result
+    # (0.02 sqrt(K)), times what the epilogue multiplies them by, then a bf16 ulp (2^-7) where they round
+    # apart - small results of cancelling sums are many of their own ulps apart.
+    order = 2 * (k / 8) * 2.0 ** -24 * 6 * 0.02 * k ** 0.5
+
+    def check(got, want, factor=1.0, ulps=1.0):
+        room = order * factor + ulps * 2.0 ** -7 * want.float().abs()
+        assert bool(((got.float() - want.float()).abs() <= room).all())
+
+    whole, room = workspace(ops.gemm_workspace_bytes(m, n, k))
+    check(matmul(x, packed, scales, group, bias=bias, workspace=room),
+          matmul(x, packed, scales, group, bias=bias, tile=14, splits=1))
+    gate = normal(m, n)
+    check(matmul(x, packed, scales, group, gate=gate, workspace=room),
+          matmul(x, packed, scales, group, gate=gate, tile=14, splits=1), factor=float(gate.abs().max()))
+    if n <= 4096 and n % 8 == 0:
+        got = ops.matmul_residual_norm(x, packed, scales, group, residual, weight, 1e-6, bits=bits, workspace=room)
+        want = ops.matmul_residual_norm(x, packed, scales, group, residual, weight, 1e-6, bits=bits, tile=14, splits=1)
+        check(got[0], want[0])
+    assert bool((whole[room.numel():] == 7.25).all())
+    whole, room = workspace(ops.gate_up_workspace_bytes(m, n, k))
+    got = gate_up(x, packed, scales, *up, group, workspace=room)
+    want = gate_up(x, packed, scales, *up, group, tile=14, splits=1)
+    # the gate is rounded to bf16 before the silu, whose slope times the gate is at most (1 + |gate|) of its value
+    top = 6 * 0.02 * k ** 0.5
+    check(got, want, factor=2 * top, ulps=2 + top)
+    assert bool((whole[room.numel():] == 7.25).all())
+    for dim in (64, 128):
+        heads = n // dim - 2
+        if n % dim or heads < 1:
+            continue
+        size = int(_lib.library().aoto_hip_w4_gemm_qkv_rope_workspace(m, k, 0, 0, heads, 1, dim))
+        whole, room = workspace(size)
+        positions = torch.arange(m, device="cuda")
+        cos, sin = normal(m + 3, dim), normal(m + 3, dim)
+        results = []
+        for plan in (dict(workspace=room), dict(tile=14, splits=1)):
+            pair = torch.full((2, 1, 1, m + 3, dim), 7.0, dtype=torch.bfloat16, device="cuda")
+            y, q = ops.matmul_qkv_rope(x, packed, scales, group, positions, cos, sin, pair, query_heads=heads,
+                                       kv_heads=1, head_dim=dim, slot0=3, bias=bias, bits=bits, **plan)
+            results.append((y, q, pair))
+        check(results[0][0], results[1][0])
+        for a, b in zip(results[0][1:], results[1][1:]):  # two rotated bf16 values, each an ulp off at most
+            assert float((a.float() - b.float()).abs().max()) <= 2.0 ** -6 * float(b.float().abs().max())
+        assert bool((whole[room.numel():] == 7.25).all())
