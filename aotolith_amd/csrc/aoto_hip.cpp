@@ -1435,6 +1435,31 @@ int decode_attention_plan(const char* what, int batch, int query_heads, int kv_h
   return AOTO_OK;
 }
 
+// Whether a split window runs with the query heads of a kv head sharing a block (decode.h): the heads per
+// block (the largest divisor of the group up to 16), 0 for one head a block, and the split count and chunk:
+// one block per CU, whole 128-key tiles or more, and never more splits than the one-head plan's, whose
+// records the workspace holds. From 2048 keys at D = 64 and 4096 at D = 128, where the shared pass is ahead
+// of its longer prologue (split + merge, us, one head -> shared, the windows below / at / above the line):
+// 14 over 2 heads of 64, 1536 / 2304 / 4096 keys 9.1 / 10.1 / 11.4 -> 8.9 / 9.0 / 9.3; 28 over 4, 1536 / 4096 /
+// 16384 8.6 / 10.5 / 20.7 -> 9.0 / 10.6 / 14.3; 32 over 8 heads of 128, 2304 / 4096 / 8192 / 16384 10.3 / 13.7 /
+// 23.5 / 44.0 -> 12.0 / 13.3 / 15.9 / 22.2. Two blocks per CU's worth of splits run in two rounds (24.1 us at 8192).
+int grouped_decode(int batch, int query_heads, int kv_heads, int capacity, int head_dim, int requested, int* splits,
+                   int* chunk) {
+  if (requested > 0 || *splits <= 1 || capacity < (head_dim == 64 ? 2048 : 4096)) return 0;
+  const int group = query_heads / kv_heads;
+  int gb = group < 16 ? group : 16;
+  while (group % gb != 0) --gb;
+  if (gb < 2) return 0;
+  const long long rows = (long long)batch * query_heads / gb;
+  long long s = (cu_count() + rows - 1) / rows;
+  const long long tiles = (capacity + 127) / 128;
+  if (s > tiles) s = tiles;
+  if (s > *splits) s = *splits;
+  *chunk = (int)((capacity + s - 1) / s);
+  *splits = (capacity + *chunk - 1) / *chunk;
+  return gb;
+}
+
 int launch_merge(int rows, int splits, int head_dim, void* workspace, void* out, void* stream) {
   return launch("aoto_decode_attention_merge", dim3(rows), dim3(128), 0, stream, (const float*)workspace, splits,
                 head_dim, out);
@@ -1459,6 +1484,18 @@ int aoto_hip_decode_attention(const void* q, const void* keys, const void* value
   if (!aligned16(q) || !aligned16(keys) || !aligned16(values) || (kv_head_stride % 8) || (kv_batch_stride % 8))
     return fail(AOTO_ERR_ARGUMENT, "decode_attention: q/keys/values must be 16-byte aligned");
   char name[64];
+  int gs = s, gchunk = chunk;
+  if (const int gb = grouped_decode(batch, query_heads, kv_heads, capacity, head_dim, splits, &gs, &gchunk)) {
+    snprintf(name, sizeof(name), "aoto_decode_attention_d%d_g", head_dim);
+    if (has_kernel(name)) {
+      if (int st = launch(name, dim3(gs, batch * query_heads / gb), dim3(256), 0, stream, q, keys, values,
+                          (long long)kv_batch_stride, (long long)kv_head_stride, mask, mask_batch_stride, valid,
+                          ring_offset, capacity, query_heads, kv_heads, gb, scale, gchunk, (float*)workspace, step_state,
+                          out))
+        return st;
+      return gs > 1 ? launch_merge(batch * query_heads, gs, head_dim, workspace, out, stream) : AOTO_OK;
+    }
+  }
   const AttnShape as = attention_shape(head_dim, chunk);
   snprintf(name, sizeof(name), "aoto_decode_attention_d%d_w%dj%d", head_dim, as.waves, as.loads);
   if (int st = launch(name, dim3(s, batch * query_heads), dim3(64 * as.waves), 0, stream, q, keys, values,
@@ -1501,10 +1538,22 @@ int aoto_hip_decode_rope_attention(const void* row, int row_width, int query_sta
     return fail(AOTO_ERR_UNSUPPORTED, "decode_rope_attention: heads, row width < 65536, capacity < 2^22 and "
                 "strides < 2^31 elements needed");
   char name[64];
-  const AttnShape as = attention_shape(head_dim, chunk);
-  snprintf(name, sizeof(name), "aoto_decode_rope_attention_d%d_w%dj%d", head_dim, as.waves, as.loads);
   const int heads = query_heads | (kv_heads << 16), starts_qk = query_start | (key_start << 16);
   const int start_v_width = value_start | (row_width << 16), chunk_cap = chunk | (capacity << 9);
+  int gs = s, gchunk = chunk;
+  if (const int gb = grouped_decode(batch, query_heads, kv_heads, capacity, head_dim, splits, &gs, &gchunk)) {
+    snprintf(name, sizeof(name), "aoto_decode_rope_attention_d%d_g", head_dim);
+    if (has_kernel(name)) {
+      if (int st = launch(name, dim3(gs, batch * query_heads / gb), dim3(256), 0, stream, row, rope_rows, keys, values,
+                          (int)kv_head_stride, (int)kv_batch_stride, heads, starts_qk, start_v_width, capacity, gchunk, gb,
+                          valid, ring_offset, position, slot, scale, (float*)workspace, step_state, cos_table,
+                          sin_table, out))
+        return st;
+      return gs > 1 ? launch_merge(batch * query_heads, gs, head_dim, workspace, out, stream) : AOTO_OK;
+    }
+  }
+  const AttnShape as = attention_shape(head_dim, chunk);
+  snprintf(name, sizeof(name), "aoto_decode_rope_attention_d%d_w%dj%d", head_dim, as.waves, as.loads);
   if (int st = launch(name, dim3(s, batch * query_heads), dim3(64 * as.waves), 0, stream, row, rope_rows, keys,
                       values, (int)kv_head_stride, (int)kv_batch_stride, heads, starts_qk, start_v_width, chunk_cap,
                       valid, ring_offset, position, slot, scale, (float*)workspace, step_state, cos_table, sin_table,

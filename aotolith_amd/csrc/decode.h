@@ -11,6 +11,8 @@
 
 namespace aoto {
 
+typedef short group_s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) group_s16x4 group_lds_s16x4;
 typedef short i16x2_t __attribute__((ext_vector_type(2)));
 
 // x * cos + rotate_half(x) * sin for one element, f32, one rounding
@@ -361,6 +363,254 @@ __device__ void decode_attention_body(const uint16_t* __restrict__ q, const uint
   }
 }
 
+// The same attention with the query heads of a kv head sharing one pass over its window, on the matrix
+// cores, for windows long enough to be split: the one-head form above streams each kv head's keys and values
+// once per query head (four times for 32 query heads over 8) and spends ~1.2 us of VALU per 128 keys and head.
+// A block is one split of `gb` (up to 16) query heads of one kv head, 4 waves; a wave takes 32 keys of each
+// 128-key tile:
+//   S^T [keys x 16 heads] = K . Q^T   v_mfma_f32_16x16x32_bf16, K straight from global memory in operand
+//                                     order (16 rows of 64 bytes a load), Q rotated in registers
+//   O^T [d x 16 heads] += V^T . P^T   V through the wave's own LDS (transposing reads); the slots of the
+//                                     product hold the keys in S^T's accumulator order for both operands
+// P keeps its f32 precision as three bf16 terms (8 + 8 + 8 bits), three products into one f32 sum. Lane l
+// owns head l % 16 in both products, so a head's running maximum and sum stay in its four lanes. The next
+// tile's loads are issued as soon as the current registers are free; a block walks its split's tiles, so the
+// split count follows the chip and not the register file, and the merge reads fewer records.
+// Bound: HBM / L2 (3 TB/s of the window at 16384 keys), then the merge launch. 32 heads over 8, D = 128, split
+// and merge: 8192 keys 23.5 -> 15.9 us, 16384 keys 44.0 -> 22.2.
+template <int D, bool FUSED, bool ROWS>
+__device__ __forceinline__ void decode_attention_group_body(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ row, int row_width, int query_start, int key_start,
+    int value_start, const uint16_t* __restrict__ cos_table, const uint16_t* __restrict__ sin_table,
+    uint16_t* __restrict__ kbase, uint16_t* __restrict__ vbase, long long kv_batch_stride, long long kv_head_stride,
+    const uint8_t* __restrict__ mask, int mask_batch_stride, int valid, int ring_offset, int position, int slot, int cap,
+    int query_heads, int kv_heads, int gb, float scale, int chunk, float* __restrict__ partials,
+    const int* __restrict__ step, const uint16_t* __restrict__ rope_rows, uint16_t* __restrict__ out) {
+  constexpr int WAVES = 4, WK = 32, TILE = WAVES * WK;
+  constexpr int DC = D / 32;           // 32-dim operand chunks of a row
+  constexpr int DT = D / 16;           // 16-dim tiles of O^T
+  constexpr int LPK = D / 8;           // lanes (16-byte chunks) of a V row
+  constexpr int VL = WK * LPK / 64;    // V chunks a lane stages
+  constexpr int STR = D + 16;          // bf16 of a staged V row
+  __shared__ __attribute__((aligned(16))) uint16_t s_v[WAVES][WK * STR];
+  __shared__ __attribute__((aligned(16))) float s_o[WAVES][16][D];
+  __shared__ float s_m[WAVES][16], s_l[WAVES][16];
+
+  const int split = blockIdx.x, splits = gridDim.x;
+  const int per_row = query_heads / gb;
+  const int b = blockIdx.y / per_row, h0 = blockIdx.y % per_row * gb;
+  const int group = query_heads / kv_heads, kvh = h0 / group;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, quad = lane >> 4;
+  const int head = min(col, gb - 1);  // columns past the group repeat its last head and are not stored
+  const int s0 = split * chunk, n = max(0, min(cap, s0 + chunk) - s0), last = max(n - 1, 0);
+  const int tiles = (n + TILE - 1) / TILE;
+  uint16_t* kh = kbase + (size_t)b * kv_batch_stride + (size_t)kvh * kv_head_stride;
+  uint16_t* vh = vbase + (size_t)b * kv_batch_stride + (size_t)kvh * kv_head_stride;
+  uint16_t* vs = s_v[wave];
+
+  // small loads first (see the one-head form); chunk c of a row: dims 32c + 8 quad .. + 7
+  uint4 qc[DC], kc[DC], cc[DC], sc[DC], vc{};
+  if (FUSED) {
+    const uint16_t* rrow = row + (size_t)b * row_width;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+      qc[c] = *reinterpret_cast<const uint4*>(rrow + query_start + (size_t)(h0 + head) * D + 32 * c + 8 * quad);
+      kc[c] = *reinterpret_cast<const uint4*>(rrow + key_start + (size_t)kvh * D + 32 * c + 8 * quad);
+      if (ROWS) {
+        cc[c] = *reinterpret_cast<const uint4*>(rope_rows + 32 * c + 8 * quad);
+        sc[c] = *reinterpret_cast<const uint4*>(rope_rows + D + 32 * c + 8 * quad);
+      }
+    }
+    vc = reinterpret_cast<const uint4*>(rrow + value_start + (size_t)kvh * D)[lane % LPK];
+  } else {
+#pragma unroll
+    for (int c = 0; c < DC; ++c)
+      qc[c] = *reinterpret_cast<const uint4*>(q + ((size_t)b * query_heads + h0 + head) * D + 32 * c + 8 * quad);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // keys of a tile, within the split: A row `col` of key group kt, and the row a lane stages of V
+  auto key_a = [&](int tile, int kt) { return tile * TILE + wave * WK + 16 * kt + col; };
+  auto key_v = [&](int tile, int i) { return tile * TILE + wave * WK + (i * 64 + lane) / LPK; };
+  uint4 kq[2][DC], vq[VL];
+  auto load_keys = [&](int tile) {
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const uint16_t* p = kh + (size_t)(s0 + min(key_a(tile, kt), last)) * D + 8 * quad;
+#pragma unroll
+      for (int c = 0; c < DC; ++c) kq[kt][c] = *reinterpret_cast<const uint4*>(p + 32 * c);
+    }
+  };
+  auto load_values = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < VL; ++i)
+      vq[i] = reinterpret_cast<const uint4*>(vh + (size_t)(s0 + min(key_v(tile, i), last)) * D)[lane % LPK];
+  };
+  load_keys(0);
+  load_values(0);
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (step != nullptr) {
+    position = step[0];
+    valid = step[1];
+    ring_offset = step[2];
+    slot = step[3];
+  }
+  if (FUSED) {
+    if (!ROWS) {
+#pragma unroll
+      for (int c = 0; c < DC; ++c) {
+        cc[c] = *reinterpret_cast<const uint4*>(cos_table + (size_t)position * D + 32 * c + 8 * quad);
+        sc[c] = *reinterpret_cast<const uint4*>(sin_table + (size_t)position * D + 32 * c + 8 * quad);
+      }
+    }
+    // RoPE, f32 with one rounding to bf16: the partner of chunk c is chunk c +- DC / 2 of the same lane
+    auto rotate = [&](uint4 (&x)[DC]) {
+      uint4 y[DC];
+#pragma unroll
+      for (int c = 0; c < DC; ++c) {
+        const uint4 o = x[(c + DC / 2) % DC];
+        const uint32_t xa[4] = {x[c].x, x[c].y, x[c].z, x[c].w}, pa[4] = {o.x, o.y, o.z, o.w};
+        const uint32_t ca[4] = {cc[c].x, cc[c].y, cc[c].z, cc[c].w}, sa[4] = {sc[c].x, sc[c].y, sc[c].z, sc[c].w};
+        const float sign = c < DC / 2 ? -1.f : 1.f;
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          w[i] = pack_bf16x2(bf16_lo(xa[i]) * bf16_lo(ca[i]) + sign * bf16_lo(pa[i]) * bf16_lo(sa[i]),
+                             bf16_hi(xa[i]) * bf16_hi(ca[i]) + sign * bf16_hi(pa[i]) * bf16_hi(sa[i]));
+        y[c] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+#pragma unroll
+      for (int c = 0; c < DC; ++c) x[c] = y[c];
+    };
+    rotate(qc);
+    rotate(kc);
+    // The block that holds `slot` stores the new (k_rot, v) row - the first heads of a kv group, wave 0;
+    // every block uses its own copy of the row in its products.
+    if (h0 % group == 0 && wave == 0 && slot >= s0 && slot < s0 + n) {
+      if (col == 0) {
+#pragma unroll
+        for (int c = 0; c < DC; ++c) *reinterpret_cast<uint4*>(kh + (size_t)slot * D + 32 * c + 8 * quad) = kc[c];
+      }
+      if (lane < LPK) reinterpret_cast<uint4*>(vh + (size_t)slot * D)[lane] = vc;
+    }
+  }
+
+  auto kept = [&](int sl) -> bool {
+    if (mask != nullptr) return mask[(size_t)b * mask_batch_stride + sl] != 0;
+    int logical = sl - ring_offset;
+    logical += logical < 0 ? cap : 0;
+    return logical >= cap - valid;
+  };
+
+  f32x4_t o[DT] = {};
+  float run_m = -INFINITY, run_l = 0.f;
+  for (int tile = 0; tile < tiles; ++tile) {
+    const int next = min(tile + 1, tiles - 1);  // the last trip reads its own tile again
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
+      const bool mine = FUSED && s0 + min(key_v(tile, i), last) == slot;
+      const uint4 v = make_uint4(mine ? vc.x : vq[i].x, mine ? vc.y : vq[i].y, mine ? vc.z : vq[i].z,
+                                 mine ? vc.w : vq[i].w);
+      *reinterpret_cast<uint4*>(vs + (i * 64 + lane) / LPK * STR + (lane % LPK) * 8) = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    f32x4_t s[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const bool mine = FUSED && s0 + min(key_a(tile, kt), last) == slot;
+      s[kt] = f32x4_t{};
+#pragma unroll
+      for (int c = 0; c < DC; ++c) {
+        const uint4 k = make_uint4(mine ? kc[c].x : kq[kt][c].x, mine ? kc[c].y : kq[kt][c].y,
+                                   mine ? kc[c].z : kq[kt][c].z, mine ? kc[c].w : kq[kt][c].w);
+        s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, k),
+                                                        __builtin_bit_cast(bf16x8_t, qc[c]), s[kt], 0, 0, 0);
+      }
+    }
+    load_keys(next);
+    load_values(next);
+    float p[8], top = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int rel = tile * TILE + wave * WK + 16 * (j >> 2) + 4 * quad + (j & 3);
+      p[j] = rel < n && kept(s0 + min(rel, last)) ? s[j >> 2][j & 3] * scale : -INFINITY;
+      top = fmaxf(top, p[j]);
+    }
+    const float m = fmaxf(run_m, xor32_max(xor16_max(top)));
+    const float f = run_m == -INFINITY ? 0.f : expf(run_m - m);
+    run_m = m;
+    run_l *= f;
+    if (__any(f != 1.f)) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t) o[t] *= f;
+    }
+    uint32_t hi[4], mid[4], lo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p0 = p[2 * i] == -INFINITY ? 0.f : expf(p[2 * i] - m);
+      const float p1 = p[2 * i + 1] == -INFINITY ? 0.f : expf(p[2 * i + 1] - m);
+      run_l += p0 + p1;
+      hi[i] = cvt_pk_bf16(p0, p1);
+      const float r0 = p0 - bf16_lo(hi[i]), r1 = p1 - bf16_hi(hi[i]);
+      mid[i] = cvt_pk_bf16(r0, r1);
+      lo[i] = cvt_pk_bf16(r0 - bf16_lo(mid[i]), r1 - bf16_hi(mid[i]));
+    }
+    const uint16_t* v0 = vs + (4 * quad + (col >> 2)) * STR + 4 * (col & 3);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      // keys 4 quad + 0..3 of both key groups at dim 16t + col
+      const auto a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((group_lds_s16x4*)(v0 + 16 * t));
+      const auto a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((group_lds_s16x4*)(v0 + 16 * STR + 16 * t));
+      const bf16x8_t va = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, __builtin_bit_cast(bf16x8_t, hi), o[t], 0, 0, 0);
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, __builtin_bit_cast(bf16x8_t, mid), o[t], 0, 0, 0);
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, __builtin_bit_cast(bf16x8_t, lo), o[t], 0, 0, 0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+
+  const float l = xor32_sum(xor16_sum(run_l));
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+    *reinterpret_cast<float4*>(&s_o[wave][col][16 * t + 4 * quad]) = make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
+  if (quad == 0) {
+    s_m[wave][col] = run_m;
+    s_l[wave][col] = l;
+  }
+  __syncthreads();
+
+  const int d = threadIdx.x % D;
+  for (int g = threadIdx.x / D; g < gb; g += 64 * WAVES / D) {
+    float mw[WAVES], big = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      mw[w] = s_m[w][g];
+      big = fmaxf(big, mw[w]);
+    }
+    float total = 0.f, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = (mw[w] == -INFINITY) ? 0.f : expf(mw[w] - big);
+      total = fmaf(f, s_o[w][g][d], total);
+      sum = fmaf(f, s_l[w][g], sum);
+    }
+    const size_t at = (size_t)b * query_heads + h0 + g;
+    if (splits == 1) {
+      out[at * D + d] = (uint16_t)f32_to_bf16(sum > 0.f ? total / sum : 0.f);
+    } else {
+      float* rec = partials + (at * splits + split) * (D + 2);
+      rec[2 + d] = total;
+      if (d == 0) {
+        rec[0] = big;
+        rec[1] = sum;
+      }
+    }
+  }
+}
+
 // Combine the split records of aoto_decode_attention_*: one block per (b, head),
 //   out = sum_s e^(m_s - M) acc_s / sum_s e^(m_s - M) l_s,  M = max_s m_s; 0 when no key is kept.
 // Thread d loads column d of the first kMergeRegSplits records into registers
@@ -409,7 +659,15 @@ extern "C" __global__ __launch_bounds__(128) void aoto_decode_attention_merge(co
     const float t = fmaf(s_w[s], a[s], num);
     num = s < splits ? t : num;
   }
-  for (int s = kMergeRegSplits; s < splits; ++s) num = fmaf(s_w[s], rec[(size_t)s * stride + 2 + dc], num);
+  // the splits past the registers, 16 loads in flight (one by one, each was a round trip)
+  for (int s0 = kMergeRegSplits; s0 < splits; s0 += 16) {
+    float t[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t[i] = rec[(size_t)min(s0 + i, splits - 1) * stride + 2 + dc];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (s0 + i < splits) num = fmaf(s_w[s0 + i], t[i], num);
+  }
   if (column) out[(size_t)bh * D + d] = (uint16_t)f32_to_bf16(den > 0.f ? num / den : 0.f);
 }
 
@@ -661,3 +919,34 @@ extern "C" __global__ void aoto_step_advance(int* __restrict__ state, int cap) {
   AOTO_DECODE_ATTENTION_INSTANCE(D, WAVES, J2)                 \
   AOTO_DECODE_ATTENTION_INSTANCE(D, WAVES, J3)                 \
   AOTO_DECODE_ATTENTION_INSTANCE(D, WAVES, J4)
+
+// Grouped decode attention (the query heads of a kv head share a block).
+#define AOTO_DECODE_ATTENTION_GROUP(D)                                                                        \
+  extern "C" __global__ __launch_bounds__(256) void aoto_decode_attention_d##D##_g(                           \
+      const uint16_t* q, uint16_t* kbase, uint16_t* vbase, long long kv_batch_stride, long long kv_head_stride, \
+      const uint8_t* mask, int mask_batch_stride, int valid, int ring_offset, int cap, int query_heads,       \
+      int kv_heads, int gb, float scale, int chunk, float* partials, const int* step, uint16_t* out) {        \
+    aoto::decode_attention_group_body<D, false, false>(                                                       \
+        q, nullptr, 0, 0, 0, 0, nullptr, nullptr, kbase, vbase, kv_batch_stride, kv_head_stride, mask,        \
+        mask_batch_stride, valid, ring_offset, 0, -1, cap, query_heads, kv_heads, gb, scale, chunk, partials, \
+        step, nullptr, out);                                                                                  \
+  }                                                                                                           \
+  extern "C" __global__ __launch_bounds__(256) void aoto_decode_rope_attention_d##D##_g(                      \
+      const uint16_t* row, const uint16_t* rope_rows, uint16_t* kbase, uint16_t* vbase, int kv_head_stride,   \
+      int kv_batch_stride, int heads, int starts_qk, int start_v_width, int cap, int chunk, int gb, int valid, \
+      int ring_offset, int position, int slot, float scale, float* partials, const int* step,                 \
+      const uint16_t* cos_table, const uint16_t* sin_table, uint16_t* out) {                                  \
+    const int query_heads = heads & 0xFFFF, kv_heads = (int)((unsigned)heads >> 16);                          \
+    const int query_start = starts_qk & 0xFFFF, key_start = (int)((unsigned)starts_qk >> 16);                 \
+    const int value_start = start_v_width & 0xFFFF, row_width = (int)((unsigned)start_v_width >> 16);         \
+    if (rope_rows != nullptr)                                                                                 \
+      aoto::decode_attention_group_body<D, true, true>(                                                       \
+          nullptr, row, row_width, query_start, key_start, value_start, cos_table, sin_table, kbase, vbase,   \
+          kv_batch_stride, kv_head_stride, nullptr, 0, valid, ring_offset, position, slot, cap, query_heads,  \
+          kv_heads, gb, scale, chunk, partials, step, rope_rows, out);                                        \
+    else                                                                                                      \
+      aoto::decode_attention_group_body<D, true, false>(                                                      \
+          nullptr, row, row_width, query_start, key_start, value_start, cos_table, sin_table, kbase, vbase,   \
+          kv_batch_stride, kv_head_stride, nullptr, 0, valid, ring_offset, position, slot, cap, query_heads,  \
+          kv_heads, gb, scale, chunk, partials, step, nullptr, out);                                          \
+  }

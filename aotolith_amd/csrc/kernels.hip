@@ -149,6 +149,8 @@ AOTO_GEMV_W8_SHAPE(1, 4)
 // (8-wave blocks measured no faster: 4.46 vs 4.38 us for the Qwen step).
 AOTO_DECODE_ATTENTION_SHAPES(64, 4, 2, 4, 6, 8)
 AOTO_DECODE_ATTENTION_SHAPES(128, 4, 2, 4, 6, 8)
+AOTO_DECODE_ATTENTION_GROUP(64)
+AOTO_DECODE_ATTENTION_GROUP(128)
 
 // Prefill attention: head dim.
 AOTO_FLASH_INSTANCE(64)

@@ -630,3 +630,66 @@ def test_argmax_at_chunk_edges_with_ties_signs_and_nans(n):
     assert torch.equal(_ops().argmax(logits).cpu(), want)
     shifted = torch.empty(8 * n + 1, dtype=torch.bfloat16, device="cuda")[1:].view(8, n).copy_(logits)
     assert torch.equal(_ops().argmax(shifted).cpu(), want)
+
+
+@pytest.mark.parametrize("hq,hkv,dim,cap,valid,batch", [
+    (14, 2, 64, 2048, 2048, 1), (7, 1, 64, 2049, 1500, 1), (4, 2, 64, 5003, 5003, 2), (40, 2, 64, 2300, 9, 1),
+    (32, 8, 128, 4096, 4000, 1), (8, 4, 128, 4131, 4131, 2), (16, 1, 128, 9000, 7777, 1), (34, 2, 64, 2500, 2500, 1)])
+@pytest.mark.parametrize("form", ["ring", "rows", "step", "plain", "mask"])
+def test_long_windows_share_a_pass_over_the_kv_head(hq, hkv, dim, cap, valid, batch, form):
+    """Windows from the length where query heads share a block (groups of 2 to 17 heads: 17 stays one head a block),
+    at tile remainders, short valid runs and a ring that wraps: against 64-bit attention and the one-head form
+    (which an explicit split count keeps), the new key and value written once."""
+
+    ops = _ops()
+    gen = torch.Generator().manual_seed(cap + hq)
+    pair = torch.randn(2, batch, hkv, cap, dim, generator=gen).bfloat16().cuda()
+    row = torch.randn(batch, (hq + 2 * hkv) * dim, generator=gen).bfloat16().cuda()
+    _, _, cos, sin = _tables(cap, dim, 1e6)
+    offset, position = cap // 3 + 1, valid - 1
+    slot = (offset - 1) % cap
+    workspace = ops.decode_attention_workspace(batch, hq, hkv, cap, dim, device="cuda")
+    logical = (torch.arange(cap, device="cuda") - offset) % cap
+    keep = (logical >= cap - valid).expand(batch, cap).clone()
+    if form in ("plain", "mask"):
+        q = row[:, : hq * dim].view(batch, hq, dim).contiguous()
+        if form == "mask":
+            keep &= torch.rand(batch, cap, generator=gen).cuda() > 0.5
+            if batch > 1:
+                keep[1] = False  # a batch row with no key
+        kwargs = dict(mask=keep) if form == "mask" else dict(valid=valid, ring_offset=offset)
+        got = ops.decode_attention(q, pair[0], pair[1], workspace=workspace, **kwargs)
+        other = ops.decode_attention(q, pair[0], pair[1], splits=40, **kwargs, workspace=ops.decode_attention_workspace(
+            batch, hq, hkv, cap, dim, 40, device="cuda"))
+        query, keys, values = q.double(), pair[0].double(), pair[1].double()
+    else:
+        kwargs = dict(query_heads=hq, query_start=0, key_start=hq * dim, value_start=(hq + hkv) * dim, position=position,
+                      slot=slot, valid=valid, ring_offset=offset)
+        if form == "step":
+            kwargs.update(position=0, slot=0, valid=0, ring_offset=0, step_state=torch.tensor(
+                [position, valid, offset, slot], dtype=torch.int32, device="cuda"))
+        if form == "rows":
+            kwargs.update(position=0, rope_rows=torch.stack([cos[position], sin[position]]).contiguous())
+        first, second = pair.clone(), pair.clone()
+        got = ops.decode_rope_attention(row, cos, sin, first, workspace=workspace, **kwargs)
+        other = ops.decode_rope_attention(row, cos, sin, second, splits=40, **kwargs,
+                                          workspace=ops.decode_attention_workspace(batch, hq, hkv, cap, dim, 40, device="cuda"))
+        assert torch.equal(first, second)
+        untouched = torch.arange(cap, device="cuda") != slot
+        assert torch.equal(first[..., untouched, :], pair[..., untouched, :])
+
+        def rotated(x):
+            x, c, s = x.float(), cos[position].float(), sin[position].float()
+            return (x * c + torch.cat((-x[..., dim // 2:], x[..., : dim // 2]), -1) * s).bfloat16().double()
+
+        heads = row.view(batch, hq + 2 * hkv, dim)
+        query, keys, values = rotated(heads[:, :hq]), first[0].double(), first[1].double()
+        assert torch.equal(values[:, :, slot], heads[:, hq + hkv:].double())
+    g = hq // hkv
+    scores = (query.view(batch, hkv, g, dim) @ keys.transpose(-1, -2)) * dim ** -0.5
+    scores = scores.masked_fill(~keep[:, None, None], float("-inf"))
+    want = (torch.nan_to_num(torch.softmax(scores, -1)) @ values).view(batch, hq, dim)
+    # f32 sums of the kept keys, then one bf16 rounding (2^-8); the forms differ by an ulp at most
+    room = 1e-5 + 2.0 ** -8 * want.abs() + 2e-4 * want.abs().amax()
+    assert bool(((got.double() - want).abs() <= room).all())
+    assert bool(((got.double() - other.double()).abs() <= 2.0 ** -7 * want.abs() + 2e-4 * want.abs().amax()).all())
