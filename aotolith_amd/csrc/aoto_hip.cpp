@@ -204,6 +204,7 @@ struct StreamShape {
   int blocks_per_cu = 2;  // persistent 4-wave blocks per CU
   bool block_x = false;   // x staged once per 4-wave block (aoto_w4_gemv_x* instances)
   int rows = 0;           // > 0: the multi-row direct form, rows per lane (aoto_w4_gemv_r* instances)
+  bool newer = false;     // an instance that an earlier build's code object does not have
 };
 
 // Rows per lane of the multi-row direct GEMV; AOTO_GEMV_ROWS overrides the
@@ -217,6 +218,26 @@ int gemv_rows(int lpr, int shape_default) {
   if (value == 0) return 0;
   const bool exists = lpr == 32 && (value == 2 || value == 4);
   return exists ? value : shape_default;
+}
+
+// Reductions without a tuned layout of their own: x staged once per block, the smallest lanes x chunks that
+// hold a row. One block per CU up to 16384 outputs, two beyond (5120 -> 5120 at 1 / 2 / 3 blocks 5.7 / 5.8 / 7.3 us,
+// 2048 -> 151936 43.6 / 31.0 / 31.2). Against the l* kernel, which has no next row in flight and takes what is left
+// (odd group counts, other groups, reductions past 16384), us over rotating weights: 512 -> 512 3.9 -> 2.6, 2048 ->
+// 2048 4.2 -> 2.9, 5120 -> 13824 16.0 -> 9.9 (paired 24.4 -> 16.9), 8192 -> 8192 17.1 -> 9.8, 13824 -> 5120 26.0 ->
+// 11.1, 2048 -> 151936 44.1 -> 31.3.
+bool block_staged_shape(int K, int N, bool paired, StreamShape* s) {
+  static const int layouts[][2] = {{32, 1}, {32, 2}, {32, 3}, {32, 4}, {32, 5}, {64, 3},
+                                   {64, 4}, {64, 5}, {64, 6}, {64, 7}, {64, 8}};
+  const int chunks = K / 32, count = paired ? 7 : 11;
+  if (K % 32 != 0) return false;
+  for (int i = 0; i < count; ++i) {
+    if (layouts[i][0] * layouts[i][1] < chunks) continue;
+    *s = {layouts[i][0], layouts[i][1], false, N > 16384 ? 2 : 1, true};
+    s->newer = true;
+    return true;
+  }
+  return false;
 }
 
 bool stream_shape(int K, int N, bool paired, StreamShape* s) {
@@ -260,7 +281,7 @@ bool stream_shape(int K, int N, bool paired, StreamShape* s) {
       // every wave load all 9.7 KB of x, ~40 KB per CU beside ~9 KB of weights
       // (Qwen down projection 3.58 -> 3.29 us, decode 2345-2359 -> 2379-2382
       // tok/s in alternating runs on one box).
-      if (paired || !short_out) return false;
+      if (paired || !short_out) return block_staged_shape(K, N, paired, s);
       *s = {64, 3, false, 1, true};
       return true;
     case 14336:
@@ -270,8 +291,7 @@ bool stream_shape(int K, int N, bool paired, StreamShape* s) {
       *s = {64, 7, false, 1, true};
       return true;
     default:
-      // Other reductions use the block-staged kernel.
-      return false;
+      return block_staged_shape(K, N, paired, s);
   }
 }
 
@@ -552,8 +572,9 @@ int aoto_hip_w4_gemv(const void* x, const int32_t* words, const void* scales, co
     snprintf(sname, sizeof(sname), "aoto_w4_gemv_%c%dx%d_n%d_p%d_b%d", ss.block_x ? 'x' : 's', ss.lpr, ss.cpl,
              norm, paired ? 1 : 0, has_bias);
     unsigned long long* no_keys = nullptr;
-    return launch(sname, dim3((unsigned)l.grid), dim3(64 * l.wpb), l.shared, stream, words, scales, x, norm_weight,
-                  K, N, l.shift, l.wpb, bias, up_words, up_scales, eps, alpha, beta, y, no_keys);
+    if (!ss.newer || has_kernel(sname))
+      return launch(sname, dim3((unsigned)l.grid), dim3(64 * l.wpb), l.shared, stream, words, scales, x, norm_weight,
+                    K, N, l.shift, l.wpb, bias, up_words, up_scales, eps, alpha, beta, y, no_keys);
   }
   int lpr = lanes_per_row;
   if (lpr == 0) {
@@ -1707,7 +1728,7 @@ int aoto_hip_w4_gemv_finish(const uint64_t* keys, int key_count, const void* emb
   StreamShape ss{};
   const bool pow2_group = group > 0 && (group & (group - 1)) == 0;
   if (!pow2_group || group < 32 || K % group != 0 || (K / group) % 2 != 0 || !stream_shape(K, N, false, &ss) ||
-      !ss.block_x || ss.lpr != 32 || (ss.cpl != 1 && ss.cpl != 4) || ss.rows != 0)
+      !ss.block_x || ss.newer || ss.lpr != 32 || (ss.cpl != 1 && ss.cpl != 4) || ss.rows != 0)
     return fail(AOTO_ERR_UNSUPPORTED, "w4_gemv_finish: the finish prologue is built for the block-staged "
                 "q/k/v GEMV shapes (K = 896 or 4096, N <= 16384, power-of-two groups; K=%d N=%d group=%d)",
                 K, N, group);

@@ -50,6 +50,20 @@ AOTO_GEMV_STREAM_BLOCKX_SINGLE(32, 4, 2)
 AOTO_GEMV_STREAM_BLOCKX_PAIRED(32, 4, 2)
 AOTO_GEMV_STREAM_BLOCKX_SINGLE(64, 3, 3)
 AOTO_GEMV_STREAM_BLOCKX_SINGLE(64, 7, 7)
+// Other reductions up to 16384 (paired: 8192), by the smallest layout that holds a row.
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(32, 2, 1)
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(32, 3, 2)
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(32, 5, 3)
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(64, 4, 4)
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(64, 5, 5)
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(64, 6, 6)
+AOTO_GEMV_STREAM_BLOCKX_SINGLE(64, 8, 8)
+AOTO_GEMV_STREAM_BLOCKX_PAIRED(32, 1, 1)
+AOTO_GEMV_STREAM_BLOCKX_PAIRED(32, 2, 1)
+AOTO_GEMV_STREAM_BLOCKX_PAIRED(32, 3, 2)
+AOTO_GEMV_STREAM_BLOCKX_PAIRED(32, 5, 3)
+AOTO_GEMV_STREAM_BLOCKX_PAIRED(64, 3, 3)
+AOTO_GEMV_STREAM_BLOCKX_PAIRED(64, 4, 4)
 // The greedy loop's first q/k/v GEMV of a step with the previous step's argmax
 // finish in its prologue (K = 896: 32x1, K = 4096: 32x4; with and without bias).
 AOTO_GEMV_STREAM_FINISH_KERNEL(32, 1, 1, 1, 1)
