@@ -1344,6 +1344,33 @@ int aoto_hip_w8_gemv(const void* x, const int32_t* words, const void* scales, co
   if (!aligned16(x) || !aligned16(words) || (up_words && !aligned16(up_words)) ||
       (norm_weight && !aligned16(norm_weight)))
     return fail(AOTO_ERR_ARGUMENT, "w8_gemv: x, words and norm weight must be 16-byte aligned");
+  // The streaming form: the smallest lanes x chunks layout that holds a row, for power-of-two groups with an
+  // even count per row (scales and bias are read as aligned 32-bit pairs). Two blocks per CU for single
+  // projections up to K = 8192 (3072 -> 8192 at 1 / 2 / 3 blocks 8.3 / 7.1 / 6.8 us, 5120 -> 5120 7.9 / 7.5 / 8.6),
+  // one for longer ones, whose staging each block repeats (11008 -> 4096 12.6 / 15.2 / 17.8), and for the pair;
+  // four for wide outputs of short rows, a wave's loads being few (896 -> 151936 at 1 / 2 / 3 / 4 blocks 46.0 /
+  // 34.1 / 27.9 / 27.3, w8.h's kernel 30.8; 1536 -> 65536 26.2 / 20.6 / 19.7 / 19.5, 26.6).
+  if ((group & (group - 1)) == 0 && (K / group) % 2 == 0 && aligned4(scales) && (!up_scales || aligned4(up_scales)) &&
+      (!bias || (N % 2 == 0 && aligned4(bias)))) {
+    static const int layouts[][2] = {{32, 1}, {32, 2}, {32, 3}, {32, 4}, {64, 3}, {64, 4},
+                                     {64, 5}, {64, 6}, {64, 8}, {64, 11}, {64, 14}, {64, 16}};
+    for (int i = 0; i < (paired ? 9 : 12); ++i) {
+      const int lpr = layouts[i][0], cpl = layouts[i][1];
+      if (lpr * cpl < K / 16) continue;
+      char sname[64];
+      snprintf(sname, sizeof(sname), "aoto_w8_gemv_x%dx%d_n%d_p%d_b%d", lpr, cpl, norm_weight ? 1 : 0, paired ? 1 : 0,
+               bias ? 1 : 0);
+      if (!has_kernel(sname)) break;
+      const int rows = 64 / lpr;
+      const long long tiles = ((long long)N + rows - 1) / rows;
+      const long long budget = (long long)cu_count() * gemv_blocks_per_cu(paired || K > 8192 ? 1 : N > 16384 && K <= 1536 ? 4 : 2) * 4;
+      const long long waves = tiles < budget ? tiles : budget;
+      int shift = 0;
+      while ((16 << shift) < group) ++shift;
+      return launch(sname, dim3((unsigned)((waves + 3) / 4)), dim3(256), (unsigned)(K * 2 + K / 4), stream, words, scales,
+                    x, norm_weight, K, N, shift, bias, up_words, up_scales, eps, alpha, beta, y);
+    }
+  }
   // A wave holds R rows x U chunks of 16 codes per lane in flight: U covers the
   // row's chunks in one pass where it can (up to 4), R fills the rest of 4.
   const int chunks = K / 16;

@@ -9,6 +9,7 @@
 #include "w4_gemm_wide.h"
 #include "w4_gemm_lds.h"
 #include "w8.h"
+#include "w8_gemv_stream.h"
 #include "generic.h"
 #include "generic_gemm.h"
 #include "decode.h"
@@ -157,6 +158,28 @@ AOTO_GEMM_ROPE_INSTANCE(8, 2, 8, 1)
 AOTO_GEMV_W8_SHAPE(4, 1)
 AOTO_GEMV_W8_SHAPE(2, 2)
 AOTO_GEMV_W8_SHAPE(1, 4)
+// Streaming int8 decode GEMV: {lanes per row} x {16-code chunks per lane} x {x vectors a thread stages}.
+AOTO_GEMV_W8_STREAM_SINGLE(32, 1, 1)
+AOTO_GEMV_W8_STREAM_SINGLE(32, 2, 1)
+AOTO_GEMV_W8_STREAM_SINGLE(32, 3, 1)
+AOTO_GEMV_W8_STREAM_SINGLE(32, 4, 1)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 3, 2)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 4, 2)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 5, 3)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 6, 3)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 8, 4)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 11, 6)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 14, 7)
+AOTO_GEMV_W8_STREAM_SINGLE(64, 16, 8)
+AOTO_GEMV_W8_STREAM_PAIRED(32, 1, 1)
+AOTO_GEMV_W8_STREAM_PAIRED(32, 2, 1)
+AOTO_GEMV_W8_STREAM_PAIRED(32, 3, 1)
+AOTO_GEMV_W8_STREAM_PAIRED(32, 4, 1)
+AOTO_GEMV_W8_STREAM_PAIRED(64, 3, 2)
+AOTO_GEMV_W8_STREAM_PAIRED(64, 4, 2)
+AOTO_GEMV_W8_STREAM_PAIRED(64, 5, 3)
+AOTO_GEMV_W8_STREAM_PAIRED(64, 6, 3)
+AOTO_GEMV_W8_STREAM_PAIRED(64, 8, 4)
 
 // Single-query attention (plain and RoPE-fused ring step): head dim.
 // Decode attention: 4-wave blocks, {2, 4, 6, 8} K and V wave loads per wave

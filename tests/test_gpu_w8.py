@@ -191,3 +191,44 @@ def test_w8_matmul_epilogues(epilogue, splits):
     expected = oracle.w4_matmul(x, packed, scales, 64, bits=8, **kwargs)
     atol = 2e-2 * max(1.0, float(np.abs(expected).max()) / 4)
     assert_bf16_parity(from_gpu_bf16(y), expected, max_ulp=2.0 if epilogue == "gate" else 1.0, atol=atol)
+
+
+@pytest.mark.parametrize("n,k,group", [
+    (1, 64, 32), (3, 128, 64), (130, 512, 64), (77, 1024, 128), (257, 1152, 64), (66, 1088, 32), (515, 2048, 64),
+    (129, 2560, 128), (131, 3200, 32), (70, 5120, 64), (65, 6016, 64), (33, 6272, 64), (514, 8192, 128), (37, 10240, 64),
+    (36, 11264, 64), (36, 12288, 64), (35, 16384, 16), (40, 16384, 64), (34, 16512, 64), (16450, 256, 64), (9000, 4864, 64)])
+def test_w8_gemv_over_every_layout_that_holds_a_row(n, k, group):
+    """Reductions between and at the edges of the lane layouts (and past them: the plain kernel), few and many rows,
+    every epilogue, against the oracle's exact sums; odd row counts only without a bias, as the paired loads need."""
+
+    rng = np.random.default_rng(n + k)
+    ops = _ops()
+    packed, scales = _packed(rng, n, k, group)
+    up_packed, up_scales = _packed(rng, n, k, group)
+    x, norm = bf16_normal(rng, (k,)), bf16_normal(rng, (k,), 0.1) + np.float32(1.0)
+    norm, bias = round_bf16(norm), bf16_normal(rng, (n,))
+    gx, gn, gb = to_gpu_bf16(x), to_gpu_bf16(norm), to_gpu_bf16(bias)
+    gp, gs = _gpu(packed, scales)
+    up = _gpu(up_packed, up_scales)
+    for kwargs, want in (
+            ({}, {}),
+            (dict(norm_weight=gn, eps=1e-6), dict(norm_weight=norm, eps=1e-6)),
+            (dict(bias=gb), dict(bias=bias)),
+            (dict(norm_weight=gn, eps=1e-6, bias=gb), dict(norm_weight=norm, eps=1e-6, bias=bias)),
+            (dict(norm_weight=gn, eps=1e-6, up=up),
+             dict(norm_weight=norm, eps=1e-6, up_packed=up_packed, up_scales_bits=up_scales)),
+            (dict(up=up), dict(up_packed=up_packed, up_scales_bits=up_scales))):
+        got = from_gpu_bf16(ops.w8_gemv(gx, gp, gs, group, **kwargs))
+        expected = oracle.w4_gemv(x, packed, scales, group, bits=8, **want)
+        # Off the exact sum: an f32 sum's roundings (K / 8 of partial sums below six deviations, 0.02 sqrt(K)); with
+        # the norm, up to four elements of x whose bf16 rounding the statistic's last bit turns (2^-8 of |x| |w|,
+        # below 5 and 0.1); both times the other factor of the pair, whose gate is rounded once more; then one
+        # bf16 rounding (2^-7 where it falls on the other side).
+        top = 6 * 0.02 * k ** 0.5
+        room = k / 8 * 2.0 ** -24 * top + ("norm_weight" in kwargs) * 4 * 2.0 ** -8 * 5 * 0.1
+        size = np.abs(expected).astype(np.float64)
+        paired = "up" in kwargs
+        bound = room * (2 * max(1.0, top) if paired else 1.0) + (3 if paired else 1) * 2.0 ** -7 * size
+        assert bool((np.abs(got.astype(np.float64) - expected) <= bound).all())
+        if n > 64:  # and nothing systematic
+            assert_bf16_parity(got, expected, max_ulp=None, atol=1.0, min_cos=0.9999)
