@@ -222,7 +222,9 @@ int gemv_rows(int lpr, int shape_default) {
 
 // Reductions without a tuned layout of their own: x staged once per block, the smallest lanes x chunks that
 // hold a row. One block per CU up to 16384 outputs, two beyond (5120 -> 5120 at 1 / 2 / 3 blocks 5.7 / 5.8 / 7.3 us,
-// 2048 -> 151936 43.6 / 31.0 / 31.2). Against the l* kernel, which has no next row in flight and takes what is left
+// 2048 -> 151936 43.6 / 31.0 / 31.2), and more for short rows, a wave's loads being few (1024 -> 16384 5.0 / 4.4 /
+// 4.3, 1024 -> 151936 at 1 / 2 / 3 / 4 blocks 33.1 / 24.8 / 21.1 / 17.9); rows of up to 640 in wide outputs leave too
+// many slots empty (512 -> 151936 17.0 against 16.1 on the l* kernel). Against the l* kernel, which has no next row in flight and takes what is left
 // (odd group counts, other groups, reductions past 16384), us over rotating weights: 512 -> 512 3.9 -> 2.6, 2048 ->
 // 2048 4.2 -> 2.9, 5120 -> 13824 16.0 -> 9.9 (paired 24.4 -> 16.9), 8192 -> 8192 17.1 -> 9.8, 13824 -> 5120 26.0 ->
 // 11.1, 2048 -> 151936 44.1 -> 31.3.
@@ -230,10 +232,11 @@ bool block_staged_shape(int K, int N, bool paired, StreamShape* s) {
   static const int layouts[][2] = {{32, 1}, {32, 2}, {32, 3}, {32, 4}, {32, 5}, {64, 3},
                                    {64, 4}, {64, 5}, {64, 6}, {64, 7}, {64, 8}};
   const int chunks = K / 32, count = paired ? 7 : 11;
-  if (K % 32 != 0) return false;
+  if (K % 32 != 0 || (N > 16384 && K <= 640)) return false;
+  const int per_cu = N > 16384 ? (K <= 1536 ? 4 : 2) : K <= 1024 ? 2 : 1;
   for (int i = 0; i < count; ++i) {
     if (layouts[i][0] * layouts[i][1] < chunks) continue;
-    *s = {layouts[i][0], layouts[i][1], false, N > 16384 ? 2 : 1, true};
+    *s = {layouts[i][0], layouts[i][1], false, per_cu, true};
     s->newer = true;
     return true;
   }
