@@ -633,11 +633,16 @@ bool wide_code(int tile) {
 // 813 / 814 = the single form's split-K partials on 128-row blocks of 4 waves, 128 x 32
 // (one wave along n, 32 x 32 per wave) / 128 x 64 (64 x 32 per wave) blocks, summed and
 // given their epilogue by the split reduce kernels (at any split count, 1 included).
+// 815 / 825 = the split form's 128 x 128 (4 waves of 64 x 64) / 256 x 128 (8 waves) blocks; 833 / 834 / 845 =
+// 813 / 814 / 825 over 8-bit codes.
+bool lds_byte_code(int tile) { return tile == 833 || tile == 834 || tile == 845; }
 bool lds_code(int tile) {
-  return tile == 811 || tile == 812 || tile == 813 || tile == 814 || tile == 821 || tile == 822 || tile == 823;
+  return tile == 815 || tile == 825 || lds_byte_code(tile) || tile == 811 || tile == 812 || tile == 813 || tile == 814 || tile == 821 || tile == 822 || tile == 823;
 }
 bool lds_paired_code(int tile) { return tile == 811 || tile == 812 || tile == 821; }
-bool lds_split_code(int tile) { return tile == 813 || tile == 814; }
+bool lds_split_code(int tile) {
+  return tile == 813 || tile == 814 || tile == 815 || tile == 825 || lds_byte_code(tile);
+}
 
 // The automatic plan's choice of the dequant-once kernel (its tile code, or 0):
 // 4-bit codes, a power-of-two group with an even count per row, no gate epilogue,
@@ -741,9 +746,11 @@ GemmPlan gemm_plan(int M, int N, int K, int tile, int splits, bool paired) {
   GemmPlan p{};
   if (lds_code(tile)) {
     p.lds = true;
-    p.lds_bm = tile / 10 == 82 ? 256 : 128;
-    p.lds_waves = tile / 10 == 82 ? 8 : 4;
-    p.lds_bn = tile == 811 || tile == 813 ? 32 : tile == 823 ? 192 : tile == 822 ? 128 : 64;
+    p.lds_bm = tile / 10 == 82 || tile == 845 ? 256 : 128;
+    p.lds_waves = p.lds_bm == 256 ? 8 : 4;
+    p.lds_bn = tile == 811 || tile == 813 || tile == 833 ? 32
+               : tile == 823                             ? 192
+               : tile == 822 || tile == 815 || tile == 825 || tile == 845 ? 128 : 64;
     p.splits = 1;
     p.kslice = K;
     if (lds_split_code(tile)) {
@@ -823,21 +830,24 @@ enum GemmTail { kTailNorm, kTailRope, kTailPaired };
 // weights, q/k/v below 512 rows) ran on 128 x 128 tiles that left most of the chip idle.
 //   us = launch + steps * max(latency, rate * blocks / 256) + tail
 // with steps the k-steps of a slice, and the tail the separate norm / RoPE / reduce launch and what it moves.
-// The constants are least squares over 370 measured shapes (7 to 14 (N, K) pairs from 896 to 14336, 10 to
-// 15 row counts from 17 to 2048, every tile and 1 to 8 slices, both widths; log error of the near-best
-// plans 0.08 to 0.10). The model's choice replaces the fixed plan's where it promises 10% less: over those
-// shapes the plans' time falls by a factor of 1.28 (4-bit) and 1.32 (8-bit), 1.12 / 1.12 for the paired
-// form, and ends 4 to 7% over the best instance and split of each shape.
+// Instances whose staging leaves one block to a CU pay whole rounds of 256. The constants are least squares
+// over 370 measured shapes (7 to 14 (N, K) pairs from 896 to 14336, 10 to 15 row counts from 17 to 2048, every
+// tile and 1 to 8 slices, both widths; log error of the near-best plans 0.08 to 0.10). The model's choice
+// replaces the fixed plan's where it promises 10% less: over those shapes the plans' time falls by a factor of
+// 1.29 (4-bit) and 1.42 (8-bit), 1.12 / 1.12 for the paired form, and ends 3 to 7% over the best instance and
+// split of each shape.
 struct GemmCost {
   int code;
   float launch, latency, rate;
 };
-const GemmCost kCost4[] = {{12, 5.72f, .476f, .368f}, {14, 6.06f, .644f, .479f}, {18, 6.23f, 1.144f, .929f},
-                           {24, 6.28f, 1.048f, .768f}, {28, 7.24f, 1.656f, 1.244f}, {241, 8.87f, .963f, 1.372f},
-                           {441, 10.63f, 1.622f, 2.19f}, {813, 5.88f, .259f, .278f}, {814, 6.17f, .347f, .375f}};
-const GemmCost kCost8[] = {{12, 6.01f, .413f, .425f}, {14, 6.15f, .637f, .547f}, {18, 6.47f, 1.155f, .956f},
-                           {24, 6.74f, 1.091f, .916f}, {28, 7.37f, 1.738f, 1.301f}, {241, 9.89f, 1.12f, 1.532f},
-                           {441, 9.54f, 1.959f, 2.498f}};
+const GemmCost kCost4[] = {{12, 5.92f, .449f, .361f}, {14, 6.24f, .615f, .496f}, {18, 6.41f, 1.113f, .99f},
+                           {24, 6.4f, 1.05f, .785f}, {28, 7.48f, 1.633f, 1.259f}, {241, 9.22f, .954f, 1.307f},
+                           {441, 10.84f, 1.616f, 2.17f}, {813, 6.05f, .253f, .278f}, {814, 6.26f, .353f, .375f},
+                           {815, 6.93f, .443f, .548f}, {825, 7.05f, .651f, .779f}};
+const GemmCost kCost8[] = {{12, 5.93f, .415f, .435f}, {14, 6.09f, .632f, .585f}, {18, 6.41f, 1.144f, 1.036f},
+                           {24, 6.74f, 1.079f, .96f}, {28, 7.54f, 1.717f, 1.342f}, {241, 9.94f, 1.111f, 1.494f},
+                           {441, 10.12f, 1.897f, 2.323f}, {833, 5.96f, .267f, .298f}, {834, 6.22f, .354f, .387f},
+                           {845, 6.82f, .811f, .79f}};
 const GemmCost kCostPaired4[] = {{12, 7.59f, .455f, .629f}, {14, 8.26f, .666f, .858f}, {18, 9.09f, 1.321f, 1.468f},
                                  {24, 9.98f, 1.586f, 1.805f}, {241, 14.78f, 1.466f, 2.43f},
                                  {811, 6.81f, .294f, .436f}, {812, 7.96f, .474f, .784f}};
@@ -868,17 +878,18 @@ int modelled_splits(int M, int N, bool paired) {
 float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits, GemmTail tail, int head_dim) {
   const GemmPlan p = gemm_plan(M, N, K, c.code, splits, tail == kTailPaired);
   const int step = p.lds ? 64 : 128;
-  const float blocks = (float)((N + p.bn() - 1) / p.bn()) * ((M + p.bm() - 1) / p.bm()) * p.splits;
+  float blocks = (float)((N + p.bn() - 1) / p.bn()) * ((M + p.bm() - 1) / p.bm()) * p.splits;
+  if (lds_split_code(c.code) && p.lds_bn == 128) blocks = 256.f * ceilf(blocks / 256.f);
   const float steps = (float)((p.kslice < K ? p.kslice : K) + step - 1) / step;
-  const float mn = (float)M * N / 1e6f, sum = 1.8f * p.splits * mn;  // us to sum the slices' partials
+  const float mn = (float)M * N / 1e6f, sum = 1.72f * p.splits * mn;  // us to sum the slices' partials
   const bool split = p.splits > 1 || lds_split_code(c.code);
   float t = c.launch + (float)(int)steps * fmaxf(c.latency, c.rate * blocks / 256.f);
   if (tail == kTailPaired)
     t += split ? 0.8f + 1.2f * sum : 0.f;
   else if (tail == kTailRope)
-    t += split ? 1.6f + sum : !p.lds && !p.wide_mt && p.bn() % head_dim == 0 && N % p.bn() == 0 ? 0.f : 1.3f + 2.f * mn;
+    t += split ? 1.6f + sum : !p.lds && !p.wide_mt && p.bn() % head_dim == 0 && N % p.bn() == 0 ? 0.f : 1.3f + 1.6f * mn;
   else
-    t += split ? 1.f + sum : 1.2f + 1.9f * mn;
+    t += split ? 1.f + sum : 1.3f + 1.7f * mn;
   return t;
 }
 
@@ -891,7 +902,7 @@ bool modelled_plan(int bits, int M, int N, int K, int group, GemmTail tail, bool
   const int count = (int)(paired ? (bits == 4 ? sizeof(kCostPaired4) : sizeof(kCostPaired8))
                                  : (bits == 4 ? sizeof(kCost4) : sizeof(kCost8))) / (int)sizeof(GemmCost);
   const bool pow2_even = (group & (group - 1)) == 0 && group >= 32 && (K / group) % 2 == 0;
-  const bool small_offsets = (long long)M * K * 2 < (1LL << 31) && (long long)N * K / 2 < (1LL << 31);
+  const bool small_offsets = (long long)M * K * 2 < (1LL << 31) && (long long)N * K / 8 * bits < (1LL << 31);
   const GemmPlan fixed = gemm_plan(M, N, K, *tile, *splits, paired);
   float best = 0.f, now = 0.f;
   int best_tile = 0, best_splits = 0;
@@ -944,7 +955,7 @@ bool automatic_model(int bits, int M, int N, int K, int group, GemmTail tail, bo
 }
 
 // Plans of a code object that an earlier build stored stay that build's.
-bool models_plans() { return has_kernel("aoto_w4_quantize_units"); }
+bool models_plans() { return has_kernel("aoto_w8_gemm_d8c2w2x2_split"); }
 
 }  // namespace
 
@@ -1082,16 +1093,17 @@ int packed_gemm(int bits, const void* x, const int32_t* words, const void* scale
   if (tile != 0 && tile != 12 && tile != 14 && tile != 18 && tile != 24 && tile != 28 && !wide_code(tile) &&
       !lds_code(tile))
     return fail(AOTO_ERR_ARGUMENT, "%s: tile code %d is not one of 12, 14, 18, 24, 28, 241, 242, 243, 281, 441, "
-                "811, 812, 813, 814, 821, 822, 823", what, tile);
+                "811, 812, 813, 814, 815, 821, 822, 823, 825, 833, 834, 845", what, tile);
   if (lds_code(tile)) {
-    if (bits != 4 || lds_paired_code(tile) != paired || gate != nullptr || (splits > 1 && !lds_split_code(tile)))
-      return fail(AOTO_ERR_ARGUMENT, "%s: tile %d is the unsplit 4-bit %s form without a gate epilogue", what, tile,
+    if (bits != (lds_byte_code(tile) ? 8 : 4) || lds_paired_code(tile) != paired || gate != nullptr || (splits > 1 && !lds_split_code(tile)))
+      return fail(AOTO_ERR_ARGUMENT, "%s: tile %d is the %s%d-bit %s form without a gate epilogue", what, tile,
+                  lds_split_code(tile) ? "" : "unsplit ", lds_byte_code(tile) ? 8 : 4,
                   lds_paired_code(tile) ? "paired" : "single");
     if ((group & (group - 1)) != 0 || K % 64 != 0 || (K / group) % 2 != 0)
       return fail(AOTO_ERR_UNSUPPORTED, "%s: tile %d needs K %% 64 == 0 and an even number of power-of-two groups "
                   "per row (K=%d group=%d)", what, tile, K, group);
     // the kernel's per-lane load offsets are 32-bit
-    if ((long long)M * K * 2 >= (1LL << 31) || (long long)N * K / 2 >= (1LL << 31))
+    if ((long long)M * K * 2 >= (1LL << 31) || (long long)N * K / 8 * bits >= (1LL << 31))
       return fail(AOTO_ERR_UNSUPPORTED, "%s: tile %d needs X and the packed words under 2 GiB (M=%d N=%d K=%d)", what,
                   tile, M, N, K);
   }
@@ -1131,7 +1143,10 @@ int packed_gemm(int bits, const void* x, const int32_t* words, const void* scale
   char name[64];
   if (lds_split) {
     // dequant-once split partials; the reduce launches below sum them with the epilogue
-    snprintf(name, sizeof(name), "aoto_w4_gemm_d4c%dw%dx1_split", p.lds_bn / 32, p.lds_bn / 32);
+    if (p.lds_bn == 128)
+      snprintf(name, sizeof(name), "aoto_w%d_gemm_d%dc2w2x2_split", bits, p.lds_waves);
+    else
+      snprintf(name, sizeof(name), "aoto_w%d_gemm_d4c%dw%dx1_split", bits, p.lds_bn / 32, p.lds_bn / 32);
     if (int st = launch(name, grid, dim3(p.threads()), 0, stream, x, words, scales, partials, M, N, K, group,
                         p.kslice))
       return st;

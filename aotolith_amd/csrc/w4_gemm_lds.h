@@ -79,10 +79,11 @@ AOTO_DEVICE int lds_unit(int r, int u) { return r * 128 + ((u ^ ((r >> 1) & 7)) 
 // for 6 at NT = 3; the 128-row paired form (4 waves, WGN = 1, MT = NT = 1) 3 for 2.
 // X takes three staging buffers where they fit 160 KB, else two (WR = 192 at 256
 // rows: each step's X is then loaded one step ahead).
+// BITS = 8: int8 codes, two packed words per 8-code unit (64 bytes a row and step, four lanes of a load).
 // PARTIAL (split-K, the single form): block z of the grid's third dimension takes k
 // in [z kslice, min(K, (z + 1) kslice)) and stores its f32 tile to partials[z][m][n]
 // (the layout the split reduce kernels of w4_gemm.h read); no epilogue.
-template <int NW, int WGN, int MT, int NT, bool PAIRED, bool BIAS, bool RESIDUAL, bool PARTIAL = false>
+template <int NW, int WGN, int MT, int NT, bool PAIRED, bool BIAS, bool RESIDUAL, bool PARTIAL = false, int BITS = 4>
 __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t* __restrict__ words,
                                  const uint16_t* __restrict__ scales, const uint32_t* __restrict__ up_words,
                                  const uint16_t* __restrict__ up_scales, const uint16_t* __restrict__ bias,
@@ -101,14 +102,17 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
   constexpr int XT = BM * 128;                       // bytes of a staged X tile
   constexpr int XDW = XT / 1024 / NW;                // 1-KB X loads per wave and step
   constexpr int WT = WR * 128;                       // bytes of a bf16 weight tile
-  constexpr int PT = WR * 32;                        // bytes of a step's packed words
+  constexpr int PB = 8 * BITS;                       // packed bytes of a row and step
+  constexpr int PT = WR * PB;                        // bytes of a step's packed words
   constexpr int PST = PT + WR * 4;                   // ... and their scale dwords
   constexpr int XS = 3 * XT + 2 * WT + 3 * PST <= 160 * 1024 ? 3 : 2;  // X staging buffers
   constexpr int PW = WR / NW;                        // packed rows each wave loads: 16, 24 or 32
   constexpr int UPT = WR * 8 / (64 * NW);            // words each lane expands per step: 2, 3 or 4
   static_assert(UPT >= 1 && WR % NW == 0, "every lane expands whole words");
   static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-  static_assert(2 * PW <= 64 && UPT <= 4, "one packed-word load per wave and step");
+  constexpr int LPR = PB / 16;                       // lanes of a packed row's load: 2 or 4
+  constexpr int PL = (PW * LPR + 63) / 64;           // packed-word loads per wave and step
+  static_assert(UPT <= 4 && (PL == 1 || PW * LPR == 64 * PL), "whole packed-word loads");
 
   __shared__ __attribute__((aligned(16))) uint8_t xs0[XT];
   __shared__ __attribute__((aligned(16))) uint8_t xs1[XT];
@@ -125,7 +129,6 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
   const int col = lane & 31, half = lane >> 5;
   const int wm = wave / WGN, wn = wave % WGN;
   const int m_block = blockIdx.y * BM, n_block = blockIdx.x * BNW;
-  const int kw = K >> 3;
   const int groups = K / group;
   const int gshift = __builtin_ctz(group);
   const int kbase = PARTIAL ? (int)blockIdx.z * kslice : 0;  // kslice % 64 == 0 (host)
@@ -152,13 +155,16 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
     xoff[i] = (uint32_t)(((size_t)min(m_block + r, M - 1) * K + 8 * c) * 2);
   }
   // Packed rows PW w .. PW w + PW - 1 of the block (the gate's rows, then the up's):
-  // lanes below 2 PW load 16 bytes each (two per row), lanes below PW one scale dword.
-  const int prow = PW * wave + (lane >> 1) % PW;
+  // lanes below LPR PW load 16 bytes each (LPR per row), lanes below PW one scale dword.
   const bool up_rows = PAIRED && PW * wave_u >= BNW;  // wave-uniform
-  const int pn = min(n_block + prow % BNW, N - 1);
   const uint8_t* pbase = reinterpret_cast<const uint8_t*>(up_rows ? up_words : words);
   const uint8_t* sbase = reinterpret_cast<const uint8_t*>(up_rows ? up_scales : scales);
-  const uint32_t poff = (uint32_t)(((size_t)pn * kw) * 4 + 16 * (lane & 1));
+  uint32_t poff[PL];
+#pragma unroll
+  for (int i = 0; i < PL; ++i) {
+    const int prow = PW * wave + (64 / LPR * i + lane / LPR) % PW;
+    poff[i] = (uint32_t)((size_t)min(n_block + prow % BNW, N - 1) * (K / 8 * BITS) + 16 * (lane % LPR));
+  }
   const int srow = PW * wave + lane % PW;
   const uint32_t soff = (uint32_t)((size_t)min(n_block + srow % BNW, N - 1) * groups * 2);
 
@@ -169,11 +175,13 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
 #pragma unroll
     for (int i = 0; i < XDW; ++i) dma16_raw(xsrc, xoff[i], xb + (wave_u * XDW + i) * 1024);
   };
-  // units k0 / 8 .. + 8 of the row (4 bytes each); the scale dword holding group k0 >> gshift
+  // units k0 / 8 .. + 8 of the row (BITS bytes each); the scale dword holding group k0 >> gshift
   // (groups per row are even, so the aligned pair never leaves the row)
   auto issue_p = [&](int st, uint8_t* pb) __attribute__((always_inline)) {
     const int k0 = kbase + min(st, steps - 1) * kLdsBK;
-    if (2 * PW == 64 || lane < 2 * PW) dma16_raw(pbase + (k0 >> 3) * 4, poff, pb + wave_u * 32 * PW);
+#pragma unroll
+    for (int i = 0; i < PL; ++i)
+      if (LPR * PW >= 64 || lane < LPR * PW) dma16_raw(pbase + (k0 >> 3) * BITS, poff[i], pb + wave_u * PB * PW + i * 1024);
     if (lane < PW) dma4_raw(sbase + ((k0 >> gshift) & ~1) * 2, soff, pb + PT + wave_u * 4 * PW);
   };
 
@@ -182,13 +190,15 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
   int dwr[UPT];
 #pragma unroll
   for (int v = 0; v < UPT; ++v) dwr[v] = lds_unit((t >> 3) + 8 * NW * v, du);
-  const WideMasks km = wide_masks<4>();
-  uint32_t dword[UPT], dscale[UPT];
+  const WideMasks km = wide_masks<BITS>();
+  using Packed = std::conditional_t<BITS == 4, uint32_t, uint2>;  // an 8-code unit
+  Packed dword[UPT];
+  uint32_t dscale[UPT];
   auto expand_read = [&](const uint8_t* pb) __attribute__((always_inline)) {
 #pragma unroll
     for (int v = 0; v < UPT; ++v) {
       const int r = (t >> 3) + 8 * NW * v;
-      dword[v] = *reinterpret_cast<const uint32_t*>(pb + r * 32 + 4 * du);
+      dword[v] = *reinterpret_cast<const Packed*>(pb + r * PB + BITS * du);
       dscale[v] = *reinterpret_cast<const uint32_t*>(pb + PT + 4 * r);
     }
   };
@@ -198,7 +208,7 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
     const int k0 = kbase + min(st, steps - 1) * kLdsBK;
     const int hsel = group == 32 ? (du >> 2) : ((k0 >> gshift) & 1);
     const float s = bf16_to_f32((dscale[v] >> (16 * hsel)) & 0xFFFFu);
-    return wide_dequant(dword[v], wide_scale<4>(s), km);
+    return wide_dequant(dword[v], wide_scale<BITS>(s), km);
   };
 
   // Operand reads: A (p, i) = weight row p BNW + 32 (NT wn + i) + col, B (u) = X row
@@ -229,7 +239,8 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
         for (int u = 0; u < MT; ++u)
           acc[p][i][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[from][p][i], b[from][u], acc[p][i][u], 0, 0, 0);
   };
-  constexpr int DPS = XDW + 2;  // a wave's loads per step
+  constexpr int PLS = PL + 1;      // a wave's packed-word and scale loads per step
+  constexpr int DPS = XDW + PLS;   // ... and all its loads
 
   // Step s: issue step s + XS - 1's X and step s + 3's words; expand step s + 1's
   // words (read at the start, stored over the sub-steps) while the products of
@@ -265,7 +276,7 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
     });
     // step s + 1's X and step s + 2's words are in (with two X buffers step s + 1's X
     // went out at this step's start, ahead of its words)
-    AOTO_WAIT_VMCNT(XS == 3 ? DPS : 2);
+    AOTO_WAIT_VMCNT(XS == 3 ? DPS : PLS);
     AOTO_WAIT_LGKMCNT(0);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");  // no LDS access moves across the barrier
@@ -279,13 +290,13 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
   if constexpr (XS == 3) issue_x(1, xs1);
   issue_p(1, ps1);
   issue_p(2, ps2);
-  AOTO_WAIT_VMCNT(XS == 3 ? DPS + 2 : 4);  // X 0 and words 0
+  AOTO_WAIT_VMCNT(XS == 3 ? DPS + PLS : 2 * PLS);  // X 0 and words 0
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   expand_read(ps0);
 #pragma unroll
   for (int v = 0; v < UPT; ++v) *reinterpret_cast<bf16x8_v*>(ws0 + dwr[v]) = expand(v, 0);
-  AOTO_WAIT_VMCNT(2);  // (X 1 and) words 1
+  AOTO_WAIT_VMCNT(PLS);  // (X 1 and) words 1
   AOTO_WAIT_LGKMCNT(0);
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -440,11 +451,12 @@ __device__ void w4_gemm_lds_body(const uint16_t* __restrict__ X, const uint32_t*
 // aoto_w4_gemm_d{NW}c{WGN}w{MT}x{NT}_split: the single form's split-K partials (f32
 // partials[z][m][n], k slice z of kslice), for short prompts whose column blocks alone
 // do not fill the chip; a reduce kernel applies the epilogue.
-#define AOTO_GEMM_LDS_SPLIT_INSTANCE(NW, WGN, MT, NT)                                                         \
-  extern "C" __global__ __launch_bounds__(64 * NW, 1) void aoto_w4_gemm_d##NW##c##WGN##w##MT##x##NT##_split(   \
+#define AOTO_GEMM_LDS_SPLIT_INSTANCE(BITS, NW, WGN, MT, NT)                                                    \
+  extern "C" __global__ __launch_bounds__(64 * NW, 1) void                                                    \
+      aoto_w##BITS##_gemm_d##NW##c##WGN##w##MT##x##NT##_split(                                                  \
       const uint16_t* X, const uint32_t* words, const uint16_t* scales, float* partials, int M, int N, int K, \
       int group, int kslice) {                                                                                \
-    aoto::w4_gemm_lds_body<NW, WGN, MT, NT, false, false, false, true>(                                       \
+    aoto::w4_gemm_lds_body<NW, WGN, MT, NT, false, false, false, true, BITS>(                                     \
         X, words, scales, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K, group, partials, kslice);     \
   }
 // aoto_w4_gemm_d{NW}c1w{MT}x{NT}_paired: the same with one wave along n (at NW = 4,

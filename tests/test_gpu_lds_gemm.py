@@ -449,3 +449,28 @@ def test_modelled_plans_match_one_fixed_plan_and_fit_their_workspace(m, n, k, gr
         for a, b in zip(results[0][1:], results[1][1:]):  # two rotated bf16 values, each an ulp off at most
             assert float((a.float() - b.float()).abs().max()) <= 2.0 ** -6 * float(b.float().abs().max())
         assert bool((whole[room.numel():] == 7.25).all())
+
+
+@pytest.mark.parametrize("bits,tile", [(4, 815), (4, 825), (8, 833), (8, 834), (8, 845)])
+@pytest.mark.parametrize("m,n,k,group,splits", [(1, 128, 128, 64, 1), (33, 144, 320, 32, 2), (129, 256, 1152, 64, 3),
+                                                (257, 400, 1280, 128, 1), (300, 1040, 1280, 64, 4), (260, 128, 768, 32, 12)])
+def test_split_forms_over_both_widths(m, n, k, group, splits, tile, bits):
+    """The 128-column and 8-bit split forms at row, column and slice remainders, slices of one to many 64-k steps and
+    32- to 128-code groups, against unsplit 64 x 64 tiles: K / 8 roundings of partial sums below six deviations in
+    each order, then a bf16 ulp where they round apart."""
+
+    from aotolith_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k + tile)
+    packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda") * 0.02).bfloat16(), group, bits)
+    x = torch.randn(m, k, generator=gen, device="cuda").bfloat16()
+    residual = torch.randn(m, n, generator=gen, device="cuda").bfloat16()
+    matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
+    got = matmul(x, packed, scales, group, residual=residual, tile=tile, splits=splits).float()
+    want = matmul(x, packed, scales, group, residual=residual, tile=14, splits=1).float()
+    room = 2 * (k / 8) * 2.0 ** -24 * 6 * 0.02 * k ** 0.5 + 2.0 ** -7 * want.abs()
+    assert bool(((got - want).abs() <= room).all())
+    other = ops.w8_matmul if bits == 4 else ops.w4_matmul
+    packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda")).bfloat16(), group, 12 - bits)
+    with pytest.raises(Exception, match="form without a gate epilogue"):
+        other(x, packed, scales, group, tile=tile, splits=splits)
