@@ -392,6 +392,27 @@ def test_packers_at_the_edges_of_their_units(n, k, group, source, bits):
         assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("scale", [1e-37, 1e-30, 3e-3, 1.0, 0.7, 1e30, 1e36])
+def test_packers_codes_at_halves(scale, bits):
+    """Weights a few last places around each half of their group's scale, where the rounding of a quotient
+    decides the code, at scales with and without a normal reciprocal: the bits of the exact quotient."""
+
+    from oracle.quant import pack_weight_bits_bf16
+
+    top = 7 if bits == 4 else 127
+    rng = np.random.default_rng(bits)
+    unit = np.float32(scale)
+    halves = (rng.integers(-2 * top, 2 * top + 1, (64, 1024)) / 2).astype(np.float32) * unit
+    weight = (halves.view(np.int32) + rng.integers(-3, 4, halves.shape, dtype=np.int32) * (halves != 0)).view(np.float32)
+    weight[:, ::64] = top * unit
+    weight = np.clip(weight, -top * unit, top * unit)
+    ref_packed, ref_scales = pack_weight_bits_bf16(weight, 64, bits)
+    packed, scales = _ops().quantize(torch.from_numpy(weight).cuda(), 64, bits)
+    np.testing.assert_array_equal(packed.cpu().numpy(), ref_packed)
+    np.testing.assert_array_equal(bf16_bits_of(scales), ref_scales)
+
+
 @pytest.mark.parametrize("n,k,group", [
     (1, 64, 32), (3, 128, 64), (130, 512, 64), (77, 1024, 128), (257, 1152, 64), (66, 1088, 32), (515, 2048, 64),
     (129, 2560, 128), (131, 3200, 32), (70, 5120, 64), (65, 6016, 64), (33, 6272, 64), (514, 8192, 128), (37, 10240, 64),
