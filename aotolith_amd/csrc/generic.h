@@ -10,10 +10,13 @@
 // target executes per node (runtime/mlx_ops/__init__.py:239-620) without its
 // per-op MLX dispatch: every node is one gfx950 launch.
 //
-// These kernels serve generality (any static-shape module), not the decoder's
-// hot path: they favour simple, always-in-bounds index arithmetic over speed.
-// Every op reads through element strides, so views (permute, expand, slice,
-// unsqueeze) never copy.
+// The kernels of this file take any static-shape module's strides, types and
+// ranks: simple, always-in-bounds index arithmetic. The layouts that models mostly
+// have go to faster forms: f32 and bf16 products and attention on the matrix cores
+// (generic_gemm.h, generic_attention.h), chains of contiguous elementwise nodes in
+// one launch of 16-byte vectors and copies of contiguous rows (below). Every op
+// reads through element strides, so views (permute, expand, slice, unsqueeze) never
+// copy.
 #pragma once
 
 #include "aoto_hip.h"

@@ -1,6 +1,7 @@
-// Prefill W4 GEMM with each packed tile dequantized once per block into LDS (long
-// prompts on 256-row blocks of 8 waves; short prompts on 128-row blocks of 4 waves:
-// the paired gate/up, and single projections as split-K partials).
+// Prefill GEMM over packed 4-bit codes (and 8-bit ones, in the split form) with each
+// packed tile dequantized once per block into LDS (long prompts on 256-row blocks of 8
+// waves; short prompts on 128-row blocks of 4 waves: the paired gate/up, and single
+// projections as split-K partials, which also come on 256 x 128 blocks of 8 waves).
 //
 //   Y[m][n] = epilogue( sum_k X[m][k] * bf16(code[n][k] * s[n][k/group]) )
 //

@@ -136,13 +136,18 @@ int aoto_hip_w4_gemv(const void* x, const int32_t* words, const void* scales,
  * 32) blocks of 4 waves; 4-bit codes, unsplit, no gate epilogue, K % 64 == 0, an even number of
  * power-of-two groups per row, x and the packed words under 2 GiB); 814 / 813 its split-K form
  * for single projections (128 x 64 / 128 x 32 blocks of 4 waves storing f32 partials that the
- * reduce launch sums with the epilogue, at every split count, so they always take a workspace).
+ * reduce launch sums with the epilogue, at every split count, so they always take a workspace);
+ * 815 / 825 the same on 128 x 128 blocks of 4 waves / 256 x 128 of 8; 8-bit codes: 834 / 833 / 845
+ * for 814 / 813 / 825.
  * Automatic codes take the dequant-once kernel for 4-bit codes from M >= 1024 when its grid's
  * last round of 256 blocks is at least 90% full, for a paired gate/up of 32-256 rows on 128-row
  * blocks (812 where that gives >= 128 blocks from 65 rows, else 811 within 256 blocks), for a
  * single projection of 32-256 rows with K >= 2048 and no RoPE epilogue the split form (814
  * where that gives >= 64 column blocks, else 813), else the wide kernel from M >= 512 when
- * K % 256 == 0 (group <= 128), else the 16x16 kernel. splits: 0 chooses (small
+ * K % 256 == 0 (group <= 128), else the instance and split count of a cost model fitted to
+ * measured times where it promises 10% less than the 16x16 kernel (not for a paired gate/up or
+ * N > K at M <= 256, nor q/k/v on 32-row blocks), else the 16x16 kernel. The workspace queries
+ * cover that choice (at most 8 slices, 6 paired, and 32 MiB). splits: 0 chooses (small
  * grids split the reduction), else the split-K count; a split launch stores f32
  * partial tiles in `workspace` (aoto_hip_w4_gemm_workspace() bytes, 16-byte
  * aligned) and a second launch sums them and applies the epilogue. Every plan is
