@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 from collections.abc import Callable
 
 import torch
@@ -365,17 +366,25 @@ def _fused_step(node: Node, meta) -> tuple[int, list, float] | None:
     return code, operands, alpha
 
 
+def _operand_key(operand):
+    """What makes two operands one: a value's name, or a scalar's bits (0.0 == -0.0 in Python, not in a division)."""
+
+    return operand if isinstance(operand, Ref) else struct.pack("<d", operand)
+
+
 def _chain(members: list[Node], steps: dict) -> FusedChain | None:
     """The members (in graph order, the root last) as a program, or None past its operands, steps or registers."""
 
     names = {node.name for node in members}
     inputs: list = []
+    slots: dict = {}  # operand key -> its position in `inputs`
     last_use: dict[str, int] = {}
     for index, node in enumerate(members):
         for operand in steps[node.name][1]:
             if isinstance(operand, Ref) and operand.name in names:
                 last_use[operand.name] = index
-            elif operand not in inputs:
+            elif _operand_key(operand) not in slots:
+                slots[_operand_key(operand)] = len(inputs)
                 inputs.append(operand)
     if len(inputs) > _MAX_FUSED_INPUTS or len(members) > _MAX_FUSED_STEPS:
         return None
@@ -384,7 +393,8 @@ def _chain(members: list[Node], steps: dict) -> FusedChain | None:
     program, alphas = [], []
     for index, node in enumerate(members):
         code, operands, alpha = steps[node.name]
-        sources = [register[o.name] if isinstance(o, Ref) and o.name in names else 4 + inputs.index(o) for o in operands]
+        sources = [register[o.name] if isinstance(o, Ref) and o.name in names else 4 + slots[_operand_key(o)]
+                   for o in operands]
         for name in {o.name for o in operands if isinstance(o, Ref) and o.name in names}:
             if last_use[name] == index:
                 free.append(register[name])

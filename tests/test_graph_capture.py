@@ -116,3 +116,38 @@ def test_graph_encoding_round_trips_through_json():
     ids = config1_ids(13)
     np.testing.assert_array_equal(GraphOracle(again).run({graph.inputs[0]: ids})[0],
                                   GraphOracle(graph).run({graph.inputs[0]: ids})[0])
+
+
+def _run_program(chain, values, node_types):
+    """A fused chain's program over CPU tensors: registers 0..3, then the operands."""
+
+    from aotolith_amd.graph_ops import EW
+
+    names = {code: name for name, code in EW.items()}
+    regs: dict[int, torch.Tensor] = {}
+    for i in range(chain.count):
+        code, dst, a, b, _ = chain.program[5 * i:5 * i + 5]
+        x, y = (regs[s] if s < 4 else values[s - 4] for s in (a, b))
+        x, y = (v.float() if isinstance(v, torch.Tensor) else torch.tensor(v, dtype=torch.float32) for v in (x, y))
+        fn = {"add": torch.add, "sub": torch.sub, "mul": torch.mul, "div": torch.div}[names[code]]
+        regs[dst] = fn(x, y).to(node_types[i]).float()
+    return regs[dst]
+
+
+@pytest.mark.parametrize("fn", [lambda x: x / 0.0 + x / -0.0, lambda x: (x + 0.0) * (x / -0.0),
+                                lambda x: (x * -0.0) * 0.0 + (x - 0.0) / -0.0, lambda x: x * 1.0 + x * 1])
+def test_a_fused_chain_keeps_scalars_of_different_bits_apart(fn):
+    """The program of each chain, interpreted here, has the bits of eager torch: 0.0 and -0.0 are two operands."""
+
+    from aotolith_amd.graph import capture
+    from aotolith_amd.graph_ops import fuse_elementwise
+
+    x = torch.tensor([1.0, -2.0, 0.0, 3.5, -0.5, 7.0, -0.0, 2.0])
+    graph = capture(fn, (x,))
+    chain, = fuse_elementwise(graph)
+    assert [n.name for n in chain.members] == [n.name for n in graph.nodes]
+    values = [x if not isinstance(v, (int, float)) else v for v in chain.inputs]
+    got = _run_program(chain, values, [n.dtype for n in chain.members])
+    want = fn(x)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num().view(torch.int32), want.nan_to_num().view(torch.int32))
