@@ -16,7 +16,8 @@
 //
 // Values that are not finite: 0 * inf would poison every query through the product, so they enter it as
 // zeros, and a tile that holds any runs a second pass (special_values) that gives +-inf / NaN to the
-// queries whose probability of such a key is not zero.
+// queries whose probability of such a key is not zero. A kept score that is NaN makes its query NaN: it stays
+// in the running sum, which no rescale to zero drops.
 //
 // Bound: latency (two tiles a wave at 512 keys), then the MFMA pipe. 14 heads of 64, 512 tokens,
 // causal, bf16: 881 us with one block per query row and scalar dots (every score a 64-step chain of
@@ -271,8 +272,8 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     const float correction = run_max == moved || run_max == -INFINITY ? 1.f : expf(run_max - moved);
     run_max = moved;
     if (__any(correction != 1.f)) {
-      // a correction of zero drops what was summed, infinities too
-      run_sum = correction == 0.f ? 0.f : run_sum * correction;
+      // a correction of zero drops the products, infinities too, and of the sum all but a NaN
+      run_sum *= correction;
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -342,7 +343,7 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     factor[w] = other[lane] == -INFINITY ? 1.f : expf(other[lane] - big);
     // both halves' keys
     const float l = other[64 + col] + other[64 + 32 + col];
-    if (factor[w] != 0.f) sum += l * factor[w];
+    sum += l * factor[w];
   }
   if (qi >= a.lq) return;
   const float inv = sum > 0.f ? 1.0f / sum : 0.f;
@@ -359,8 +360,8 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
         const float x = reinterpret_cast<const float*>(lds[w])[(2 + 4 * g + i) * 64 + lane];
         if (factor[w] != 0.f) v += x * factor[w];
       }
-      // a row with no kept key (and one whose scores are all NaN) gives zeros
-      store_float_type(a.out, a.out_dtype, ob + d, big == -INFINITY ? 0.f : v * inv);
+      // a row with no kept key (and one whose kept scores are all NaN or -inf) gives zeros
+      store_float_type(a.out, a.out_dtype, ob + d, big == -INFINITY ? 0.f : sum != sum ? sum : v * inv);
     }
   }
 }

@@ -332,6 +332,53 @@ def test_attention_over_its_tiles_layouts_masks_and_types(batch, heads, kv_heads
         assert bool(((got - want).abs() <= bound)[fine].all())
 
 
+@pytest.mark.parametrize("types", ["bf16", "f32"])
+@pytest.mark.parametrize("d", [64, 128, 160])
+@pytest.mark.parametrize("case", ["nan", "nan_outweighed", "nan_outweighed_by_another_wave", "inf", "minus_inf",
+                                  "only_nan"])
+def test_attention_with_scores_that_are_not_finite(case, d, types):
+    """Every form alike: a kept score that is NaN or +inf makes its query NaN however small it is beside a later one, a
+    masked one does not, and a query with no kept score above -inf gives zeros."""
+
+    from aotolith_amd.graph_ops import launch_attention
+
+    dtype = torch.bfloat16 if types == "bf16" else torch.float32
+    lq, lk = 3, 600
+    gen = torch.Generator().manual_seed(d)
+    scores = torch.zeros(lk)
+    v = torch.randn(1, 1, lk, d, generator=gen)
+    mask = torch.ones(1, 1, lq, lk, dtype=torch.bool)
+    mask[..., 2, 5] = False  # the last query does not keep the key in question
+    scores[5] = {"inf": float("inf"), "minus_inf": float("-inf")}.get(case, float("nan"))
+    if case == "nan_outweighed":
+        scores[261] = 200.0
+    if case == "nan_outweighed_by_another_wave":
+        scores[5 + 64 + 32] = 200.0
+    if case == "only_nan":
+        mask[...] = False
+        mask[..., :2, 5] = True
+    q, k = torch.zeros(1, 1, lq, d), torch.zeros(1, 1, lk, d)
+    q[..., 0], k[..., 0] = 8.0, scores
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+
+    kept = torch.where(mask, scores.double(), -torch.inf)[0, 0]
+    top = kept.nan_to_num(nan=-torch.inf, posinf=torch.inf, neginf=-torch.inf).amax(-1, keepdim=True)
+    broken = (mask[0, 0] & scores.isnan()).any(-1, keepdim=True) | (top == torch.inf)
+    p = torch.exp(kept - top).float().double()  # (an f32's range: what falls below it is zero)
+    p = torch.where(p >= 2.0 ** -149, p, torch.zeros_like(p))
+    want = torch.where(p[..., None] > 0, p[..., None] * v[0, 0].double(), 0.0).sum(1) / p.sum(-1, keepdim=True)
+    want = torch.where(top == -torch.inf, torch.zeros_like(want), want)
+    want = torch.where(broken & (top != -torch.inf), torch.full_like(want, torch.nan), want)
+
+    out = torch.full((1, 1, lq, d), 7.0, device="cuda")
+    launch_attention(out, q.cuda(), k.cuda(), v.cuda(), mask.cuda(), False, 0.125)
+    got = out[0, 0].double().cpu()
+    fine = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), fine) and torch.equal(got.isnan(), want.isnan())
+    # (600 f32 additions of values up to about 4 at most, and the exponentials' last places)
+    assert bool(((got - want).abs() <= 2.0 ** -24 * 1200 * 4)[fine].all())
+
+
 def _views(gen, dtype):
     """Pairs of operands of one broadcast shape: collapsible, broadcast, permuted, offset and odd-sized."""
 
