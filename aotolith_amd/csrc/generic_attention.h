@@ -15,9 +15,10 @@
 // f32 (and mixed) operands: 32-key tiles on v_mfma_f32_32x32x2_f32, V read in operand order.
 //
 // Values that are not finite: 0 * inf would poison every query through the product, so they enter it as
-// zeros, and a tile that holds any runs a second pass (special_values) that gives +-inf / NaN to the
-// queries whose probability of such a key is not zero. A kept score that is NaN makes its query NaN: it stays
-// in the running sum, which no rescale to zero drops.
+// zeros, and a wave that met any goes over its tiles once more (special_values) with the row's final
+// maximum and gives +-inf / NaN to the queries whose probability of such a key is not zero. (Within the loop
+// a key's probability is still relative to the maximum so far: one that ends as zero may not be zero yet.)
+// A kept score that is NaN makes its query NaN: it stays in the running sum, which no rescale to zero drops.
 //
 // Bound: latency (two tiles a wave at 512 keys), then the MFMA pipe. 14 heads of 64, 512 tokens,
 // causal, bf16: 881 us with one block per query row and scalar dots (every score a 64-step chain of
@@ -132,8 +133,54 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     return load_float(a.v, a.v_dtype, vbase + (long long)j * a.vs[2] + (long long)d * a.vs[3]);
   };
 
-  f32x16_t o[DT] = {}, p[KT];
+  f32x16_t o[DT] = {}, p[KT], sc[KT];
   float run_max = -INFINITY, run_sum = 0.f;
+
+  // sc = K . q of the loaded keys
+  auto products = [&]() {
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub) {
+      sc[sub] = f32x16_t{};
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if constexpr (F32) {
+          const uint32_t kw[4] = {kf[sub][s].x, kf[sub][s].y, kf[sub][s].z, kf[sub][s].w};
+          const uint32_t qw[4] = {qf[s].x, qf[s].y, qf[s].z, qf[s].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sc[sub] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kw[e]), __uint_as_float(qw[e]), sc[sub], 0,
+                                                           0, 0);
+        } else {
+          sc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[sub][s]),
+                                                            __builtin_bit_cast(bf16x8_t, qf[s]), sc[sub], 0, 0, 0);
+        }
+      }
+    }
+  };
+  // p = the scaled and masked scores of sc; returns the lane's largest
+  const long long mrow = b * a.ms[0] + h * a.ms[1] + (long long)qrow * a.ms[2];
+  auto masked_scores = [&](int j0) -> float {
+    float top = -INFINITY;
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int j = j0 + 32 * sub + 8 * (e >> 2) + 4 * half + (e & 3);
+        bool keep = j < a.lk && !(a.causal && j > qi);
+        float add = 0.f;
+        if (a.mask != nullptr && keep) {
+          const long long mo = mrow + (long long)j * a.ms[3];
+          if (a.mask_dtype == AOTO_DT_BOOL)
+            keep = static_cast<const uint8_t*>(a.mask)[mo] != 0;
+          else
+            add = load_float(a.mask, a.mask_dtype, mo);
+        }
+        const float v = keep ? sc[sub][e] * a.scale + add : -INFINITY;
+        p[sub][e] = v;
+        top = fmaxf(top, v);
+      }
+    return top;
+  };
 
   // +-inf and NaN of a tile's values, for the queries whose p of their key is not zero: per class, the
   // product of the class's indicator with [p != 0], and the special value where it is not zero. The
@@ -195,11 +242,11 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     load_keys(wave * BK);
     load_values(wave * BK);
   }
+  bool odd = false;  // the lane has met a value that is not finite
   for (int tile = wave; tile < tiles; tile += kGenAttnWaves) {
     const int j0 = tile * BK;
     const int next = min(tile + kGenAttnWaves, tiles - 1) * BK;
 
-    bool odd = false;  // a value that is not finite
     if constexpr (!F32) {
       wave_lds_order();
 #pragma unroll
@@ -223,56 +270,18 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
       wave_lds_order();
     }
 
-    f32x16_t sc[KT];
-#pragma unroll
-    for (int sub = 0; sub < KT; ++sub) {
-      sc[sub] = f32x16_t{};
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        if constexpr (F32) {
-          const uint32_t kw[4] = {kf[sub][s].x, kf[sub][s].y, kf[sub][s].z, kf[sub][s].w};
-          const uint32_t qw[4] = {qf[s].x, qf[s].y, qf[s].z, qf[s].w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            sc[sub] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kw[e]), __uint_as_float(qw[e]), sc[sub], 0,
-                                                           0, 0);
-        } else {
-          sc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[sub][s]),
-                                                            __builtin_bit_cast(bf16x8_t, qf[s]), sc[sub], 0, 0, 0);
-        }
-      }
-    }
+    products();
     // the next tile's loads work under this one's softmax and products (the last trip reads its own again)
     load_keys(next);
     load_values(next);
 
-    float tile_max = -INFINITY;
-    const long long mrow = b * a.ms[0] + h * a.ms[1] + (long long)qrow * a.ms[2];
-#pragma unroll
-    for (int sub = 0; sub < KT; ++sub)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int j = j0 + 32 * sub + 8 * (e >> 2) + 4 * half + (e & 3);
-        bool keep = j < a.lk && !(a.causal && j > qi);
-        float add = 0.f;
-        if (a.mask != nullptr && keep) {
-          const long long mo = mrow + (long long)j * a.ms[3];
-          if (a.mask_dtype == AOTO_DT_BOOL)
-            keep = static_cast<const uint8_t*>(a.mask)[mo] != 0;
-          else
-            add = load_float(a.mask, a.mask_dtype, mo);
-        }
-        const float v = keep ? sc[sub][e] * a.scale + add : -INFINITY;
-        p[sub][e] = v;
-        tile_max = fmaxf(tile_max, v);
-      }
-    tile_max = xor32_max(tile_max);
+    const float tile_max = xor32_max(masked_scores(j0));
     const float moved = fmaxf(run_max, tile_max);
     // (a maximum of -inf has only zeros, or a NaN score's NaN, behind it: kept as they are)
     const float correction = run_max == moved || run_max == -INFINITY ? 1.f : expf(run_max - moved);
     run_max = moved;
     if (__any(correction != 1.f)) {
-      // a correction of zero drops the products, infinities too, and of the sum all but a NaN
+      // a correction of zero drops the products, overflowed ones too, and of the sum all but a NaN
       run_sum *= correction;
 #pragma unroll
       for (int t = 0; t < DT; ++t)
@@ -320,21 +329,18 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
         }
       }
     }
-    if (__any(odd)) special_values(j0);
   }
 
-  // The waves' states (the V stages are dead: a wave's records lie in its own), combined by all four:
-  // wave w takes every fourth run of 4 output columns.
+  // The waves' states (the V stages are dead: a wave's records lie in its own): maxima and sums first, whose
+  // sign bit says that the wave has met a value that is not finite.
+  const bool special = __any(odd);
   wave_lds_order();
   float* rec = reinterpret_cast<float*>(lds[wave]);
   rec[lane] = run_max;
-  rec[64 + lane] = run_sum;
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) rec[(2 + 16 * t + e) * 64 + lane] = o[t][e];
+  rec[64 + lane] = __uint_as_float((__float_as_uint(run_sum) & 0x7FFFFFFFu) | (special ? 0x80000000u : 0u));
   __syncthreads();
   float big = -INFINITY, sum = 0.f, factor[kGenAttnWaves];
+  uint32_t any_special = 0u;
 #pragma unroll
   for (int w = 0; w < kGenAttnWaves; ++w) big = fmaxf(big, reinterpret_cast<const float*>(lds[w])[lane]);
 #pragma unroll
@@ -342,9 +348,32 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     const float* other = reinterpret_cast<const float*>(lds[w]);
     factor[w] = other[lane] == -INFINITY ? 1.f : expf(other[lane] - big);
     // both halves' keys
-    const float l = other[64 + col] + other[64 + 32 + col];
+    any_special |= __float_as_uint(other[64 + col]);
+    const float l = fabsf(other[64 + col]) + fabsf(other[64 + 32 + col]);
     sum += l * factor[w];
   }
+  if (any_special >> 31) {  // (uniform)
+    __syncthreads();  // the maxima and sums are read: the special pass stages over them
+    if (special) {
+      for (int tile = wave; tile < tiles; tile += kGenAttnWaves) {
+        load_keys(tile * BK);
+        products();
+        masked_scores(tile * BK);
+#pragma unroll
+        for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) p[sub][e] = p[sub][e] == -INFINITY ? 0.f : expf(p[sub][e] - big);
+        special_values(tile * BK);
+      }
+    }
+  }
+  // The products' records, combined by all four waves: wave w takes every fourth run of 4 output columns.
+  wave_lds_order();
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) rec[(2 + 16 * t + e) * 64 + lane] = o[t][e];
+  __syncthreads();
   if (qi >= a.lq) return;
   const float inv = sum > 0.f ? 1.0f / sum : 0.f;
   const long long ob = ((long long)(b * a.heads + h) * a.lq + qi) * a.dv;

@@ -335,10 +335,11 @@ def test_attention_over_its_tiles_layouts_masks_and_types(batch, heads, kv_heads
 @pytest.mark.parametrize("types", ["bf16", "f32"])
 @pytest.mark.parametrize("d", [64, 128, 160])
 @pytest.mark.parametrize("case", ["nan", "nan_outweighed", "nan_outweighed_by_another_wave", "inf", "minus_inf",
-                                  "only_nan"])
+                                  "only_nan", "underflowed_value"])
 def test_attention_with_scores_that_are_not_finite(case, d, types):
     """Every form alike: a kept score that is NaN or +inf makes its query NaN however small it is beside a later one, a
-    masked one does not, and a query with no kept score above -inf gives zeros."""
+    masked one does not, a query with no kept score above -inf gives zeros, and an infinite value whose key's
+    probability ends as zero (after two rescales that are not zero each) contributes nothing."""
 
     from aotolith_amd.graph_ops import launch_attention
 
@@ -349,14 +350,18 @@ def test_attention_with_scores_that_are_not_finite(case, d, types):
     v = torch.randn(1, 1, lk, d, generator=gen)
     mask = torch.ones(1, 1, lq, lk, dtype=torch.bool)
     mask[..., 2, 5] = False  # the last query does not keep the key in question
-    scores[5] = {"inf": float("inf"), "minus_inf": float("-inf")}.get(case, float("nan"))
-    if case == "nan_outweighed":
-        scores[261] = 200.0
-    if case == "nan_outweighed_by_another_wave":
-        scores[5 + 64 + 32] = 200.0
-    if case == "only_nan":
-        mask[...] = False
-        mask[..., :2, 5] = True
+    if case == "underflowed_value":  # keys 5, 261 and 517 fall to one wave, whatever the tile
+        scores[5], scores[261], scores[517] = 0.0, 60.0, 120.0
+        v[0, 0, 5, 1], v[0, 0, 5, 2], v[0, 0, 261, 3] = float("inf"), float("nan"), float("-inf")
+    else:
+        scores[5] = {"inf": float("inf"), "minus_inf": float("-inf")}.get(case, float("nan"))
+        if case == "nan_outweighed":
+            scores[261] = 200.0
+        if case == "nan_outweighed_by_another_wave":
+            scores[5 + 64 + 32] = 200.0
+        if case == "only_nan":
+            mask[...] = False
+            mask[..., :2, 5] = True
     q, k = torch.zeros(1, 1, lq, d), torch.zeros(1, 1, lk, d)
     q[..., 0], k[..., 0] = 8.0, scores
     q, k, v = (t.to(dtype) for t in (q, k, v))
