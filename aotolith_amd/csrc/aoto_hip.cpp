@@ -959,9 +959,29 @@ bool models_plans() { return has_kernel("aoto_w8_gemm_d8c2w2x2_split"); }
 
 }  // namespace
 
+namespace {
+
+// Automatic codes where the scales start at an odd element: the 16x16 kernel, which reads them one by one (the
+// dequant-once and wide kernels read aligned pairs), with its own split count as far as a workspace of `room`
+// bytes holds it.
+void unpaired_scales_plan(int M, int N, int K, bool paired, size_t room, int* tile, int* splits) {
+  const GemmPlan p = gemm_plan(M, N, K, 0, 0, paired);
+  const size_t slices = room / ((size_t)M * N * sizeof(float) * (paired ? 2 : 1));
+  *tile = 10 * p.tn + p.tm;
+  *splits = (size_t)p.splits <= slices ? p.splits : slices > 1 ? (int)slices : 1;
+}
+
+}  // namespace
+
 // Automatic codes resolved to the explicit plan aoto_hip_w4_gemm would run (for
 // the allocation-free entry point, which sizes its split against its scratch).
-extern "C++" void aoto::resolve_gemm_codes(int M, int N, int K, int group, bool gate, int* tile, int* splits) {
+// scale_pairs: the scales are 4-byte aligned.
+extern "C++" void aoto::resolve_gemm_codes(int M, int N, int K, int group, bool gate, bool scale_pairs, int* tile,
+                                           int* splits) {
+  if (*tile == 0 && *splits == 0 && !scale_pairs) {
+    unpaired_scales_plan(M, N, K, false, aoto_hip_w4_gemm_workspace(M, N, K, 0, 0), tile, splits);
+    return;
+  }
   if (*tile == 0 && *splits == 0) {
     if (const int code = lds_auto(4, M, N, K, group, false, gate, false)) {
       *tile = code;
@@ -1115,6 +1135,15 @@ int packed_gemm(int bits, const void* x, const int32_t* words, const void* scale
       return fail(AOTO_ERR_UNSUPPORTED, "%s: wide tile %d needs K %% 128 == 0 and an even number of "
                   "power-of-two groups per row (K=%d group=%d)", what, tile, K, group);
   }
+  const bool scale_pairs = aligned4(scales) && (!paired || aligned4(up_scales));
+  if (!scale_pairs && (lds_code(tile) || wide_code(tile)))
+    return fail(AOTO_ERR_ARGUMENT, "%s: tile %d reads scales as pairs: they must be 4-byte aligned", what, tile);
+  if (tile == 0 && splits == 0 && !scale_pairs) {
+    const size_t room = workspace == nullptr ? 0
+                        : paired             ? aoto_hip_w4_gemm_gate_up_workspace(M, N, K, 0, 0)
+                                             : aoto_hip_w4_gemm_workspace(M, N, K, 0, 0);
+    unpaired_scales_plan(M, N, K, paired, room, &tile, &splits);
+  }
   if (tile == 0 && splits == 0) {
     if (const int code = lds_auto(bits, M, N, K, group, paired, gate != nullptr, rope != nullptr))
       tile = code;
@@ -1237,7 +1266,8 @@ int qkv_rope_gemm(int bits, const void* x, const int32_t* words, const void* sca
   if (!wide_auto_rows(M, K)) {
     const bool automatic = tile == 0 && splits == 0;
     qkv_rope_plan(M, N, K, head_dim, &tile, &splits);
-    if (automatic && group > 0 && modelled_rope(M, K, head_dim) && modelled_shape(bits, M, N, K, group, false, false, true) && models_plans())
+    if (automatic && group > 0 && aligned4(scales) && modelled_rope(M, K, head_dim) &&
+        modelled_shape(bits, M, N, K, group, false, false, true) && models_plans())
       automatic_model(bits, M, N, K, group, kTailRope, false, head_dim, &tile, &splits);
   }
   return packed_gemm(bits, x, words, scales, bias, nullptr, nullptr, y, M, N, K, group, tile, splits, workspace,

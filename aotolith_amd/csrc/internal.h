@@ -12,8 +12,8 @@ int set_error(int code, const char* fmt, ...);
 void noalloc_prepare_device(int device);
 
 // Automatic (0) tile / split codes of the unpaired 4-bit prefill GEMM (group size,
-// gate epilogue or not) resolved to the explicit plan aoto_hip_w4_gemm runs
+// gate epilogue or not, 4-byte aligned scales or not) resolved to the explicit plan aoto_hip_w4_gemm runs
 // (aoto_hip.cpp); other codes pass unchanged.
-void resolve_gemm_codes(int M, int N, int K, int group, bool gate, int* tile, int* splits);
+void resolve_gemm_codes(int M, int N, int K, int group, bool gate, bool scale_pairs, int* tile, int* splits);
 
 }  // namespace aoto

@@ -125,7 +125,8 @@ int aoto_hip_w4_gemv(const void* x, const int32_t* words, const void* scales,
  *   residual bf16 [M, N]  -> bf16(residual[m][n] + acc)
  *   gate     bf16 [M, N]  -> bf16(acc * silu(gate[m][n]))
  * Limits: K % 64 == 0, N % 16 == 0, group % 32 == 0 dividing K. x 16-byte and
- * y/bias/residual/gate 8-byte aligned. tile: 0 chooses; 12/14/18/24/28 the
+ * y/bias/residual/gate 8-byte aligned; scales 4-byte aligned except for the 16x16
+ * kernel, which automatic codes take for scales that are not. tile: 0 chooses; 12/14/18/24/28 the
  * 16x16x32-MFMA kernel (n tiles x m tiles of 16 per wave; 12: 32-row blocks);
  * 241/242/243/281/441 the wide-tile 32x32x16 kernel for long prompts (100 *
  * waves per block / 2 + 10 * 32-row tiles per wave + 32-column tiles per wave;

@@ -176,3 +176,22 @@ def test_hold_graph_is_released_when_the_graph_is_collected():
     del graph
     gc.collect()
     assert lib.aoto_hip_graph_holds() == 0
+
+
+def test_tiles_that_read_scale_pairs_refuse_scales_at_an_odd_element():
+    """The dequant-once and wide kernels load scales as aligned 32-bit pairs: an explicit code with a base that is only
+    2-byte aligned is an argument error before anything is launched (the addresses here are never read)."""
+
+    from aotolith_amd import _lib, ops
+
+    lib = _lib.library()
+    at = 1 << 20
+    for entry, tiles in ((lib.aoto_hip_w4_gemm, (241, 242, 243, 281, 441, 813, 814, 815, 822, 823, 825)),
+                         (lib.aoto_hip_w8_gemm, (241, 242, 441, 833, 834, 845))):
+        for tile in tiles:
+            status = entry(at, at, at + 2, None, None, None, at, 256, 1024, 1024, 64, tile, 1, at, None)
+            assert status == _lib.AOTO_ERR_ARGUMENT and "4-byte aligned" in _lib.last_error(), tile
+    for tile in (ops.LDS_PAIRED_TILE, 811, 812, 241):
+        for gate, up in ((at + 2, at), (at, at + 2)):
+            status = lib.aoto_hip_w4_gemm_gate_up(at, at, gate, at, up, at, 256, 1024, 1024, 64, tile, 1, at, None)
+            assert status == _lib.AOTO_ERR_ARGUMENT and "4-byte aligned" in _lib.last_error(), tile

@@ -12,6 +12,8 @@ plan's choice at 2048 rows and at short prompts; graph replays against eager; th
 
 from __future__ import annotations
 
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -474,3 +476,84 @@ def test_split_forms_over_both_widths(m, n, k, group, splits, tile, bits):
     packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda")).bfloat16(), group, 12 - bits)
     with pytest.raises(Exception, match="form without a gate epilogue"):
         other(x, packed, scales, group, tile=tile, splits=splits)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(1, 896, 896), (128, 896, 4864), (128, 1152, 896), (300, 896, 896), (333, 1024, 2048),
+                                   (512, 768, 1024), (1030, 640, 896), (2048, 4096, 512)])
+def test_automatic_codes_take_scales_at_an_odd_element(m, n, k, bits):
+    """Scales that start at an odd bf16 (a contiguous view) are read one by one, so every form runs on the 16x16 kernel:
+    the dequant-once and wide kernels load aligned pairs. Against the same call on aligned scales with unsplit 64 x 64
+    tiles, the bound of test_modelled_plans_match_one_fixed_plan_and_fit_their_workspace; nothing past the workspace."""
+
+    from aotolith_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k + bits)
+    group = 64
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(*shape, generator=gen, device="cuda") * std).bfloat16()
+
+    def odd(scales):
+        view = torch.empty(scales.numel() + 1, dtype=torch.bfloat16, device="cuda")[1:].view(scales.shape)
+        view.copy_(scales)
+        assert view.is_contiguous() and view.data_ptr() % 4 == 2
+        return view
+
+    packed, scales = ops.quantize(normal(n, k, std=0.02), group, bits)
+    up, up_scales = ops.quantize(normal(n, k, std=0.02), group, bits)
+    x, residual, weight, bias = normal(m, k), normal(m, n), normal(n), normal(n)
+    matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
+    gate_up = ops.w4_matmul_gate_up if bits == 4 else ops.w8_matmul_gate_up
+    order = 2 * (k / 8) * 2.0 ** -24 * 6 * 0.02 * k ** 0.5
+
+    def check(got, want, factor=1.0, ulps=1.0):
+        room = order * factor + ulps * 2.0 ** -7 * want.float().abs()
+        assert bool(((got.float() - want.float()).abs() <= room).all())
+
+    def workspace(size):
+        whole = torch.full((size // 4 + 4096,), 7.25, device="cuda")
+        return whole, whole[:size // 4]
+
+    def run(fn):
+        out, names = _traced(fn)
+        gemms = [name for name in names if "_gemm_" in name and "_reduce" not in name]
+        assert gemms and all(re.match(r"aoto_w[48]_gemm_n\d_m\d_", name) for name in gemms), names
+        return out
+
+    whole, room = workspace(ops.gemm_workspace_bytes(m, n, k))
+    check(run(lambda: matmul(x, packed, odd(scales), group, bias=bias, workspace=room)),
+          matmul(x, packed, scales, group, bias=bias, tile=14, splits=1))
+    if bits == 4:
+        shifted, y = odd(scales), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        _lib.check(run(lambda: _lib.library().aoto_hip_w4_gemm_noalloc(
+            ops._ptr(x), ops._ptr(packed), ops._ptr(shifted), ops._ptr(bias), None, None, ops._ptr(y), m, n, k, group, 0,
+            0, ops._stream())))
+        check(y, matmul(x, packed, scales, group, bias=bias, tile=14, splits=1))
+    if n <= 4096:
+        got = run(lambda: ops.matmul_residual_norm(x, packed, odd(scales), group, residual, weight, 1e-6, bits=bits,
+                                                   workspace=room))
+        want = ops.matmul_residual_norm(x, packed, scales, group, residual, weight, 1e-6, bits=bits, tile=14, splits=1)
+        check(got[0], want[0])
+    assert bool((whole[room.numel():] == 7.25).all())
+    whole, room = workspace(ops.gate_up_workspace_bytes(m, n, k))
+    want = gate_up(x, packed, scales, up, up_scales, group, tile=14, splits=1)
+    top = 6 * 0.02 * k ** 0.5
+    for pair in ((odd(scales), odd(up_scales)), (scales, odd(up_scales))):
+        got = run(lambda: gate_up(x, packed, pair[0], up, pair[1], group, workspace=room))
+        check(got, want, factor=2 * top, ulps=2 + top)
+    assert bool((whole[room.numel():] == 7.25).all())
+    heads = n // 64 - 2
+    size = int(_lib.library().aoto_hip_w4_gemm_qkv_rope_workspace(m, k, 0, 0, heads, 1, 64))
+    whole, room = workspace(size)
+    cos, sin = normal(m, 64), normal(m, 64)
+    results = []
+    for s, plan in ((odd(scales), dict(workspace=room)), (scales, dict(tile=14, splits=1))):
+        pair = torch.full((2, 1, 1, m, 64), 7.0, dtype=torch.bfloat16, device="cuda")
+        results.append(run(lambda: ops.matmul_qkv_rope(
+            x, packed, s, group, torch.arange(m, device="cuda"), cos, sin, pair, query_heads=heads, kv_heads=1,
+            head_dim=64, slot0=0, bias=bias, bits=bits, **plan)) + (pair,))
+    check(results[0][0], results[1][0])
+    for a, b in zip(results[0][1:], results[1][1:]):
+        assert float((a.float() - b.float()).abs().max()) <= 2.0 ** -6 * float(b.float().abs().max())
+    assert bool((whole[room.numel():] == 7.25).all())
