@@ -789,6 +789,13 @@ GemmPlan gemm_plan(int M, int N, int K, int tile, int splits, bool paired) {
     // (Llama-8B shapes, gate/up at M = 512 / 2048: 161 / 571 us at 64 columns,
     // 183 / 638 at 128).
     p.tn = !paired && (p.tm == 8 || mb * ((N + 127) / 128) >= 256) ? 2 : 1;
+    // Wide outputs of up to 128 rows (that grid on 32-row blocks has no instance): 64 columns, on 64-row blocks
+    // from 33 rows (us on 32- / 64-row blocks: 64 rows, 1024 -> 16384 9.4 / 8.9, -> 151936 59.5 / 43.8; 16 rows,
+    // 896 -> 151936 25.1 / 33.1; 128 columns on 64-row blocks 11.8, 38.6, 29.3).
+    if (p.tm == 2 && p.tn == 2) {
+      p.tn = 1;
+      p.tm = M > 32 ? 4 : 2;
+    }
   } else {
     p.tn = tile / 10;
     p.tm = tile % 10;

@@ -557,3 +557,20 @@ def test_automatic_codes_take_scales_at_an_odd_element(m, n, k, bits):
     for a, b in zip(results[0][1:], results[1][1:]):
         assert float((a.float() - b.float()).abs().max()) <= 2.0 ** -6 * float(b.float().abs().max())
     assert bool((whole[room.numel():] == 7.25).all())
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(128, 8192, 512), (97, 8208, 448), (33, 16400, 512), (16, 32768, 256), (32, 32784, 320)])
+def test_automatic_codes_at_wide_outputs_of_few_rows(m, n, k, bits):
+    """From 256 blocks of 32 x 128 on, up to 128 rows: an instance that the code object has, with the bits of the same
+    k order on 64 x 64 tiles."""
+
+    from aotolith_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda") * 0.02).bfloat16(), 64, bits)
+    x = torch.randn(m, k, generator=gen, device="cuda").bfloat16()
+    bias = torch.randn(n, generator=gen, device="cuda").bfloat16()
+    matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
+    assert torch.equal(matmul(x, packed, scales, 64, bias=bias),
+                       matmul(x, packed, scales, 64, bias=bias, tile=14, splits=1))
