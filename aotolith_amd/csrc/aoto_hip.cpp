@@ -985,31 +985,30 @@ void unpaired_scales_plan(int M, int N, int K, bool paired, size_t room, int* ti
 // scale_pairs: the scales are 4-byte aligned.
 extern "C++" void aoto::resolve_gemm_codes(int M, int N, int K, int group, bool gate, bool scale_pairs, int* tile,
                                            int* splits) {
-  if (*tile == 0 && *splits == 0 && !scale_pairs) {
+  if (*tile != 0 || *splits != 0) return;
+  if (!scale_pairs) {
     unpaired_scales_plan(M, N, K, false, aoto_hip_w4_gemm_workspace(M, N, K, 0, 0), tile, splits);
     return;
   }
-  if (*tile == 0 && *splits == 0) {
-    if (const int code = lds_auto(4, M, N, K, group, false, gate, false)) {
-      *tile = code;
-      *splits = gemm_plan(M, N, K, code, 0, false).splits;  // 1 unless the short split form
-      return;
-    }
-    if (modelled_shape(4, M, N, K, group, false, gate, false) && models_plans()) {
-      const GemmPlan fixed = gemm_plan(M, N, K, 0, 0, false);
-      if (automatic_model(4, M, N, K, group, kTailNorm, gate, 0, tile, splits)) {
-        const GemmPlan p = gemm_plan(M, N, K, *tile, *splits, false);
-        if ((p.splits == 1 && !lds_split_code(*tile)) ||
-            (size_t)p.splits * M * N * sizeof(float) <= AOTO_HIP_NOALLOC_SCRATCH_BYTES)
-          return;
-      }
-      // (the fixed plan by name: automatic codes would come back to the modelled one)
-      *tile = 10 * fixed.tn + fixed.tm;
-      *splits = fixed.splits;
-      return;
-    }
+  if (const int code = lds_auto(4, M, N, K, group, false, gate, false)) {
+    *tile = code;
+    *splits = gemm_plan(M, N, K, code, 0, false).splits;  // 1 unless the short split form
+    return;
   }
   resolve_auto(M, N, K, false, tile, splits);
+  if (*tile != 0) return;
+  if (modelled_shape(4, M, N, K, group, false, gate, false) && models_plans() &&
+      automatic_model(4, M, N, K, group, kTailNorm, gate, 0, tile, splits)) {
+    const GemmPlan p = gemm_plan(M, N, K, *tile, *splits, false);
+    if ((p.splits == 1 && !lds_split_code(*tile)) ||
+        (size_t)p.splits * M * N * sizeof(float) <= AOTO_HIP_NOALLOC_SCRATCH_BYTES)
+      return;
+  }
+  // The 16x16 plan by name: the workspace query for automatic codes covers every plan they may lead to, which
+  // is more than this one needs and may be more than the scratch holds.
+  const GemmPlan fixed = gemm_plan(M, N, K, 0, 0, false);
+  *tile = 10 * fixed.tn + fixed.tm;
+  *splits = fixed.splits;
 }
 
 namespace {

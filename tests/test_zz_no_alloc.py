@@ -181,3 +181,25 @@ def test_noalloc_gemm_fits_automatic_plans_to_its_scratch():
         assert torch.cuda.mem_get_info()[0] == free_before
         assert status == 0, _last_error()
         assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (m, n, k, explicit)
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 16400, 896), (256, 8192, 896), (128, 8192, 512), (64, 4864, 896)])
+def test_noalloc_gemm_runs_wide_outputs_of_short_prompts_like_the_workspace_entry_point(m, n, k):
+    """N > K at up to 256 rows: the 16x16 kernel's own plan, unsplit in the first three, whatever the queried workspace of
+    automatic codes would be (16400 outputs at 256 rows: one copy of f32 partials alone is past the scratch) - the
+    same launches and bits as the workspace entry point."""
+
+    from aotolith_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n)
+    packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda") * 0.02).bfloat16(), 64, 4)
+    x = torch.randn(m, k, generator=gen, device="cuda").bfloat16()
+    got = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    with ops.recording_launches() as take:
+        take()
+        want = ops.w4_matmul(x, packed, scales, 64)
+        names = take()
+        status = _noalloc(x, packed, scales, 64, got)
+        assert status == 0, _last_error()
+        assert take() == names
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
