@@ -875,11 +875,11 @@ bool modelled_rope(int M, int K, int head_dim) {
 }
 
 // Most slices of a modelled plan: partials of at most 32 MiB, and 8 (6 for the paired form, whose slices
-// hold two sums). The workspace queries size for it whatever the plan turns out to be.
+// hold two sums); 0 where one slice's are more, which leaves the unsplit forms that store none.
 int modelled_splits(int M, int N, bool paired) {
   const long long fit = (8LL << 20) / ((long long)M * N * (paired ? 2 : 1));
   const int most = paired ? 6 : 8;
-  return fit < 1 ? 1 : fit < most ? (int)fit : most;
+  return fit < most ? (int)fit : most;
 }
 
 float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits, GemmTail tail, int head_dim) {
@@ -902,13 +902,12 @@ float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits
 
 // The modelled instance and split count (explicit codes), or false where the fixed plan (`tile`, `splits`
 // as it resolves, with 1 or more slices) is within 10% of the model's best.
-bool modelled_plan(int bits, int M, int N, int K, int group, GemmTail tail, bool gate, int head_dim, int* tile,
+bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail, bool gate, int head_dim, int* tile,
                    int* splits) {
   const bool paired = tail == kTailPaired;
   const GemmCost* table = paired ? (bits == 4 ? kCostPaired4 : kCostPaired8) : (bits == 4 ? kCost4 : kCost8);
   const int count = (int)(paired ? (bits == 4 ? sizeof(kCostPaired4) : sizeof(kCostPaired8))
                                  : (bits == 4 ? sizeof(kCost4) : sizeof(kCost8))) / (int)sizeof(GemmCost);
-  const bool pow2_even = (group & (group - 1)) == 0 && group >= 32 && (K / group) % 2 == 0;
   const bool small_offsets = (long long)M * K * 2 < (1LL << 31) && (long long)N * K / 8 * bits < (1LL << 31);
   const GemmPlan fixed = gemm_plan(M, N, K, *tile, *splits, paired);
   float best = 0.f, now = 0.f;
@@ -921,7 +920,8 @@ bool modelled_plan(int bits, int M, int N, int K, int group, GemmTail tail, bool
     if (lds_code(c.code) && (!pow2_even || !small_offsets || gate)) continue;
     const int steps = K / (lds_code(c.code) ? 64 : 128);
     for (int s : slices) {
-      if (s > most || (s > 1 && (2 * s > steps || (lds_code(c.code) && !lds_split_code(c.code))))) break;
+      if (s > most && (s > 1 || lds_split_code(c.code))) break;
+      if ( (s > 1 && (2 * s > steps || (lds_code(c.code) && !lds_split_code(c.code))))) break;
       const float t = modelled_cost(c, bits, M, N, K, s, tail, head_dim);
       if (best_tile == 0 || t < best) {
         best = t;
@@ -936,7 +936,12 @@ bool modelled_plan(int bits, int M, int N, int K, int group, GemmTail tail, bool
   return true;
 }
 
-// modelled_plan, remembered per thread: a prefill asks for the same few shapes at every layer.
+// modelled_plan, remembered per thread: a prefill asks for the same few shapes at every layer. Of the group only
+// this matters to it:
+bool pow2_even_groups(int K, int group) {
+  return (group & (group - 1)) == 0 && group >= 32 && (K / group) % 2 == 0;
+}
+
 bool automatic_model(int bits, int M, int N, int K, int group, GemmTail tail, bool gate, int head_dim, int* tile,
                      int* splits) {
   struct Entry {
@@ -944,21 +949,57 @@ bool automatic_model(int bits, int M, int N, int K, int group, GemmTail tail, bo
     int tile, splits;
     bool chosen, valid;
   };
-  thread_local Entry memo[64];
-  const long long a = ((long long)M << 32) | (unsigned)N, b = ((long long)K << 32) | ((long long)(unsigned)group << 8) |
-                                                             (bits == 8) | (gate ? 2 : 0) | (tail << 2) |
-                                                             (head_dim == 128 ? 16 : 0) | (head_dim == 64 ? 32 : 0);
+  thread_local Entry memo[256];
+  const bool pow2_even = pow2_even_groups(K, group);
+  const long long a = ((long long)M << 32) | (unsigned)N;
+  const long long b = ((long long)K << 32) | (bits == 8) | (gate ? 2 : 0) | (tail << 2) | (head_dim == 128 ? 16 : 0) |
+                      (head_dim == 64 ? 32 : 0) | (pow2_even ? 64 : 0);
   const bool known_head = tail != kTailRope || head_dim == 64 || head_dim == 128;
-  Entry& e = memo[((unsigned long long)(a * 0x9E3779B97F4A7C15ull ^ b * 0xC2B2AE3D27D4EB4Full)) >> 58];
+  Entry& e = memo[((unsigned long long)(a * 0x9E3779B97F4A7C15ull ^ b * 0xC2B2AE3D27D4EB4Full)) >> 56];
   if (known_head && e.valid && e.key[0] == a && e.key[1] == b) {
     if (e.chosen) *tile = e.tile, *splits = e.splits;
     return e.chosen;
   }
   int t = *tile, s = *splits;
-  const bool chosen = modelled_plan(bits, M, N, K, group, tail, gate, head_dim, &t, &s);
+  const bool chosen = modelled_plan(bits, M, N, K, pow2_even, tail, gate, head_dim, &t, &s);
   if (known_head) e = {{a, b}, t, s, chosen, true};
   if (chosen) *tile = t, *splits = s;
   return chosen;
+}
+
+// The q/k/v projection's plan: the requested tile and split count, or with 0 the
+// unsplit plan when its blocks' columns are whole heads (the RoPE epilogue: one
+// launch, measured on MI355X at M = 128 / 512 / 2048: 9.9 / 61.5 / 142.6 us against
+// 9.8 / 63.6 / 148.7 for the auto split and its RoPE reduce), on 32-row blocks up to
+// 128 rows (twice the blocks; each wave's dequant per step is the same: 7.5 against
+// 9.3 us on 64-row blocks for Qwen2-0.5B at 128 rows), else the auto split.
+void qkv_rope_plan(int M, int N, int K, int head_dim, int* tile, int* splits) {
+  if (*splits != 0 || head_dim <= 0 || wide_code(*tile) || lds_code(*tile)) return;
+  const int t = *tile == 0 && M <= 128 && 64 % head_dim == 0 ? 12 : *tile;
+  const GemmPlan p = gemm_plan(M, N, K, t, 1, false);
+  const int bn = 64 * p.tn;
+  if (bn % head_dim == 0 && N % bn == 0) {
+    *tile = t;
+    *splits = 1;
+  }
+}
+
+// Partials of the largest plan the model leads these shapes to, over what the workspace queries are not told:
+// the code width, whether the groups are an even power of two, a gate epilogue.
+size_t modelled_workspace(int M, int N, int K, GemmTail tail, int head_dim) {
+  size_t most = 0;
+  for (int which = 0; which < (tail == kTailNorm ? 8 : 4); ++which) {
+    const int bits = which & 1 ? 8 : 4, group = which & 2 ? K : 32;
+    const bool gate = (which & 4) != 0, paired = tail == kTailPaired;
+    if (!modelled_shape(bits, M, N, K, group, paired, gate, tail == kTailRope)) continue;
+    int tile = 0, splits = 0;
+    if (tail == kTailRope) qkv_rope_plan(M, N, K, head_dim, &tile, &splits);
+    if (!automatic_model(bits, M, N, K, group, tail, gate, head_dim, &tile, &splits)) continue;
+    const GemmPlan p = gemm_plan(M, N, K, tile, splits, paired);
+    const size_t bytes = (size_t)p.splits * M * N * sizeof(float) * (paired ? 2 : 1);
+    if ((p.splits > 1 || lds_split_code(tile)) && bytes > most) most = bytes;
+  }
+  return most;
 }
 
 // Plans of a code object that an earlier build stored stay that build's.
@@ -1011,27 +1052,6 @@ extern "C++" void aoto::resolve_gemm_codes(int M, int N, int K, int group, bool 
   *splits = fixed.splits;
 }
 
-namespace {
-
-// The q/k/v projection's plan: the requested tile and split count, or with 0 the
-// unsplit plan when its blocks' columns are whole heads (the RoPE epilogue: one
-// launch, measured on MI355X at M = 128 / 512 / 2048: 9.9 / 61.5 / 142.6 us against
-// 9.8 / 63.6 / 148.7 for the auto split and its RoPE reduce), on 32-row blocks up to
-// 128 rows (twice the blocks; each wave's dequant per step is the same: 7.5 against
-// 9.3 us on 64-row blocks for Qwen2-0.5B at 128 rows), else the auto split.
-void qkv_rope_plan(int M, int N, int K, int head_dim, int* tile, int* splits) {
-  if (*splits != 0 || head_dim <= 0 || wide_code(*tile) || lds_code(*tile)) return;
-  const int t = *tile == 0 && M <= 128 && 64 % head_dim == 0 ? 12 : *tile;
-  const GemmPlan p = gemm_plan(M, N, K, t, 1, false);
-  const int bn = 64 * p.tn;
-  if (bn % head_dim == 0 && N % bn == 0) {
-    *tile = t;
-    *splits = 1;
-  }
-}
-
-}  // namespace
-
 size_t aoto_hip_w4_gemm_workspace(int M, int N, int K, int tile, int splits) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64) return 0;
   // automatic codes: enough for the short prompts' split dequant-once plan too, which
@@ -1045,9 +1065,8 @@ size_t aoto_hip_w4_gemm_workspace(int M, int N, int K, int tile, int splits) {
     const size_t lds_bytes = (size_t)gemm_plan(M, N, K, short_split, 0, false).splits * M * N * sizeof(float);
     if (lds_bytes > bytes) bytes = lds_bytes;
   }
-  if (automatic && !wide_auto_rows(M, K)) {
-    // a modelled plan, whichever the code width, group and epilogue lead to
-    const size_t most = (size_t)modelled_splits(M, N, false) * M * N * sizeof(float);
+  if (automatic) {
+    const size_t most = modelled_workspace(M, N, K, kTailNorm, 0);
     if (most > bytes) bytes = most;
   }
   return bytes;
@@ -1055,12 +1074,11 @@ size_t aoto_hip_w4_gemm_workspace(int M, int N, int K, int tile, int splits) {
 
 size_t aoto_hip_w4_gemm_gate_up_workspace(int M, int N, int K, int tile, int splits) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64) return 0;
-  const bool modelled = tile == 0 && splits == 0 && !wide_auto_rows(M, K);
+  const size_t most = tile == 0 && splits == 0 ? modelled_workspace(M, N, K, kTailPaired, 0) : 0;
   resolve_auto(M, N, K, true, &tile, &splits);
   const GemmPlan p = gemm_plan(M, N, K, tile, splits, true);
-  int most = p.splits;
-  if (modelled && modelled_splits(M, N, true) > most) most = modelled_splits(M, N, true);
-  return most > 1 ? 2 * (size_t)most * M * N * sizeof(float) : 0;
+  const size_t bytes = p.splits > 1 ? 2 * (size_t)p.splits * M * N * sizeof(float) : 0;
+  return most > bytes ? most : bytes;
 }
 
 size_t aoto_hip_w4_gemm_qkv_rope_workspace(int M, int K, int tile, int splits, int query_heads, int kv_heads,
@@ -1070,8 +1088,7 @@ size_t aoto_hip_w4_gemm_qkv_rope_workspace(int M, int K, int tile, int splits, i
   const bool modelled = tile == 0 && splits == 0 && modelled_rope(M, K, head_dim);
   if (!wide_auto_rows(M, K)) qkv_rope_plan(M, N, K, head_dim, &tile, &splits);
   const size_t bytes = aoto_hip_w4_gemm_workspace(M, N, K, tile, splits);
-  const size_t most = modelled && M > 0 && K > 0 && K % 64 == 0
-                          ? (size_t)modelled_splits(M, N, false) * M * N * sizeof(float) : 0;
+  const size_t most = modelled && M > 0 && K > 0 && K % 64 == 0 ? modelled_workspace(M, N, K, kTailRope, head_dim) : 0;
   return most > bytes ? most : bytes;
 }
 

@@ -195,3 +195,35 @@ def test_tiles_that_read_scale_pairs_refuse_scales_at_an_odd_element():
         for gate, up in ((at + 2, at), (at, at + 2)):
             status = lib.aoto_hip_w4_gemm_gate_up(at, at, gate, at, up, at, 256, 1024, 1024, 64, tile, 1, at, None)
             assert status == _lib.AOTO_ERR_ARGUMENT and "4-byte aligned" in _lib.last_error(), tile
+
+
+def test_modelled_workspaces_are_what_a_plan_takes_and_at_most_32_mib():
+    """The cost model's share of the automatic workspace queries: whole f32 copies of a plan it leads to, never past
+    32 MiB, and nothing for shapes it leaves alone (more than 8M outputs in one copy, or N > K up to 256 rows) -
+    beyond what the 16x16 kernel's own plan takes (from 129 rows that of tile 28) and the short prompts' split form."""
+
+    from aotolith_amd import _lib, ops
+
+    lib = _lib.library()
+    for m, n, k in ((1024, 151936, 896), (2048, 4864, 896), (256, 151936, 896), (256, 8192, 896), (129, 16384, 640)):
+        assert ops.gemm_workspace_bytes(m, n, k) == 0, (m, n, k)
+        assert ops.gate_up_workspace_bytes(m, n, k) == 0, (m, n, k)
+    modelled = 0
+    for m in (129, 200, 256, 300, 333, 511, 700, 1030, 1900):
+        for n in (128, 896, 1152, 2560, 4096, 6144, 11008, 14336, 28672, 151936):
+            for k in (448, 896, 1088, 2048, 4096, 4864, 14336):
+                fixed = max(ops.gemm_workspace_bytes(m, n, k, 28, 0), ops.gemm_workspace_bytes(m, n, k, 813, 0),
+                            ops.gemm_workspace_bytes(m, n, k, 814, 0)) if m <= 256 else \
+                    ops.gemm_workspace_bytes(m, n, k, 28, 0)
+                if ops.wide_plan(m, n, k) is not None:
+                    continue
+                need = ops.gemm_workspace_bytes(m, n, k)
+                assert need % (m * n * 4) == 0 and need <= max(fixed, 32 << 20), (m, n, k, need)
+                modelled += need > fixed
+                pair = ops.gate_up_workspace_bytes(m, n, k)
+                fixed = ops.gate_up_workspace_bytes(m, n, k, 18, 0)
+                assert pair % (2 * m * n * 4) == 0 and pair <= max(fixed, 32 << 20), (m, n, k, pair)
+                rope = lib.aoto_hip_w4_gemm_qkv_rope_workspace(m, k, 0, 0, n // 64 - 2, 1, 64) if n >= 192 else 0
+                fixed = ops.gemm_workspace_bytes(m, n, k, 28, 0)
+                assert rope % (m * n // 64 * 64 * 4) == 0 and rope <= max(fixed, 32 << 20, need), (m, n, k, rope)
+    assert modelled > 20  # (the model does add plans that need one)
