@@ -984,6 +984,14 @@ void qkv_rope_plan(int M, int N, int K, int head_dim, int* tile, int* splits) {
   }
 }
 
+bool stores_partials(int M, int N, int K, int tile, int splits, bool paired) {
+  return lds_split_code(tile) || gemm_plan(M, N, K, tile, splits, paired).splits > 1;
+}
+
+// A caller without a workspace (a model's choice may store partials where the fixed plan stores none) keeps the
+// fixed plan.
+bool usable_workspace(const void* workspace) { return workspace != nullptr && aligned16(workspace); }
+
 // Partials of the largest plan the model leads these shapes to, over what the workspace queries are not told:
 // the code width, whether the groups are an even power of two, a gate epilogue.
 size_t modelled_workspace(int M, int N, int K, GemmTail tail, int head_dim) {
@@ -997,7 +1005,7 @@ size_t modelled_workspace(int M, int N, int K, GemmTail tail, int head_dim) {
     if (!automatic_model(bits, M, N, K, group, tail, gate, head_dim, &tile, &splits)) continue;
     const GemmPlan p = gemm_plan(M, N, K, tile, splits, paired);
     const size_t bytes = (size_t)p.splits * M * N * sizeof(float) * (paired ? 2 : 1);
-    if ((p.splits > 1 || lds_split_code(tile)) && bytes > most) most = bytes;
+    if (stores_partials(M, N, K, tile, splits, paired) && bytes > most) most = bytes;
   }
   return most;
 }
@@ -1170,9 +1178,12 @@ int packed_gemm(int bits, const void* x, const int32_t* words, const void* scale
   if (tile == 0 && splits == 0) {
     if (const int code = lds_auto(bits, M, N, K, group, paired, gate != nullptr, rope != nullptr))
       tile = code;
-    else if (rope == nullptr && modelled_shape(bits, M, N, K, group, paired, gate != nullptr, false) && models_plans())
-      automatic_model(bits, M, N, K, group, paired ? kTailPaired : kTailNorm, gate != nullptr, 0,
-                      &tile, &splits);
+    else if (rope == nullptr && modelled_shape(bits, M, N, K, group, paired, gate != nullptr, false) && models_plans()) {
+      int t = 0, s = 0;
+      if (automatic_model(bits, M, N, K, group, paired ? kTailPaired : kTailNorm, gate != nullptr, 0, &t, &s) &&
+          (usable_workspace(workspace) || !stores_partials(M, N, K, t, s, paired)))
+        tile = t, splits = s;
+    }
   }
   resolve_auto(M, N, K, paired, &tile, &splits);
   if (bits == 8 && tile == 243) tile = 441;  // no 8-bit 243 instance; the same (unsplit) grid class
@@ -1290,8 +1301,12 @@ int qkv_rope_gemm(int bits, const void* x, const int32_t* words, const void* sca
     const bool automatic = tile == 0 && splits == 0;
     qkv_rope_plan(M, N, K, head_dim, &tile, &splits);
     if (automatic && group > 0 && aligned4(scales) && modelled_rope(M, K, head_dim) &&
-        modelled_shape(bits, M, N, K, group, false, false, true) && models_plans())
-      automatic_model(bits, M, N, K, group, kTailRope, false, head_dim, &tile, &splits);
+        modelled_shape(bits, M, N, K, group, false, false, true) && models_plans()) {
+      int t = tile, s = splits;
+      if (automatic_model(bits, M, N, K, group, kTailRope, false, head_dim, &t, &s) &&
+          (usable_workspace(workspace) || !stores_partials(M, N, K, t, s, false)))
+        tile = t, splits = s;
+    }
   }
   return packed_gemm(bits, x, words, scales, bias, nullptr, nullptr, y, M, N, K, group, tile, splits, workspace,
                      stream, nullptr, nullptr, nullptr, 0.f, nullptr, &rope);

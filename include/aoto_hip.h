@@ -149,7 +149,7 @@ int aoto_hip_w4_gemv(const void* x, const int32_t* words, const void* scales,
  * measured times where it promises 10% less than the 16x16 kernel (not for a paired gate/up or
  * N > K at M <= 256, nor q/k/v on 32-row blocks), else the 16x16 kernel. The workspace queries
  * cover that choice for either code width and every group (at most 8 slices, 6 paired, and
- * 32 MiB). splits: 0 chooses (small
+ * 32 MiB); without a workspace the model's split plans are left out. splits: 0 chooses (small
  * grids split the reduction), else the split-K count; a split launch stores f32
  * partial tiles in `workspace` (aoto_hip_w4_gemm_workspace() bytes, 16-byte
  * aligned) and a second launch sums them and applies the epilogue. Every plan is

@@ -574,3 +574,44 @@ def test_automatic_codes_at_wide_outputs_of_few_rows(m, n, k, bits):
     matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
     assert torch.equal(matmul(x, packed, scales, 64, bias=bias),
                        matmul(x, packed, scales, 64, bias=bias, tile=14, splits=1))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(257, 11008, 448), (257, 11008, 4096), (1030, 6144, 896)])
+def test_automatic_codes_run_without_a_workspace_where_the_fixed_plan_needs_none(m, n, k, bits):
+    """A model's plan may store partials where the 16x16 plan (tile 28, unsplit) stores none: a caller without a
+    workspace gets the latter, bit for bit, single and q/k/v projections alike."""
+
+    from aotolith_amd import _lib, ops
+
+    lib = _lib.library()
+    assert ops.gemm_workspace_bytes(m, n, k, 28, 0) == 0 < ops.gemm_workspace_bytes(m, n, k)
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda") * 0.02).bfloat16(), 64, bits)
+    x = torch.randn(m, k, generator=gen, device="cuda").bfloat16()
+    bias = torch.randn(n, generator=gen, device="cuda").bfloat16()
+    matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
+    want = matmul(x, packed, scales, 64, bias=bias, tile=28, splits=1)
+    got = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    entry = lib.aoto_hip_w4_gemm if bits == 4 else lib.aoto_hip_w8_gemm
+    _lib.check(entry(ops._ptr(x), ops._ptr(packed), ops._ptr(scales), ops._ptr(bias), None, None, ops._ptr(got), m, n, k,
+                     64, 0, 0, None, ops._stream()))
+    assert torch.equal(got, want)
+    entry = lib.aoto_hip_w4_gemm_gate_up if bits == 4 else lib.aoto_hip_w8_gemm_gate_up
+    pair = (ops._ptr(packed), ops._ptr(scales))
+    _lib.check(entry(ops._ptr(x), *pair, *pair, ops._ptr(got), m, n, k, 64, 0, 0, None, ops._stream()))
+    gate_up = ops.w4_matmul_gate_up if bits == 4 else ops.w8_matmul_gate_up
+    assert ops.gate_up_workspace_bytes(m, n, k) == 0  # (the pair's plan needs none here: the same with and without)
+    assert torch.equal(got, gate_up(x, packed, scales, packed, scales, 64))
+    heads = n // 64 - 2
+    cos, sin = torch.randn(2, m, 64, generator=gen, device="cuda").bfloat16()
+    positions, results = torch.arange(m, device="cuda"), []
+    entry = lib.aoto_hip_w4_gemm_qkv_rope if bits == 4 else lib.aoto_hip_w8_gemm_qkv_rope
+    for tile, splits in ((0, 0), (28, 1)):
+        y, q = torch.empty_like(got), torch.empty(1, heads, m, 64, dtype=torch.bfloat16, device="cuda")
+        cache = torch.zeros(2, 1, 1, m, 64, dtype=torch.bfloat16, device="cuda")
+        _lib.check(entry(ops._ptr(x), ops._ptr(packed), ops._ptr(scales), ops._ptr(bias), ops._ptr(y), m, k, 64, tile,
+                         splits, None, ops._ptr(positions), ops._ptr(cos), ops._ptr(sin), ops._ptr(q), ops._ptr(cache),
+                         heads, 1, 64, m, 0, 1, ops._stream()))
+        results.append((q, cache))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
