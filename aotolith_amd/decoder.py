@@ -1202,24 +1202,31 @@ class DecoderStaticCacheRuntime:
 
         if valid_length < 1 or valid_length >= self.cache_capacity:
             raise PlanInputError(f"valid_length must be in [1, {self.cache_capacity}), got {valid_length}")
-        token = _as_ids(token, self.engine.device).reshape(-1)[:1]
+        device = self.engine.device
+        if verify_token and not (isinstance(token, torch.Tensor) and token.is_cuda):
+            token = _as_ids(token, "cpu").reshape(-1)[:1]  # a host id is known before anything is launched
+            self._check_token(int(token.item()))
+            verify_token = False
+        token = _as_ids(token, device).reshape(-1)[:1]
         if not verify_token:
             return self.decode(token, cache, valid_length)
-        # The token is read back while the step is being launched (an id outside the table embeds as zeros,
+        # A device id is read back while the step is being launched (an id outside the table embeds as zeros,
         # so the launches are safe before it is known): the copy waits for whatever made the token, and
         # waiting for that first would leave the GPU idle until the step's first launch.
         host = torch.empty((1,), dtype=torch.int64, pin_memory=True)
         host.copy_(token, non_blocking=True)
         arrived = torch.cuda.Event()
-        arrived.record()
+        arrived.record(torch.cuda.current_stream(token.device))
         result = self.decode(token, cache, valid_length)
         arrived.synchronize()
-        value = int(host.item())
+        self._check_token(int(host.item()))
+        return result
+
+    def _check_token(self, value: int) -> None:
         if not 0 <= value < self.spec.vocab:
             from .errors import IndexBoundsError
 
             raise IndexBoundsError(f"token {value} is outside the vocabulary [0, {self.spec.vocab})")
-        return result
 
     def greedy_generate(self, input_ids, *, max_new_tokens: int | None = None, sync_each_step: bool = False,
                         use_graph: bool = True, events: dict | None = None) -> torch.Tensor:

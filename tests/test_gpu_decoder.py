@@ -260,6 +260,34 @@ def test_runtime_rejects_bad_inputs():
         runtime.greedy_generate(np.zeros(PROMPT, dtype=np.int64), max_new_tokens=NEW + 1)
 
 
+@pytest.mark.parametrize("where", ["list", "numpy", "cpu", "cuda"])
+def test_decode_token_refuses_ids_outside_the_vocabulary(where):
+    """A bad id is refused - on the host before anything is launched, on the device with the step's launches on their
+    way - with the caller's cache untouched and the next step's results those of a step without the bad call."""
+
+    from aotolith_amd import ops
+    from aotolith_amd.errors import IndexBoundsError
+
+    runtime, _ = _pair(seed=24)
+    make = {"list": lambda v: [[v]], "numpy": lambda v: np.array([v], dtype=np.int32),
+            "cpu": lambda v: torch.tensor([[v]]), "cuda": lambda v: torch.tensor([[v]], device="cuda")}[where]
+    logits, compact = runtime.prefill_ids(np.arange(PROMPT, dtype=np.int64))
+    cache = runtime.pad_cache(compact)
+    kept = cache.clone()
+    want_logits, want_cache = runtime.decode_token(make(3), cache, PROMPT + 1)
+    for value in (-1, TINY.vocab, 1 << 40) if where != "numpy" else (-1, TINY.vocab):
+        with ops.recording_launches() as take:
+            take()
+            with pytest.raises(IndexBoundsError, match=str(value)):
+                runtime.decode_token(make(value), cache, PROMPT + 1)
+            assert bool(take()) == (where == "cuda")
+        assert torch.equal(cache.view(torch.int16), kept.view(torch.int16))
+        got_logits, got_cache = runtime.decode_token(make(3), cache, PROMPT + 1)
+        assert torch.equal(got_logits, want_logits)
+        assert torch.equal(got_cache.view(torch.int16), want_cache.view(torch.int16))
+    runtime.decode_token(make(TINY.vocab - 1), cache, PROMPT + 1)
+
+
 # hidden 896: the shapes whose q/k/v GEMV takes the argmax finish in its prologue
 NARROW = DecoderShape(vocab=4096, hidden=896, intermediate=1024, layers=2, heads=14, kv_heads=2, head_dim=64,
                       eps=1e-6, theta=1e6)
