@@ -728,6 +728,23 @@ def save_graph_plan(compiled, path: str | os.PathLike[str]) -> Path:
                           graph=encode_graph(graph))
 
 
+#: Symbols that an earlier build recorded for whole families of kernels of its code object.
+_FAMILY_RECORDS = frozenset({"aoto_generic_gemm_*", "aoto_generic_attention*", "aoto_generic_{fused,elementwise}",
+                             "aoto_generic_{copy,copy_rows*,fused}"})
+
+
+def _same_graph_selections(rebuilt: list[dict[str, Any]], stored: list[dict[str, Any]]) -> bool:
+    """Whether a graph's rebuilt records are the stored ones; where a stored record names a family, or a chain that
+    the rebuilt plan runs node by node, all but the symbol and its reason."""
+
+    def same(new: dict[str, Any], old: dict[str, Any]) -> bool:
+        if old.get("artifact_name") in _FAMILY_RECORDS or old.get("artifact_name") == "aoto_generic_fused":
+            new, old = ({k: v for k, v in d.items() if k not in ("artifact_name", "reason")} for d in (new, old))
+        return new == old
+
+    return len(rebuilt) == len(stored) and all(same(new, old) for new, old in zip(rebuilt, stored))
+
+
 def _load_graph(contents: ArtifactContents, device):
     from .compiler import CompilationResult, CompiledModulePlan
     from .graph_ops import build_graph_plan
@@ -741,7 +758,7 @@ def _load_graph(contents: ArtifactContents, device):
     plan._keepalive = runner
     rebuilt = [_encode_selection(s) for s in plan.selections]
     stored = [_encode_selection(s) for s in contents.selections]
-    if rebuilt != stored:
+    if not _same_graph_selections(rebuilt, stored):
         raise ArtifactCompatibilityError("the rebuilt graph plan selects different kernels than the artifact records",
                                          hint="the artifact was written by another version of this package")
     result = CompilationResult(plan=plan, input_graph=graph, lowered_graph=graph)

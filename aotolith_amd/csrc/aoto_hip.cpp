@@ -138,12 +138,14 @@ bool has_kernel(const char* name) {
 }
 
 // Kernel symbols launched by this thread while recording is on (aoto_hip_trace_launches),
-// newline-separated, for plans that name the kernels they run.
-thread_local bool g_trace = false;
+// newline-separated, for plans that name the kernels they run; with kTraceOnly they are recorded and not
+// launched, for plans that settle which kernels they run before they have any data.
+constexpr int kTraceOff = 0, kTraceOnly = 2;
+thread_local int g_trace = kTraceOff;
 thread_local std::string g_trace_names;
 
 void trace_launch(const char* name) {
-  if (g_trace) {
+  if (g_trace != kTraceOff) {
     g_trace_names += name;
     g_trace_names += '\n';
   }
@@ -153,6 +155,10 @@ template <typename... Args>
 int launch(const char* name, dim3 grid, dim3 block, unsigned shared, void* stream, Args... args) {
   hipFunction_t fn = nullptr;
   if (int s = lookup(name, &fn)) return s;
+  if (g_trace == kTraceOnly) {
+    trace_launch(name);
+    return AOTO_OK;
+  }
   void* params[] = {static_cast<void*>(&args)...};
   hipError_t err = hipModuleLaunchKernel(fn, grid.x, grid.y, grid.z, block.x, block.y, block.z, shared,
                                          static_cast<hipStream_t>(stream), params, nullptr);
@@ -395,9 +401,9 @@ extern "C" {
 int aoto_hip_abi_version(void) { return AOTO_HIP_ABI_VERSION; }
 
 int aoto_hip_trace_launches(int enable) {
-  const int previous = g_trace ? 1 : 0;
-  g_trace = enable != 0;
-  if (g_trace && !previous) g_trace_names.clear();
+  const int previous = g_trace;
+  g_trace = enable == kTraceOnly ? kTraceOnly : enable != 0;
+  if (g_trace != kTraceOff && previous == kTraceOff) g_trace_names.clear();
   return previous;
 }
 

@@ -53,6 +53,7 @@ class AotoTensor(ctypes.Structure):
 #: bounded, so a program with ever new shapes keeps none of them for long.
 _DESCRIPTORS: dict[tuple, AotoTensor] = {}
 _MAX_DESCRIPTORS = 4096
+_NO_STORAGE = 1 << 20
 
 
 def describe(value) -> AotoTensor:
@@ -66,7 +67,9 @@ def describe(value) -> AotoTensor:
                 _DESCRIPTORS.clear()
             known = _DESCRIPTORS[key] = _describe_layout(value)
         d = AotoTensor.from_buffer_copy(known)
-        d.data = value.data_ptr() if value.numel() else 1  # a non-null pointer for empty tensors
+        # (empty tensors and those without storage, which GraphRunner._settle passes, get an address that is not
+        # null and aligned as the allocator's are)
+        d.data = value.data_ptr() or _NO_STORAGE
         return d
     return _describe_layout(value)
 
@@ -257,17 +260,17 @@ FAMILIES[RMS_NORM] = "rms_norm"
 KERNELS = {"elementwise": "aoto_generic_elementwise", "reduction": "aoto_generic_reduce",
            "matmul": "aoto_generic_gemm", "gather": "aoto_generic_index", "copy": "aoto_generic_copy",
            "fill": "aoto_generic_fill", "rms_norm": "aoto_generic_rms_norm", "attention": "aoto_generic_attention"}
-#: Families whose kernel an earlier build's code object does not have: the symbol that tells, and the
-#: names this build's selections record (a family prefix: the instance follows the operands' strides).
-NEWER = {"matmul": ("aoto_generic_gemm_f32_a_t1k1", "aoto_generic_gemm_*",
+#: Families whose kernels an earlier build's code object does not have: the symbol that tells, and the reason
+#: recorded with the instance that the operands' layouts lead to.
+NEWER = {"matmul": ("aoto_generic_gemm_f32_a_t1k1",
                     "strided batched GEMM on the matrix cores, LDS-staged tiles, f32 accumulation"),
-         "attention": ("aoto_generic_attention_f32_d64_a", "aoto_generic_attention*",
+         "attention": ("aoto_generic_attention_f32_d64_a",
                        "legalized scaled-dot-product attention (bool/float mask, causal, GQA) on the matrix cores, "
                        "f32 softmax"),
-         "elementwise": ("aoto_generic_fused", "aoto_generic_{fused,elementwise}",
+         "elementwise": ("aoto_generic_fused",
                          "strided broadcasting elementwise kernel (eight elements a thread where rows allow), f32 "
                          "compute, one rounding to the output type"),
-         "copy": ("aoto_generic_fused", "aoto_generic_{copy,copy_rows*,fused}",
+         "copy": ("aoto_generic_fused",
                   "strided copy with element-type conversion (whole 1- to 16-byte units where rows allow)")}
 REASONS = {
     "elementwise": "strided broadcasting elementwise kernel, f32 compute, one rounding to the output type",
@@ -466,26 +469,78 @@ class GraphRunner:
         chains = (fuse_elementwise(graph) if _lib.library().aoto_hip_has_kernel(b"aoto_generic_fused") else [])
         #: node name -> its chain; a chain runs where its last member stands
         self.chains = {node.name: chain for chain in chains for node in chain.members}
-        self.handlers: list[tuple[Node, Callable]] = []
-        for node in graph.nodes:
-            handler = self._handler(node)
-            chain = self.chains.get(node.name)
-            if chain is None:
-                self.handlers.append((node, handler))
-            elif chain.root is node:
-                self.handlers.append((node, lambda env, node, chain=chain: self._fused(env, chain)))
+        #: node name -> the kernel it launches on contiguous, aligned inputs
+        self.symbols: dict[str, str] = {}
         self.error = None
+        self._settle()
+        self.handlers = self._handlers()
         # only gathers can meet an index out of range: a graph without one has no flag to set or read back
         self.gathers = any(node.op in INDEX_OPS for node in graph.nodes)
         self.state_ptrs = {t.data_ptr() for t in self.state.values() if isinstance(t, torch.Tensor)}
 
+    def _handlers(self) -> list[tuple[Node, Callable]]:
+        handlers: list[tuple[Node, Callable]] = []
+        for node in self.graph.nodes:
+            handler = self._handler(node)
+            chain = self.chains.get(node.name)
+            if chain is None:
+                handlers.append((node, handler))
+            elif chain.root is node:
+                handlers.append((node, lambda env, node, chain=chain: self._fused(env, chain)))
+        return handlers
+
+    def _settle(self) -> None:
+        """Which kernel each node launches, and which chains have whole vectors, before any call.
+
+        One pass over the nodes with inputs and intermediates that have shapes and strides and no storage, through
+        the launchers themselves, which record and launch nothing. A chain whose rows are not whole vectors is
+        dropped here instead of being refused at every call.
+        """
+
+        env: dict = dict(self.state)
+        for name in self.graph.inputs:
+            shape, dtype = self.graph.input_meta[name]
+            env[name] = torch.empty(shape, dtype=dtype, device="meta")
+        device, self.device = self.device, torch.device("meta")
+        self.error = torch.empty((1,), dtype=torch.int32, device="meta")
+
+        def settle(node: Node) -> None:
+            env[node.name] = self._handler(node)(env, node)
+            names = take()
+            if names and not node.is_view:
+                family = KERNELS[FAMILIES[node.op]]
+                self.symbols[node.name] = next((n for n in names if n.startswith(family)), names[0])
+
+        try:
+            with ops.recording_launches(only=True) as take:
+                for node, handler in self._handlers():
+                    chain = self.chains.get(node.name)
+                    take()
+                    if chain is None:
+                        settle(node)
+                        continue
+                    out = self._out(node)
+                    inputs = [_value(env, x) for x in chain.inputs]
+                    if launch_fused(out, inputs, chain.program, chain.alphas, chain.count):
+                        env[node.name] = out
+                        continue
+                    for member in chain.members:
+                        del self.chains[member.name]
+                        settle(member)
+        except Exception:
+            pass  # a node that no kernel takes says so when the plan is called
+        finally:
+            self.device = device
+            self.error = None
+
     # -- selection records --------------------------------------------------------
     def selections(self, device_name: str | None) -> tuple[KernelSelection, ...]:
         out = []
-        kernels, reasons = dict(KERNELS), dict(REASONS)
-        for family, (symbol, name, reason) in NEWER.items():
+        reasons, settled = dict(REASONS), set()
+        for family, (symbol, reason) in NEWER.items():
             if _lib.library().aoto_hip_has_kernel(symbol.encode()):
-                kernels[family], reasons[family] = name, reason
+                reasons[family] = reason
+                settled.add(family)
         for node in self.graph.nodes:
             if node.is_view:
                 continue
@@ -501,7 +556,8 @@ class GraphRunner:
             out.append(KernelSelection(
                 op_index=len(out), op=node.op.split(".")[1] if node.op.startswith("aten.") else node.op,
                 output_id=node.name, implementation="hip_kernel", kind=family, reason=reasons[family],
-                artifact_name=kernels[family], device_name=device_name, device_architecture=ARCHITECTURE,
+                artifact_name=self.symbols.get(node.name, KERNELS[family]) if family in settled else KERNELS[family],
+                device_name=device_name, device_architecture=ARCHITECTURE,
             ))
         return tuple(out)
 

@@ -73,11 +73,14 @@ def take_launches() -> list[str]:
 
 
 @contextlib.contextmanager
-def recording_launches():
-    """Record the kernel symbols this thread launches (read them with :func:`take_launches`)."""
+def recording_launches(*, only: bool = False):
+    """Record the kernel symbols this thread launches (read them with :func:`take_launches`).
+
+    ``only=True`` records what it would launch and launches nothing.
+    """
 
     lib = _lib.library()
-    previous = int(lib.aoto_hip_trace_launches(1))
+    previous = int(lib.aoto_hip_trace_launches(2 if only else 1))
     try:
         yield take_launches
     finally:

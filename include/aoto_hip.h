@@ -43,7 +43,8 @@ int aoto_hip_abi_version(void);
 /* Record the kernel symbols this host thread launches (the counterpart of the
  * reference's KernelSelection.artifact_name, selection.py:19-34, which names the
  * kernel each node emitted): enable != 0 starts recording (clearing the record),
- * 0 stops. Returns the previous state. */
+ * 0 stops; 2 records the symbols that calls of this thread would launch and launches
+ * none of them. Returns the previous state. */
 int aoto_hip_trace_launches(int enable);
 
 /* Copy the recorded symbols, newline-separated, into buf (NUL-terminated) and

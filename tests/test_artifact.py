@@ -206,3 +206,23 @@ def test_not_an_archive_is_refused(tmp_path):
     path.write_bytes(b"not a zip file")
     with pytest.raises(ArtifactCompatibilityError, match="not an aotolith artifact"):
         artifact.read_artifact_manifest(path)
+
+
+def test_graph_records_of_kernel_families_load_by_their_nodes():
+    """An earlier build recorded a family of kernels, or a chain, where records now name the kernel: such records are
+    compared without the symbol and its reason, all others whole."""
+
+    from aotolith_amd.artifact import _same_graph_selections
+
+    def record(index, kind, symbol, reason="r"):
+        return {"op_index": index, "op": "mm", "output_id": f"n{index}", "implementation": "hip_kernel", "kind": kind,
+                "reason": reason, "artifact_name": symbol}
+
+    new = [record(0, "matmul", "aoto_generic_gemm_bf16_v_t1k4"), record(1, "reduction", "aoto_generic_reduce"),
+           record(2, "elementwise", "aoto_generic_elementwise")]
+    family = [record(0, "matmul", "aoto_generic_gemm_*"), new[1], record(2, "elementwise", "aoto_generic_fused", "chain")]
+    assert _same_graph_selections(new, new) and _same_graph_selections(new, family)
+    assert not _same_graph_selections(new, family[:2])
+    assert not _same_graph_selections(new, [dict(family[0], output_id="other")] + family[1:])
+    assert not _same_graph_selections(new, [dict(new[0], artifact_name="aoto_generic_gemm_f32_a_t1k1")] + new[1:])
+    assert not _same_graph_selections(new, [new[0], dict(new[1], reason="other"), new[2]])

@@ -450,7 +450,7 @@ def test_copies_of_whole_numbers_keep_their_bits(dtype):
 @pytest.mark.parametrize("width", [64, 60])
 def test_fused_chains_keep_the_bits_of_their_nodes(width):
     """Chains (gated MLP through f32, rotary mix, broadcast, scalars, a value read twice) against the same nodes run
-    one by one: equal bits, on whole vectors and on rows that have none."""
+    one by one: equal bits, on rows of whole vectors and on rows that are whole vectors only together (60)."""
 
     import aotolith_amd as aoto
     from aotolith_amd.graph_ops import GraphRunner
@@ -481,3 +481,61 @@ def test_fused_chains_keep_the_bits_of_their_nodes(width):
         assert torch.allclose(got.cpu().float(), want, atol=0.06, rtol=0.03)  # a handful of bf16 roundings
     names = {s.artifact_name for s in result.plan.selections}
     assert "aoto_generic_fused" in names
+
+
+def _chained(gate, up, cos, sin, x):
+    act = torch.nn.functional.silu(gate) * up
+    return act, torch.maximum(act - (x * cos + torch.sigmoid(x) * sin), -x)
+
+
+@pytest.mark.parametrize("rows,width,chained", [((3, 50), 64, True), ((3, 50), 60, True), ((3, 50), 63, False),
+                                                ((4,), 63, False), ((5,), 100, False), ((1,), 8, True)])
+def test_chains_without_whole_vectors_are_settled_when_the_plan_is_built(rows, width, chained):
+    """Rows are whole vectors of eight where the dims that every operand walks as one are: such chains run as one
+    launch, the others as their nodes, with no refused call at each run; the records name what is launched, and a plan
+    with chains gives its nodes' bits on strided inputs too."""
+
+    import aotolith_amd as aoto
+    from aotolith_amd import ops
+    from aotolith_amd.graph_ops import GraphRunner
+
+    gen = torch.Generator().manual_seed(width)
+    inputs = [torch.randn(*s, width, generator=gen).to(torch.bfloat16) for s in
+              (rows, rows, rows[-1:], rows[-1:], rows)]
+    result = aoto.compile_callable(_chained, tuple(inputs), target="hip-gfx950")
+    plan = result.plan
+    assert ("aoto_generic_fused" in plan.kernel_names()) == chained
+    runner = GraphRunner(result.lowered_graph, torch.device("cuda", torch.cuda.current_device()))
+    assert bool(runner.chains) == chained
+    plain = GraphRunner(result.lowered_graph, runner.device)
+    plain.chains = {}
+    plain.handlers = plain._handlers()
+    values = [x.cuda() for x in inputs]
+    with ops.recording_launches() as take:
+        take()
+        got = plan(*values)
+        assert set(take()) == set(plan.kernel_names())
+    bound = dict(zip(result.lowered_graph.inputs, values))
+    assert all(torch.equal(a, b) for a, b in zip(got, plain.run(bound)))
+    wide = [torch.empty(*x.shape[:-1], 2 * width, dtype=x.dtype, device="cuda")[..., ::2].copy_(x) for x in values]
+    assert all(torch.equal(a, b) for a, b in zip(plan(*wide), got))
+
+
+@pytest.mark.parametrize("name,fn,make,tol", CASES, ids=[c[0] for c in CASES])
+def test_graph_plans_record_the_symbols_they_launch(name, fn, make, tol):
+    """Every recorded symbol is launched by a call, and a call launches nothing else but the copies that views and
+    transposed operands make and the fill of the gathers' flag."""
+
+    import aotolith_amd as aoto
+    from aotolith_amd import ops
+
+    inputs = make()
+    plan = aoto.compile_callable(fn, inputs, target="hip-gfx950").plan
+    values = [x.cuda() if isinstance(x, torch.Tensor) else x for x in inputs]
+    with ops.recording_launches() as take:
+        take()
+        plan(*values)
+        launched = set(take())
+    recorded = set(plan.kernel_names())
+    assert recorded <= launched, recorded - launched
+    assert all(n.startswith(("aoto_generic_copy", "aoto_generic_fill")) for n in launched - recorded), launched - recorded
