@@ -210,8 +210,12 @@ struct StreamShape {
   int blocks_per_cu = 2;  // persistent 4-wave blocks per CU
   bool block_x = false;   // x staged once per 4-wave block (aoto_w4_gemv_x* instances)
   int rows = 0;           // > 0: the multi-row direct form, rows per lane (aoto_w4_gemv_r* instances)
-  bool newer = false;     // an instance that an earlier build's code object does not have
+  bool newer = false;     // a layout that an earlier build did not choose
 };
+
+// In every code object whose build chose the `newer` layouts. Not the instance itself: earlier code objects hold
+// some of those (32 x 1, 32 x 4, 64 x 3 and 64 x 7) for other shapes, and a stored plan keeps its own kernels.
+const char kNewerLayouts[] = "aoto_w4_gemv_x32x2_n1_p0_b0";
 
 // Rows per lane of the multi-row direct GEMV; AOTO_GEMV_ROWS overrides the
 // shape's default (0 selects the streaming form) where that instance exists.
@@ -581,7 +585,7 @@ int aoto_hip_w4_gemv(const void* x, const int32_t* words, const void* scales, co
     snprintf(sname, sizeof(sname), "aoto_w4_gemv_%c%dx%d_n%d_p%d_b%d", ss.block_x ? 'x' : 's', ss.lpr, ss.cpl,
              norm, paired ? 1 : 0, has_bias);
     unsigned long long* no_keys = nullptr;
-    if (!ss.newer || has_kernel(sname))
+    if (!ss.newer || has_kernel(kNewerLayouts))
       return launch(sname, dim3((unsigned)l.grid), dim3(64 * l.wpb), l.shared, stream, words, scales, x, norm_weight,
                     K, N, l.shift, l.wpb, bias, up_words, up_scales, eps, alpha, beta, y, no_keys);
   }

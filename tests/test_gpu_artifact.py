@@ -154,3 +154,35 @@ def test_strict_device_match_refuses_another_device(tmp_path):
     read_artifact(decode_path)                                # portable load: accepted
     with pytest.raises(ArtifactCompatibilityError, match="device mismatch"):
         read_artifact(decode_path, require_device_match=True)
+
+
+def test_decode_gemvs_over_an_earlier_code_object_keep_its_kernels():
+    """Under a code object without the layouts of this build's rule (their names changed in this one's symbol tables), a
+    reduction without a tuned layout runs on the kernel that the earlier build recorded, also where the instance this
+    build would choose is there for other shapes (32 x 1 at K = 256); tuned layouts are unaffected."""
+
+    from aotolith_amd import _lib, ops
+
+    def names(k, n):
+        packed, scales = ops.quantize(torch.randn(n, k, generator=gen, device="cuda").bfloat16(), 64, 4)
+        x = torch.randn(k, generator=gen, device="cuda").bfloat16()
+        with ops.recording_launches() as take:
+            take()
+            ops.w4_gemv(x, packed, scales, 64)
+            return take()
+
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    image = _lib.default_code_object()
+    marker = b"aoto_w4_gemv_x32x2_n1_p0_b0"
+    assert marker in image
+    tuned = names(896, 1152)
+    assert all(n.startswith("aoto_w4_gemv_x") for k, rows in ((256, 512), (5120, 4096)) for n in names(k, rows))
+    _lib.install_code_object(image.replace(marker, marker[:-1] + b"Z"))
+    try:
+        assert names(896, 1152) == tuned
+        for k, rows in ((256, 512), (5120, 4096), (8192, 1024)):
+            assert all(n.startswith("aoto_w4_gemv_l") for n in names(k, rows)), (k, rows)
+        torch.cuda.synchronize()
+    finally:
+        _lib.install_code_object(image)
+    assert names(256, 512)[0].startswith("aoto_w4_gemv_x32x1")
