@@ -51,6 +51,13 @@ def _expect(tensor: torch.Tensor, name: str, dtype: torch.dtype, shape: tuple[in
         raise ValueError(f"{name} must have shape {tuple(shape)}, got {tuple(tensor.shape)}")
 
 
+def _on_device(workspace: torch.Tensor | None) -> None:
+    """A workspace in host memory is an illegal access for the kernel that stores its partial sums there."""
+
+    if workspace is not None and not workspace.is_cuda:
+        raise ValueError(f"the workspace must be on a GPU, got {workspace.device}")
+
+
 def _ready(tensor: torch.Tensor) -> None:
     _lib.ensure_code_object(tensor.get_device())
 
@@ -314,6 +321,7 @@ def _matmul(
         if out.numel() != m * n:
             raise ValueError(f"out has {out.numel()} elements, expected {m * n}")
     _ready(x)
+    _on_device(workspace)
     need = gemm_workspace_bytes(m, n, k, tile, splits)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty((need // 4,), dtype=torch.float32, device=x.device)
@@ -487,6 +495,7 @@ def _matmul_gate_up(bits, x, gate_packed, gate_scales, up_packed, up_scales, gro
         if out.numel() != m * n:
             raise ValueError(f"out has {out.numel()} elements, expected {m * n}")
     _ready(x)
+    _on_device(workspace)
     need = gate_up_workspace_bytes(m, n, k, tile, splits)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty((need // 4,), dtype=torch.float32, device=x.device)
@@ -557,6 +566,7 @@ def matmul_residual_norm(x, packed, scales, group_size, residual, norm_weight, e
         if t.numel() != m * n:
             raise ValueError(f"{name} has {t.numel()} elements, expected {m * n}")
     _ready(x)
+    _on_device(workspace)
     need = gemm_workspace_bytes(m, n, k, tile, splits)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty((need // 4,), dtype=torch.float32, device=x.device)
@@ -722,6 +732,7 @@ def matmul_qkv_rope(
         _expect(q_out, "q_out", BF16, (1, query_heads, m, head_dim))
     _ready(x)
     lib = _lib.library()
+    _on_device(workspace)
     need = int(lib.aoto_hip_w4_gemm_qkv_rope_workspace(m, k, int(tile), int(splits), query_heads, kv_heads, head_dim))
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty((need // 4,), dtype=torch.float32, device=x.device)
@@ -784,7 +795,8 @@ def rope_kv_cache_append(
 
 def decode_attention_workspace(batch: int, query_heads: int, kv_heads: int, capacity: int, head_dim: int,
                                splits: int = 0, device=None) -> torch.Tensor:
-    """A workspace for the split-K records of :func:`decode_attention` with these shapes."""
+    """A workspace for the split-K records of :func:`decode_attention` with these shapes (on ``device``; a GPU's, and
+    torch's default device is the host unless a program sets it)."""
 
     size = _lib.library().aoto_hip_decode_attention_workspace(batch, query_heads, kv_heads, capacity, head_dim, splits)
     return torch.zeros((max(size, 16),), dtype=torch.uint8, device=device)
@@ -827,6 +839,7 @@ def decode_attention(
         raise ValueError("pass valid=, mask= or step_state=")
     if out is None:
         out = torch.empty_like(q)
+    _on_device(workspace)
     _ready(q)
     _lib.check(
         _lib.library().aoto_hip_decode_attention(
@@ -877,6 +890,7 @@ def decode_rope_attention(
     if rope_rows is not None:
         _expect(rope_rows, "rope_rows", BF16, (2, head_dim))
     keys, values = pair[0], pair[1]
+    _on_device(workspace)
     _ready(row)
     _lib.check(
         _lib.library().aoto_hip_decode_rope_attention(
