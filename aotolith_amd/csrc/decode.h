@@ -363,6 +363,11 @@ __device__ void decode_attention_body(const uint16_t* __restrict__ q, const uint
   }
 }
 
+// The upper halves of two floats (bf16 by truncation), packed.
+AOTO_DEVICE uint32_t upper_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+
 // The same attention with the query heads of a kv head sharing one pass over its window, on the matrix
 // cores, for windows long enough to be split: the one-head form above streams each kv head's keys and values
 // once per query head (four times for 32 query heads over 8) and spends ~1.2 us of VALU per 128 keys and head.
@@ -372,7 +377,9 @@ __device__ void decode_attention_body(const uint16_t* __restrict__ q, const uint
 //                                     order (16 rows of 64 bytes a load), Q rotated in registers
 //   O^T [d x 16 heads] += V^T . P^T   V through the wave's own LDS (transposing reads); the slots of the
 //                                     product hold the keys in S^T's accumulator order for both operands
-// P keeps its f32 precision as three bf16 terms (8 + 8 + 8 bits), three products into one f32 sum. Lane l
+// P keeps its f32 precision as three bf16 terms (8 + 8 + 8 bits), three products into one f32 sum: cut, not
+// rounded, so that none is negative, and at least the smallest normal number where P is not zero, so that an
+// infinite value stays one through all three (2^-126 beside P is nothing to the f32 sum). Lane l
 // owns head l % 16 in both products, so a head's running maximum and sum stay in its four lanes. The next
 // tile's loads are issued as soon as the current registers are free; a block walks its split's tiles, so the
 // split count follows the chip and not the register file, and the merge reads fewer records.
@@ -511,9 +518,16 @@ __device__ __forceinline__ void decode_attention_group_body(
 #pragma unroll
     for (int i = 0; i < VL; ++i) {
       const bool mine = FUSED && s0 + min(key_v(tile, i), last) == slot;
-      const uint4 v = make_uint4(mine ? vc.x : vq[i].x, mine ? vc.y : vq[i].y, mine ? vc.z : vq[i].z,
-                                 mine ? vc.w : vq[i].w);
+      uint4 v = make_uint4(mine ? vc.x : vq[i].x, mine ? vc.y : vq[i].y, mine ? vc.z : vq[i].z,
+                           mine ? vc.w : vq[i].w);
       *reinterpret_cast<uint4*>(vs + (i * 64 + lane) / LPK * STR + (lane % LPK) * 8) = v;
+    }
+    // (the split's last row is read again past its end: its weight is zero there, and so are its values)
+    if ((tile + 1) * TILE > n) {
+#pragma nounroll
+      for (int i = 0; i < VL; ++i)
+        if (key_v(tile, i) >= n)
+          *reinterpret_cast<uint4*>(vs + (i * 64 + lane) / LPK * STR + (lane % LPK) * 8) = make_uint4(0u, 0u, 0u, 0u);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -553,10 +567,12 @@ __device__ __forceinline__ void decode_attention_group_body(
       const float p0 = p[2 * i] == -INFINITY ? 0.f : expf(p[2 * i] - m);
       const float p1 = p[2 * i + 1] == -INFINITY ? 0.f : expf(p[2 * i + 1] - m);
       run_l += p0 + p1;
-      hi[i] = cvt_pk_bf16(p0, p1);
+      hi[i] = upper_halves(p0, p1);
       const float r0 = p0 - bf16_lo(hi[i]), r1 = p1 - bf16_hi(hi[i]);
-      mid[i] = cvt_pk_bf16(r0, r1);
-      lo[i] = cvt_pk_bf16(r0 - bf16_lo(mid[i]), r1 - bf16_hi(mid[i]));
+      const uint32_t m2 = upper_halves(r0, r1), m3 = upper_halves(r0 - bf16_lo(m2), r1 - bf16_hi(m2));
+      const i16x2_t least = __builtin_elementwise_min(__builtin_bit_cast(i16x2_t, hi[i]), i16x2_t{0x80, 0x80});
+      mid[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2_t, m2), least));
+      lo[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2_t, m3), least));
     }
     const uint16_t* v0 = vs + (4 * quad + (col >> 2)) * STR + 4 * (col & 3);
 #pragma unroll

@@ -695,6 +695,48 @@ def test_long_windows_share_a_pass_over_the_kv_head(hq, hkv, dim, cap, valid, ba
     assert bool(((got.double() - other.double()).abs() <= 2.0 ** -7 * want.abs() + 2e-4 * want.abs().amax()).all())
 
 
+@pytest.mark.parametrize("hq,hkv,dim,cap", [(14, 2, 64, 2304), (7, 1, 64, 2051), (32, 8, 128, 4131), (16, 1, 128, 9000)])
+@pytest.mark.parametrize("form", ["ring", "plain", "mask"])
+def test_long_windows_keep_infinite_values(hq, hkv, dim, cap, form):
+    """+inf, -inf and NaN in the values of kept keys reach the outputs of their kv head's queries as one f32 product per
+    key would give them (inf - inf is NaN), in the first and last keys of the window and within, the other columns
+    and heads as without them."""
+
+    ops = _ops()
+    gen = torch.Generator().manual_seed(cap + hq)
+    pair = torch.randn(2, 1, hkv, cap, dim, generator=gen).bfloat16().cuda()
+    row = torch.randn(1, (hq + 2 * hkv) * dim, generator=gen).bfloat16().cuda()
+    _, _, cos, sin = _tables(cap, dim, 1e6)
+    workspace = ops.decode_attention_workspace(1, hq, hkv, cap, dim, device="cuda")
+    slot = cap // 2
+
+    def run(pair):
+        if form == "ring":
+            return ops.decode_rope_attention(row, cos, sin, pair.clone(), query_heads=hq, query_start=0, key_start=hq * dim,
+                                             value_start=(hq + hkv) * dim, position=cap - 1, slot=slot, valid=cap,
+                                             ring_offset=(slot + 1) % cap, workspace=workspace)
+        q = row[:, : hq * dim].view(1, hq, dim).contiguous()
+        kwargs = dict(valid=cap) if form == "plain" else dict(mask=torch.ones(1, cap, dtype=torch.bool, device="cuda"))
+        return ops.decode_attention(q, pair[0], pair[1], workspace=workspace, **kwargs)
+
+    group, top = hq // hkv, hkv - 1
+    want = run(pair).float()
+    wild = pair.clone()
+    for key, column, value in ((0, 3, "inf"), (cap - 1, 5, "-inf"), (cap // 3, dim - 1, "nan"), (cap - 2, 17, "inf"),
+                               (700, 17, "-inf"), (129, 40, "inf"), (cap - 1, 40, "inf")):
+        wild[1, 0, top, key, column] = float(value)
+    got = run(wild).float()
+    mine = torch.zeros(1, hq, dim, dtype=torch.bool, device="cuda")
+    mine[:, group * top:] = True
+    expected = torch.zeros(dim, device="cuda")
+    for column, value in ((3, "inf"), (5, "-inf"), (dim - 1, "nan"), (17, "nan"), (40, "inf")):
+        expected[column] = float(value)
+    special = mine & (expected != 0.0)
+    assert torch.equal(got[special].nan_to_num(nan=7.0), expected.expand_as(got)[special].nan_to_num(nan=7.0))
+    # (the second walk sums the terms in another order: an f32 sum of 9000 keys apart, then a bf16 rounding)
+    assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-5)[~special].all())
+
+
 def test_workspaces_in_host_memory_are_refused():
     """Refused by the wrappers before anything is launched: the kernels would store to a host address."""
 
