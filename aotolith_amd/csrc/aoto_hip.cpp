@@ -2532,8 +2532,13 @@ int aoto_hip_generic_attention(const aoto_tensor* out, const aoto_tensor* q, con
     for (int d = 0; d < 4; ++d) args.ms[d] = o.strides[d];
   }
   args.scale = scale;
-  if (B == 0 || H == 0 || Lq == 0) return AOTO_OK;
-  if (D <= 128 && Dv <= 128 && has_kernel("aoto_generic_attention_f32_d64_a")) {
+  if (B == 0 || H == 0 || Lq == 0 || Dv == 0) return AOTO_OK;
+  // A few keys of small heads are less than the matrix kernel's prologue and combination: up to 4 keys of 16 columns
+  // run one block a row (us, that -> the matrix kernel: 8 heads of 16, one query over 1 / 4 / 8 / 16 keys, bf16 7.1 /
+  // 7.7 / 8.4 / 10.0 -> 8.8, f32 6.7 / 7.2 / 8.0 / 9.6 -> 8.5; 512 rows over 4 / 8 keys 8.0 / 8.8 -> 8.4; heads of 32, one
+  // key 11.2 -> 9.0).
+  const bool few = D <= 16 && Dv <= 16 && Lk <= 4 && B * H * Lq <= 512;
+  if (D <= 128 && Dv <= 128 && !few && has_kernel("aoto_generic_attention_f32_d64_a")) {
     char name[64];
     generic_attention_plan(args, name, sizeof(name));
     return launch(name, dim3((unsigned)((Lq + 31) / 32), (unsigned)(B * H)), dim3(256), 0, stream, args);

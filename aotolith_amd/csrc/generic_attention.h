@@ -15,14 +15,17 @@
 // f32 (and mixed) operands: 32-key tiles on v_mfma_f32_32x32x2_f32, V read in operand order.
 //
 // Values that are not finite: 0 * inf would poison every query through the product, so they enter it as
-// zeros, and a wave that met any goes over its tiles once more (special_values) with the row's final
+// zeros, and a wave that met any goes over its keys once more (special_values) with the row's final
 // maximum and gives +-inf / NaN to the queries whose probability of such a key is not zero. (Within the loop
 // a key's probability is still relative to the maximum so far: one that ends as zero may not be zero yet.)
 // A kept score that is NaN makes its query NaN: it stays in the running sum, which no rescale to zero drops.
 //
 // Bound: latency (two tiles a wave at 512 keys), then the MFMA pipe. 14 heads of 64, 512 tokens,
 // causal, bf16: 881 us with one block per query row and scalar dots (every score a 64-step chain of
-// typed loads) -> 19.7 us.
+// typed loads) -> 14.8 us. The loads of V and of the mask are free of branches on types (one per tile) and edges
+// (clamped, their weights zero): with a branch an element it was 16.9 us, 8 heads of f32 41.1 against 22.6, one query
+// of 8 heads over 64 f32 keys 15.0 against 10.0 - and the masks of those branches and 460 registers made the compiler
+// split live ranges across them, in one form of this source with a copy under the wrong lanes.
 #pragma once
 
 #include "aoto_hip.h"
@@ -42,10 +45,7 @@ AOTO_DEVICE void wave_lds_order() {
   __builtin_amdgcn_wave_barrier();
 }
 
-AOTO_DEVICE bool not_finite_bf16(uint32_t bits16) { return (bits16 & 0x7F80u) == 0x7F80u; }
 AOTO_DEVICE bool not_finite_f32(float v) { return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u; }
-// The class of a value that is not finite: 0 +inf, 1 -inf, 2 NaN.
-AOTO_DEVICE int special_class(float v) { return v != v ? 2 : v < 0.f ? 1 : 0; }
 
 // One 16-byte operand chunk (8 bf16 or 4 f32) at `off` along stride `step`, elements from `count` on zero.
 template <bool F32, bool VEC>
@@ -126,47 +126,47 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
       }
     }
   };
-  // f32 V in operand order: key (e, half) of a tile, column 32 t + col
-  auto value_f32 = [&](int j0, int e, int t) -> float {
-    const int j = j0 + 8 * (e >> 2) + 4 * half + (e & 3), d = 32 * t + col;
-    if (j >= a.lk || d >= a.dv) return 0.f;
-    return load_float(a.v, a.v_dtype, vbase + (long long)j * a.vs[2] + (long long)d * a.vs[3]);
-  };
-
-  f32x16_t o[DT] = {}, p[KT], sc[KT];
-  float run_max = -INFINITY, run_sum = 0.f;
-
-  // sc = K . q of the loaded keys
-  auto products = [&]() {
+  // f32 V in operand order: key (e, half) of a tile, column 32 t + col. One branch on the type and none on the
+  // edges: a branch a load serialized the loads and spilled the scalar registers of their masks.
+  float vf32[F32 ? 16 : 1][F32 ? DT : 1];
+  auto load_values_f32 = [&](int j0) {
+    if constexpr (F32) {
+      auto at = [&](int e, int t) {
+        const int j = min(j0 + 8 * (e >> 2) + 4 * half + (e & 3), a.lk - 1), d = min(32 * t + col, a.dv - 1);
+        return vbase + (long long)j * a.vs[2] + (long long)d * a.vs[3];
+      };
+      if (a.v_dtype == AOTO_DT_F32) {
 #pragma unroll
-    for (int sub = 0; sub < KT; ++sub) {
-      sc[sub] = f32x16_t{};
+        for (int e = 0; e < 16; ++e)
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        if constexpr (F32) {
-          const uint32_t kw[4] = {kf[sub][s].x, kf[sub][s].y, kf[sub][s].z, kf[sub][s].w};
-          const uint32_t qw[4] = {qf[s].x, qf[s].y, qf[s].z, qf[s].w};
+          for (int t = 0; t < DT; ++t) vf32[e][t] = static_cast<const float*>(a.v)[at(e, t)];
+      } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            sc[sub] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kw[e]), __uint_as_float(qw[e]), sc[sub], 0,
-                                                           0, 0);
-        } else {
-          sc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[sub][s]),
-                                                            __builtin_bit_cast(bf16x8_t, qf[s]), sc[sub], 0, 0, 0);
-        }
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+          for (int t = 0; t < DT; ++t) vf32[e][t] = bf16_to_f32(static_cast<const uint16_t*>(a.v)[at(e, t)]);
       }
     }
   };
-  // p = the scaled and masked scores of sc; returns the lane's largest
+
   const long long mrow = b * a.ms[0] + h * a.ms[1] + (long long)qrow * a.ms[2];
-  auto masked_scores = [&](int j0) -> float {
-    float top = -INFINITY;
-#pragma unroll
-    for (int sub = 0; sub < KT; ++sub)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int j = j0 + 32 * sub + 8 * (e >> 2) + 4 * half + (e & 3);
-        bool keep = j < a.lk && !(a.causal && j > qi);
+  f32x16_t o[DT] = {}, p[KT];
+  float run_max = -INFINITY, run_sum = 0.f;
+
+  // +-inf and NaN of the wave's keys, added to its recorded products for the queries whose probability of the key is
+  // not zero. Key by key and column by column: the pass is as rare as such values, and its code is kept short.
+  auto special_values = [&](float* products_record, float top) {
+    const long long qbase = b * a.qs[0] + h * a.qs[1] + qrow * a.qs[2];
+#pragma nounroll
+    for (int tile = wave; tile < tiles; tile += kGenAttnWaves) {
+#pragma nounroll
+      for (int j = tile * BK; j < min(tile * BK + BK, a.lk); ++j) {
+        const long long vrow = vbase + (long long)j * a.vs[2];
+        bool any = false;
+#pragma nounroll
+        for (int d = lane; d < a.dv; d += 64) any = any || not_finite_f32(load_float(a.v, a.v_dtype, vrow + d * a.vs[3]));
+        if (!__any(any)) continue;
+        bool keep = !(a.causal && j > qi);
         float add = 0.f;
         if (a.mask != nullptr && keep) {
           const long long mo = mrow + (long long)j * a.ms[3];
@@ -175,66 +175,20 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
           else
             add = load_float(a.mask, a.mask_dtype, mo);
         }
-        const float v = keep ? sc[sub][e] * a.scale + add : -INFINITY;
-        p[sub][e] = v;
-        top = fmaxf(top, v);
-      }
-    return top;
-  };
-
-  // +-inf and NaN of a tile's values, for the queries whose p of their key is not zero: per class, the
-  // product of the class's indicator with [p != 0], and the special value where it is not zero. The
-  // values are read again (the staged ones are gone); the pass is as rare as such values.
-  auto special_values = [&](int j0) {
-    for (int cls = 0; cls < 3; ++cls) {
-      f32x16_t hits[DT] = {};
-      if constexpr (F32) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float pe = p[0][e] != 0.f ? 1.f : 0.f;
-#pragma unroll
-          for (int t = 0; t < DT; ++t) {
-            const float v = value_f32(j0, e, t);
-            const float ind = not_finite_f32(v) && special_class(v) == cls ? 1.f : 0.f;
-            hits[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(ind, pe, hits[t], 0, 0, 0);
-          }
-        }
-      } else {
-        wave_lds_order();
-        for (int c = lane; c < BK * RC; c += 64) {
-          const int row = c / RC, d0 = (c % RC) * E;
-          const uint4 r = attn_chunk<F32, VEC>(
-              a.v, a.v_dtype, vbase + (long long)min(j0 + row, a.lk - 1) * a.vs[2] + d0 * a.vs[3], a.vs[3], a.dv - d0);
-          const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint32_t bits = (w[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
-            const bool hit = not_finite_bf16(bits) && special_class(bf16_to_f32(bits)) == cls;
-            vs[row * STRV + d0 + i] = hit ? (uint16_t)0x3F80u : (uint16_t)0u;
-          }
-        }
-        wave_lds_order();
-#pragma unroll
-        for (int kt = 0; kt < 2 * KT; ++kt) {
-          uint32_t w[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float p0 = p[kt >> 1][8 * (kt & 1) + 2 * i], p1 = p[kt >> 1][8 * (kt & 1) + 2 * i + 1];
-            w[i] = (p0 != 0.f ? 0x3F80u : 0u) | (p1 != 0.f ? 0x3F800000u : 0u);
-          }
-          const fa_bf16x8 pb = __builtin_bit_cast(fa_bf16x8, w);
-#pragma unroll
-          for (int t = 0; t < DT; ++t)
-            hits[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(flash_v_operand<STRV>(vs, kt, 32 * t, lane), pb, hits[t],
-                                                              0, 0, 0);
+        float dot = 0.f;
+#pragma nounroll
+        for (int d = 0; d < a.d; ++d)
+          dot = fmaf(load_float(a.q, a.q_dtype, qbase + d * a.qs[3]),
+                     load_float(a.k, a.k_dtype, kbase + (long long)j * a.ks[2] + d * a.ks[3]), dot);
+        const float score = keep ? dot * a.scale + add : -INFINITY;
+        if (score == -INFINITY || expf(score - top) == 0.f) continue;
+#pragma nounroll
+        for (int r = 0; r < 16 * DT; ++r) {
+          const int d = 8 * (r >> 2) + 4 * half + (r & 3);
+          const float v = d < a.dv ? load_float(a.v, a.v_dtype, vrow + d * a.vs[3]) : 0.f;
+          if (not_finite_f32(v)) products_record[r * 64 + lane] += v;
         }
       }
-      const float value = cls == 0 ? INFINITY : cls == 1 ? -INFINITY : NAN;
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          if (hits[t][e] > 0.f) o[t][e] += value;
     }
   };
 
@@ -270,12 +224,68 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
       wave_lds_order();
     }
 
-    products();
+    f32x16_t sc[KT];
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub) {
+      sc[sub] = f32x16_t{};
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        if constexpr (F32) {
+          const uint32_t kw[4] = {kf[sub][s].x, kf[sub][s].y, kf[sub][s].z, kf[sub][s].w};
+          const uint32_t qw[4] = {qf[s].x, qf[s].y, qf[s].z, qf[s].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sc[sub] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kw[e]), __uint_as_float(qw[e]), sc[sub], 0,
+                                                           0, 0);
+        } else {
+          sc[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[sub][s]),
+                                                            __builtin_bit_cast(bf16x8_t, qf[s]), sc[sub], 0, 0, 0);
+        }
+      }
+    }
     // the next tile's loads work under this one's softmax and products (the last trip reads its own again)
+    load_values_f32(j0);
     load_keys(next);
     load_values(next);
 
-    const float tile_max = xor32_max(masked_scores(j0));
+    // Scaled and masked, with one branch on the mask's type and none on its edges (the mask of a key past the last
+    // is read at the last).
+    auto key_of = [&](int sub, int e) { return j0 + 32 * sub + 8 * (e >> 2) + 4 * half + (e & 3); };
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) p[sub][e] = sc[sub][e] * a.scale;
+    if (a.mask != nullptr) {
+      auto mask_at = [&](int sub, int e) { return mrow + (long long)min(key_of(sub, e), a.lk - 1) * a.ms[3]; };
+      if (a.mask_dtype == AOTO_DT_BOOL) {
+#pragma unroll
+        for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            p[sub][e] = static_cast<const uint8_t*>(a.mask)[mask_at(sub, e)] != 0 ? p[sub][e] : -INFINITY;
+      } else if (a.mask_dtype == AOTO_DT_F32) {
+#pragma unroll
+        for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) p[sub][e] += static_cast<const float*>(a.mask)[mask_at(sub, e)];
+      } else {
+#pragma unroll
+        for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)
+            p[sub][e] += bf16_to_f32(static_cast<const uint16_t*>(a.mask)[mask_at(sub, e)]);
+      }
+    }
+    float tile_max = -INFINITY;
+    const int keys_end = a.causal ? min(a.lk, qi + 1) : a.lk;
+#pragma unroll
+    for (int sub = 0; sub < KT; ++sub)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        p[sub][e] = key_of(sub, e) < keys_end ? p[sub][e] : -INFINITY;
+        tile_max = fmaxf(tile_max, p[sub][e]);
+      }
+    tile_max = xor32_max(tile_max);
     const float moved = fmaxf(run_max, tile_max);
     // (a maximum of -inf has only zeros, or a NaN score's NaN, behind it: kept as they are)
     const float correction = run_max == moved || run_max == -INFINITY ? 1.f : expf(run_max - moved);
@@ -301,11 +311,10 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
       for (int e = 0; e < 16; ++e)
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-          float v = value_f32(j0, e, t);
-          if (not_finite_f32(v)) {
-            odd = true;
-            v = 0.f;
-          }
+          // (rows past the keys and columns past the head repeat the last: their weight is zero, or they are not stored)
+          const bool special = not_finite_f32(vf32[e][t]);
+          odd = odd || special;
+          const float v = special ? 0.f : vf32[e][t];
           o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, p[0][e], o[t], 0, 0, 0);
         }
     } else {
@@ -331,13 +340,18 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     }
   }
 
-  // The waves' states (the V stages are dead: a wave's records lie in its own): maxima and sums first, whose
-  // sign bit says that the wave has met a value that is not finite.
+  // The waves' states (the V stages are dead: a wave's records lie in its own), combined by all four: wave w
+  // takes every fourth run of 4 output columns. A sum's sign bit says that its wave has met a value that is not
+  // finite.
   const bool special = __any(odd);
   wave_lds_order();
   float* rec = reinterpret_cast<float*>(lds[wave]);
   rec[lane] = run_max;
   rec[64 + lane] = __uint_as_float((__float_as_uint(run_sum) & 0x7FFFFFFFu) | (special ? 0x80000000u : 0u));
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) rec[(2 + 16 * t + e) * 64 + lane] = o[t][e];
   __syncthreads();
   float big = -INFINITY, sum = 0.f, factor[kGenAttnWaves];
   uint32_t any_special = 0u;
@@ -352,28 +366,10 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
     const float l = fabsf(other[64 + col]) + fabsf(other[64 + 32 + col]);
     sum += l * factor[w];
   }
-  if (any_special >> 31) {  // (uniform)
-    __syncthreads();  // the maxima and sums are read: the special pass stages over them
-    if (special) {
-      for (int tile = wave; tile < tiles; tile += kGenAttnWaves) {
-        load_keys(tile * BK);
-        products();
-        masked_scores(tile * BK);
-#pragma unroll
-        for (int sub = 0; sub < KT; ++sub)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) p[sub][e] = p[sub][e] == -INFINITY ? 0.f : expf(p[sub][e] - big);
-        special_values(tile * BK);
-      }
-    }
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(any_special) >> 31, 0)) {  // (uniform)
+    if (special) special_values(rec + 128, big);
+    __syncthreads();
   }
-  // The products' records, combined by all four waves: wave w takes every fourth run of 4 output columns.
-  wave_lds_order();
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) rec[(2 + 16 * t + e) * 64 + lane] = o[t][e];
-  __syncthreads();
   if (qi >= a.lq) return;
   const float inv = sum > 0.f ? 1.0f / sum : 0.f;
   const long long ob = ((long long)(b * a.heads + h) * a.lq + qi) * a.dv;

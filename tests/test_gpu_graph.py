@@ -384,6 +384,32 @@ def test_attention_with_scores_that_are_not_finite(case, d, types):
     assert bool(((got - want).abs() <= 2.0 ** -24 * 1200 * 4)[fine].all())
 
 
+@pytest.mark.parametrize("types", ["bf16", "f32"])
+@pytest.mark.parametrize("heads,lq,lk,d,dv,few", [(4, 4, 4, 16, 16, True), (4, 4, 5, 16, 16, False),
+                                                  (2, 1, 1, 7, 12, True), (2, 3, 17, 16, 16, False),
+                                                  (128, 4, 3, 16, 16, True), (128, 5, 3, 16, 16, False),
+                                                  (1, 2, 3, 17, 16, False), (1, 2, 3, 16, 17, False)])
+def test_attention_over_few_keys_of_small_heads(heads, lq, lk, d, dv, few, types):
+    """Up to 512 rows of 16 columns and 4 keys run on the one-row kernel, all else on the matrix cores: both against
+    64-bit attention, within the bound of test_attention_over_its_tiles_layouts_masks_and_types."""
+
+    from aotolith_amd import ops
+    from aotolith_amd.graph_ops import launch_attention
+
+    gen = torch.Generator().manual_seed(lk * d)
+    dtype = torch.bfloat16 if types == "bf16" else torch.float32
+    q, k, v = (torch.randn(1, heads, rows, dim, generator=gen).to(dtype).cuda()
+               for rows, dim in ((lq, d), (lk, d), (lk, dv)))
+    mask = torch.rand(lq, lk, generator=gen).cuda() > 0.3
+    want, size, room = _attention_reference(q, k, v, mask, False, d ** -0.5)
+    with ops.recording_launches() as take:
+        take()
+        got = launch_attention(torch.full((1, heads, lq, dv), 7.0, device="cuda"), q, k, v, mask, False, d ** -0.5)
+        assert (take() == ["aoto_generic_attention"]) == few
+    bound = (4 * ((d + 4) * 2.0 ** -24 * float(room)) + (lk + 16) * 2.0 ** -24) * size + 2.0 ** -24 * want.abs()
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
 def _views(gen, dtype):
     """Pairs of operands of one broadcast shape: collapsible, broadcast, permuted, offset and odd-sized."""
 
