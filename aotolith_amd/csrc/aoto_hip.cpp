@@ -2049,8 +2049,15 @@ bool fused_layout(aoto::FusedArgs& f, long long total) {
 
 unsigned grid_for(long long total);
 
+// From how many elements a single node runs as vectors: below, the fused kernel's arguments and program cost
+// more than its loads save (us, general -> fused: add and silu of 8 elements 2.5 -> 3.1, 128 x 896 3.1 -> 3.6, 256 x
+// 896 3.7 -> 3.7, 384 x 896 4.2 -> 3.8; a cast, against the copy kernel, 128 x 896 2.5 -> 3.2, 512 x 896 3.3 -> 3.4, 768
+// x 896 3.9 -> 3.7). A chain is worth its launch at any size.
+constexpr long long kFusedNode = 1 << 18, kFusedCast = 1 << 19;
+
 int launch_elementwise(aoto::EwArgs& args, void* stream) {
-  if (args.domain == 0 && fused_op(args.op) && has_kernel("aoto_generic_fused")) {
+  if (args.domain == 0 && args.total >= (args.op == AOTO_EW_CAST ? kFusedCast : kFusedNode) && fused_op(args.op) &&
+      has_kernel("aoto_generic_fused")) {
     aoto::FusedArgs f;
     memset(&f, 0, sizeof(f));
     f.inputs = args.op >= AOTO_EW_ADD ? 2 : 1;
@@ -2377,7 +2384,8 @@ int aoto_hip_generic_copy(const aoto_tensor* dst, const aoto_tensor* src, void* 
   args.ndim = dst->ndim;
   args.total = numel(dst);
   if (args.total == 0) return AOTO_OK;
-  if (args.src_dtype != args.dst_dtype && float_dtype(src->dtype) && float_dtype(dst->dtype) && contiguous(dst)) {
+  if (args.src_dtype != args.dst_dtype && float_dtype(src->dtype) && float_dtype(dst->dtype) && contiguous(dst) &&
+      args.total >= kFusedCast) {
     // a conversion between the float types into a contiguous tensor: the elementwise cast
     aoto::EwArgs cast;
     memset(&cast, 0, sizeof(cast));

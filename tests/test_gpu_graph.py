@@ -461,6 +461,42 @@ def test_elementwise_and_copies_over_strides_and_sizes(dtype):
             wide.zero_()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows", [127, 128, 511, 512, 513])
+def test_elementwise_nodes_on_both_sides_of_their_vector_sizes(rows, dtype):
+    """Single nodes run as vectors from 2^18 elements (256 rows of 1024) and casts from 2^19, the general kernels below
+    and where rows are not whole vectors: torch's bits for contiguous, broadcast, offset and permuted operands."""
+
+    from aotolith_amd import ops
+    from aotolith_amd.graph_ops import EW, launch_copy, launch_elementwise
+
+    gen = torch.Generator().manual_seed(rows)
+    other = torch.bfloat16 if dtype == torch.float32 else torch.float32
+
+    def t(*shape):
+        return (torch.randn(*shape, generator=gen) * 3).to(dtype).cuda()
+
+    x = t(rows, 2, 1024)
+    operands = (t(rows, 2, 1024), t(1024), t(rows, 2, 1), t(2, rows, 1024).transpose(0, 1), t(rows, 2, 1040)[..., 8:1032],
+                t(rows, 2, 1030)[..., 3:1027], 0.5)
+    for index, y in enumerate(operands):
+        with ops.recording_launches() as take:
+            take()
+            out = launch_elementwise(EW["mul"], torch.empty_like(x), x, y)
+            names = take()
+        vector = rows >= 128 and index != 5
+        assert names == ["aoto_generic_fused" if vector else "aoto_generic_elementwise"], (index, names)
+        assert torch.equal(out, (x.float() * (y if isinstance(y, float) else y.float())).to(dtype)), index
+    for index, y in enumerate(operands[:1] + operands[3:6]):
+        with ops.recording_launches() as take:
+            take()
+            out = launch_copy(torch.empty(y.shape, dtype=other, device="cuda"), y)
+            names = take()
+        vector = rows >= 256 and index != 3
+        assert (names == ["aoto_generic_fused"]) == vector, (index, names)
+        assert torch.equal(out, y.to(other)), index
+
+
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32, torch.bool, torch.uint8, torch.int8])
 def test_copies_of_whole_numbers_keep_their_bits(dtype):
     from aotolith_amd.graph_ops import launch_copy
