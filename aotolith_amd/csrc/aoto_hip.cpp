@@ -137,6 +137,10 @@ bool has_kernel(const char* name) {
   return f != nullptr;
 }
 
+// Whether the code object is of a build that chose plans by the present rules: one stored by an earlier build
+// keeps the rules it was built with, which the selections recorded beside it name.
+bool present_rules() { return has_kernel("aoto_plan_rules_3"); }
+
 // Kernel symbols launched by this thread while recording is on (aoto_hip_trace_launches),
 // newline-separated, for plans that name the kernels they run; with kTraceOnly they are recorded and not
 // launched, for plans that settle which kernels they run before they have any data.
@@ -243,6 +247,9 @@ bool block_staged_shape(int K, int N, bool paired, StreamShape* s) {
                                    {64, 4}, {64, 5}, {64, 6}, {64, 7}, {64, 8}};
   const int chunks = K / 32, count = paired ? 7 : 11;
   if (K % 32 != 0 || (N > 16384 && K <= 640)) return false;
+  // (the pair has such rows earlier: two blocks per CU, l* against staged, 128 -> 2 x 8192 / 11008 / 16384 4.1 / 4.1 / 4.1
+  // against 4.0 / 4.7 / 5.3, 256 -> 2 x 16384 4.5 against 5.3, 384 -> 2 x 16384 4.8 against 5.3)
+  if (paired && K <= 384 && N > 8192 && present_rules()) return false;
   const int per_cu = N > 16384 ? (K <= 1536 ? 4 : 2) : K <= 1024 ? 2 : 1;
   for (int i = 0; i < count; ++i) {
     if (layouts[i][0] * layouts[i][1] < chunks) continue;
@@ -849,10 +856,11 @@ enum GemmTail { kTailNorm, kTailRope, kTailPaired };
 // with steps the k-steps of a slice, and the tail the separate norm / RoPE / reduce launch and what it moves.
 // Instances whose staging leaves one block to a CU pay whole rounds of 256. The constants are least squares
 // over 370 measured shapes (7 to 14 (N, K) pairs from 896 to 14336, 10 to 15 row counts from 17 to 2048, every
-// tile and 1 to 8 slices, both widths; log error of the near-best plans 0.08 to 0.10). The model's choice
-// replaces the fixed plan's where it promises 10% less: over those shapes the plans' time falls by a factor of
-// 1.29 (4-bit) and 1.42 (8-bit), 1.12 / 1.12 for the paired form, and ends 3 to 7% over the best instance and
-// split of each shape.
+// tile and 1 to 8 slices, both widths; log error of the near-best plans 0.08 to 0.10; the measurements are not
+// kept). The model's choice replaces the fixed plan's where it promises 20% less, twice that error: at 10% some
+// plans it picked were slower (511 x 8960 -> 1536 35.4 -> 39.5 us, 1500 x 896 -> 4864 28.7 -> 31.8, kept now).
+// Over 1896 GEMMs of 14 (N, K) pairs and 2 to 2048 rows, every form and both widths, times fall by 12% in the
+// geometric mean.
 struct GemmCost {
   int code;
   float launch, latency, rate;
@@ -911,9 +919,9 @@ float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits
 }
 
 // The modelled instance and split count (explicit codes), or false where the fixed plan (`tile`, `splits`
-// as it resolves, with 1 or more slices) is within 10% of the model's best.
-bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail, bool gate, int head_dim, int* tile,
-                   int* splits) {
+// as it resolves, with 1 or more slices) is within the promise (a share of its time) of the model's best.
+bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail, bool gate, int head_dim, float promise,
+                   int* tile, int* splits) {
   const bool paired = tail == kTailPaired;
   const GemmCost* table = paired ? (bits == 4 ? kCostPaired4 : kCostPaired8) : (bits == 4 ? kCost4 : kCost8);
   const int count = (int)(paired ? (bits == 4 ? sizeof(kCostPaired4) : sizeof(kCostPaired8))
@@ -940,7 +948,7 @@ bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail,
       }
     }
   }
-  if (best_tile == 0 || now == 0.f || best >= 0.9f * now) return false;
+  if (best_tile == 0 || now == 0.f || best >= promise * now) return false;
   *tile = best_tile;
   *splits = best_splits;
   return true;
@@ -960,10 +968,10 @@ bool automatic_model(int bits, int M, int N, int K, int group, GemmTail tail, bo
     bool chosen, valid;
   };
   thread_local Entry memo[256];
-  const bool pow2_even = pow2_even_groups(K, group);
+  const bool pow2_even = pow2_even_groups(K, group), present = present_rules();
   const long long a = ((long long)M << 32) | (unsigned)N;
   const long long b = ((long long)K << 32) | (bits == 8) | (gate ? 2 : 0) | (tail << 2) | (head_dim == 128 ? 16 : 0) |
-                      (head_dim == 64 ? 32 : 0) | (pow2_even ? 64 : 0);
+                      (head_dim == 64 ? 32 : 0) | (pow2_even ? 64 : 0) | (present ? 128 : 0);
   const bool known_head = tail != kTailRope || head_dim == 64 || head_dim == 128;
   Entry& e = memo[((unsigned long long)(a * 0x9E3779B97F4A7C15ull ^ b * 0xC2B2AE3D27D4EB4Full)) >> 56];
   if (known_head && e.valid && e.key[0] == a && e.key[1] == b) {
@@ -971,7 +979,7 @@ bool automatic_model(int bits, int M, int N, int K, int group, GemmTail tail, bo
     return e.chosen;
   }
   int t = *tile, s = *splits;
-  const bool chosen = modelled_plan(bits, M, N, K, pow2_even, tail, gate, head_dim, &t, &s);
+  const bool chosen = modelled_plan(bits, M, N, K, pow2_even, tail, gate, head_dim, present ? 0.8f : 0.9f, &t, &s);
   if (known_head) e = {{a, b}, t, s, chosen, true};
   if (chosen) *tile = t, *splits = s;
   return chosen;
@@ -1453,6 +1461,9 @@ int aoto_hip_w8_gemv(const void* x, const int32_t* words, const void* scales, co
     for (int i = 0; i < (paired ? 9 : 12); ++i) {
       const int lpr = layouts[i][0], cpl = layouts[i][1];
       if (lpr * cpl < K / 16) continue;
+      // (the pair's widest layout leaves lanes idle below K = 8192: wide outputs stay on w8.h's kernel, which takes 26.5 /
+      // 30.5 / 55.3 us for 7168 -> 2 x 10240 / 14336 / 28672 against 26.5 / 33.1 / 58.4 here)
+      if (paired && cpl == 8 && N > 10240 && present_rules()) break;
       char sname[64];
       snprintf(sname, sizeof(sname), "aoto_w8_gemv_x%dx%d_n%d_p%d_b%d", lpr, cpl, norm_weight ? 1 : 0, paired ? 1 : 0,
                bias ? 1 : 0);

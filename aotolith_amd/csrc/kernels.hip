@@ -17,6 +17,9 @@
 #include "flash_attention.h"
 #include "generic_attention.h"
 
+// Marks the code objects whose build chose plans by the present rules (present_rules in aoto_hip.cpp).
+extern "C" __global__ void aoto_plan_rules_3() {}
+
 // W4 decode GEMV: {lanes per row} x {norm prologue} x {paired} x {bias epilogue}.
 AOTO_GEMV_LPR(0, 0, 0)
 AOTO_GEMV_LPR(0, 0, 1)

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import json
 import os
+import re
 import subprocess
 import sys
 from pathlib import Path
@@ -186,3 +187,47 @@ def test_decode_gemvs_over_an_earlier_code_object_keep_its_kernels():
     finally:
         _lib.install_code_object(image)
     assert names(256, 512)[0].startswith("aoto_w4_gemv_x32x1")
+
+
+def test_plan_rules_are_those_of_the_code_object():
+    """Paired GEMVs of short int4 rows and of the widest int8 layout leave the staged layouts for wide outputs, and a
+    modelled GEMM has to promise a fifth - with a code object of this build; one whose mark is missing (its name changed
+    in the symbol tables) keeps the earlier lines, as the selections stored with it say."""
+
+    from aotolith_amd import _lib, ops
+
+    gen = torch.Generator(device="cuda").manual_seed(4)
+
+    def pair(k, n, bits):
+        packed, scales = ops.quantize(torch.randn(n, k, generator=gen, device="cuda").bfloat16(), 64, bits)
+        x = torch.randn(k, generator=gen, device="cuda").bfloat16()
+        gemv = ops.w4_gemv if bits == 4 else ops.w8_gemv
+        with ops.recording_launches() as take:
+            take()
+            gemv(x, packed, scales, 64, up=(packed, scales))
+            return take()[0].split("_n")[0]
+
+    def names():
+        out = [pair(256, 8192, 4), pair(256, 8208, 4), pair(448, 8208, 4), pair(384, 8208, 4), pair(7168, 10240, 8),
+               pair(7168, 10256, 8), pair(6144, 10256, 8)]
+        packed, scales = ops.quantize(torch.randn(1536, 8960, generator=gen, device="cuda").bfloat16(), 64, 4)
+        x = torch.randn(511, 8960, generator=gen, device="cuda").bfloat16()
+        with ops.recording_launches() as take:
+            take()
+            ops.w4_matmul(x, packed, scales, 64)
+            return out, take()[0]
+
+    image = _lib.default_code_object()
+    mark = b"aoto_plan_rules_3"
+    assert mark in image
+    now, gemm = names()
+    assert [n[5:12] for n in now] == ["w4_gemv"] * 4 + ["w8_gemv"] * 3
+    assert [n[13] for n in now] == ["x", "l", "l", "l", "x", "r", "x"], now  # (448 is an odd count of groups)
+    _lib.install_code_object(image.replace(mark, mark[:-1] + b"Z"))
+    try:
+        before, earlier = names()
+        torch.cuda.synchronize()
+    finally:
+        _lib.install_code_object(image)
+    assert [n[13] for n in before] == ["x", "x", "l", "x", "x", "x", "x"], before
+    assert re.match(r"aoto_w4_gemm_n\d_m\d", gemm) and not re.match(r"aoto_w4_gemm_n\d_m\d", earlier), (gemm, earlier)
