@@ -577,10 +577,11 @@ def test_automatic_codes_at_wide_outputs_of_few_rows(m, n, k, bits):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("m,n,k", [(257, 11008, 448), (257, 11008, 4096), (1030, 6144, 896)])
+@pytest.mark.parametrize("m,n,k", [(400, 8192, 1536), (400, 8192, 3584), (511, 8192, 4096)])
 def test_automatic_codes_run_without_a_workspace_where_the_fixed_plan_needs_none(m, n, k, bits):
     """A model's plan may store partials where the 16x16 plan (tile 28, unsplit) stores none: a caller without a
-    workspace gets the latter, bit for bit, single and q/k/v projections alike."""
+    workspace gets the latter, bit for bit, single and q/k/v projections alike. (The model promises more than 20% at
+    these shapes: 815 or 825 over int4 codes, 845 over int8, and 825 for the 3584-wide q/k/v.)"""
 
     from aotolith_amd import _lib, ops
 
