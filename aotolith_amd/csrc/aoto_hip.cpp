@@ -238,17 +238,17 @@ int gemv_rows(int lpr, int shape_default) {
 // hold a row. One block per CU up to 16384 outputs, two beyond (5120 -> 5120 at 1 / 2 / 3 blocks 5.7 / 5.8 / 7.3 us,
 // 2048 -> 151936 43.6 / 31.0 / 31.2), and more for short rows, a wave's loads being few (1024 -> 16384 5.0 / 4.4 /
 // 4.3, 1024 -> 151936 at 1 / 2 / 3 / 4 blocks 33.1 / 24.8 / 21.1 / 17.9); rows of up to 640 in wide outputs leave too
-// many slots empty (512 -> 151936 17.0 against 16.1 on the l* kernel). Against the l* kernel, which has no next row in flight and takes what is left
-// (odd group counts, other groups, reductions past 16384), us over rotating weights: 512 -> 512 3.9 -> 2.6, 2048 ->
-// 2048 4.2 -> 2.9, 5120 -> 13824 16.0 -> 9.9 (paired 24.4 -> 16.9), 8192 -> 8192 17.1 -> 9.8, 13824 -> 5120 26.0 ->
-// 11.1, 2048 -> 151936 44.1 -> 31.3.
+// many slots empty (512 -> 151936 17.0 against 16.1 on the l* kernel). Against the l* kernel, which has no next row
+// in flight and takes what is left (odd group counts, other groups, reductions past 16384), us over rotating
+// weights: 512 -> 512 3.9 -> 2.6, 2048 -> 2048 4.2 -> 2.9, 5120 -> 13824 16.0 -> 9.9 (paired 24.4 -> 16.9), 8192 ->
+// 8192 17.1 -> 9.8, 13824 -> 5120 26.0 -> 11.1, 2048 -> 151936 44.1 -> 31.3.
 bool block_staged_shape(int K, int N, bool paired, StreamShape* s) {
   static const int layouts[][2] = {{32, 1}, {32, 2}, {32, 3}, {32, 4}, {32, 5}, {64, 3},
                                    {64, 4}, {64, 5}, {64, 6}, {64, 7}, {64, 8}};
   const int chunks = K / 32, count = paired ? 7 : 11;
   if (K % 32 != 0 || (N > 16384 && K <= 640)) return false;
-  // (the pair has such rows earlier: two blocks per CU, l* against staged, 128 -> 2 x 8192 / 11008 / 16384 4.1 / 4.1 / 4.1
-  // against 4.0 / 4.7 / 5.3, 256 -> 2 x 16384 4.5 against 5.3, 384 -> 2 x 16384 4.8 against 5.3)
+  // (the pair has such rows earlier: two blocks per CU, l* against staged, 128 -> 2 x 8192 / 11008 / 16384 4.1 / 4.1 /
+  // 4.1 against 4.0 / 4.7 / 5.3, 256 -> 2 x 16384 4.5 against 5.3, 384 -> 2 x 16384 4.8 against 5.3)
   if (paired && K <= 384 && N > 8192 && present_rules()) return false;
   const int per_cu = N > 16384 ? (K <= 1536 ? 4 : 2) : K <= 1024 ? 2 : 1;
   for (int i = 0; i < count; ++i) {
@@ -654,7 +654,7 @@ bool wide_code(int tile) {
 // 813 / 814 / 825 over 8-bit codes.
 bool lds_byte_code(int tile) { return tile == 833 || tile == 834 || tile == 845; }
 bool lds_code(int tile) {
-  return tile == 815 || tile == 825 || lds_byte_code(tile) || tile == 811 || tile == 812 || tile == 813 || tile == 814 || tile == 821 || tile == 822 || tile == 823;
+  return (tile >= 811 && tile <= 815) || (tile >= 821 && tile <= 823) || tile == 825 || lds_byte_code(tile);
 }
 bool lds_paired_code(int tile) { return tile == 811 || tile == 812 || tile == 821; }
 bool lds_split_code(int tile) {
@@ -912,7 +912,9 @@ float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits
   if (tail == kTailPaired)
     t += split ? 0.8f + 1.2f * sum : 0.f;
   else if (tail == kTailRope)
-    t += split ? 1.6f + sum : !p.lds && !p.wide_mt && p.bn() % head_dim == 0 && N % p.bn() == 0 ? 0.f : 1.3f + 1.6f * mn;
+    t += split                                                                        ? 1.6f + sum
+         : !p.lds && !p.wide_mt && p.bn() % head_dim == 0 && N % p.bn() == 0 ? 0.f
+                                                                             : 1.3f + 1.6f * mn;
   else
     t += split ? 1.f + sum : 1.3f + 1.7f * mn;
   return t;
@@ -939,7 +941,7 @@ bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail,
     const int steps = K / (lds_code(c.code) ? 64 : 128);
     for (int s : slices) {
       if (s > most && (s > 1 || lds_split_code(c.code))) break;
-      if ( (s > 1 && (2 * s > steps || (lds_code(c.code) && !lds_split_code(c.code))))) break;
+      if (s > 1 && (2 * s > steps || (lds_code(c.code) && !lds_split_code(c.code)))) break;
       const float t = modelled_cost(c, bits, M, N, K, s, tail, head_dim);
       if (best_tile == 0 || t < best) {
         best = t;
@@ -1164,7 +1166,8 @@ int packed_gemm(int bits, const void* x, const int32_t* words, const void* scale
     return fail(AOTO_ERR_ARGUMENT, "%s: tile code %d is not one of 12, 14, 18, 24, 28, 241, 242, 243, 281, 441, "
                 "811, 812, 813, 814, 815, 821, 822, 823, 825, 833, 834, 845", what, tile);
   if (lds_code(tile)) {
-    if (bits != (lds_byte_code(tile) ? 8 : 4) || lds_paired_code(tile) != paired || gate != nullptr || (splits > 1 && !lds_split_code(tile)))
+    if (bits != (lds_byte_code(tile) ? 8 : 4) || lds_paired_code(tile) != paired || gate != nullptr ||
+        (splits > 1 && !lds_split_code(tile)))
       return fail(AOTO_ERR_ARGUMENT, "%s: tile %d is the %s%d-bit %s form without a gate epilogue", what, tile,
                   lds_split_code(tile) ? "" : "unsplit ", lds_byte_code(tile) ? 8 : 4,
                   lds_paired_code(tile) ? "paired" : "single");
@@ -1196,7 +1199,8 @@ int packed_gemm(int bits, const void* x, const int32_t* words, const void* scale
   if (tile == 0 && splits == 0) {
     if (const int code = lds_auto(bits, M, N, K, group, paired, gate != nullptr, rope != nullptr))
       tile = code;
-    else if (rope == nullptr && modelled_shape(bits, M, N, K, group, paired, gate != nullptr, false) && models_plans()) {
+    else if (rope == nullptr && modelled_shape(bits, M, N, K, group, paired, gate != nullptr, false) &&
+             models_plans()) {
       int t = 0, s = 0;
       if (automatic_model(bits, M, N, K, group, paired ? kTailPaired : kTailNorm, gate != nullptr, 0, &t, &s) &&
           (usable_workspace(workspace) || !stores_partials(M, N, K, t, s, paired)))
@@ -1461,8 +1465,8 @@ int aoto_hip_w8_gemv(const void* x, const int32_t* words, const void* scales, co
     for (int i = 0; i < (paired ? 9 : 12); ++i) {
       const int lpr = layouts[i][0], cpl = layouts[i][1];
       if (lpr * cpl < K / 16) continue;
-      // (the pair's widest layout leaves lanes idle below K = 8192: wide outputs stay on w8.h's kernel, which takes 26.5 /
-      // 30.5 / 55.3 us for 7168 -> 2 x 10240 / 14336 / 28672 against 26.5 / 33.1 / 58.4 here)
+      // (the pair's widest layout leaves lanes idle below K = 8192: wide outputs stay on w8.h's kernel, which takes
+      // 26.5 / 30.5 / 55.3 us for 7168 -> 2 x 10240 / 14336 / 28672 against 26.5 / 33.1 / 58.4 here)
       if (paired && cpl == 8 && N > 10240 && present_rules()) break;
       char sname[64];
       snprintf(sname, sizeof(sname), "aoto_w8_gemv_x%dx%d_n%d_p%d_b%d", lpr, cpl, norm_weight ? 1 : 0, paired ? 1 : 0,
@@ -1470,12 +1474,13 @@ int aoto_hip_w8_gemv(const void* x, const int32_t* words, const void* scales, co
       if (!has_kernel(sname)) break;
       const int rows = 64 / lpr;
       const long long tiles = ((long long)N + rows - 1) / rows;
-      const long long budget = (long long)cu_count() * gemv_blocks_per_cu(paired || K > 8192 ? 1 : N > 16384 && K <= 1536 ? 4 : 2) * 4;
+      const int per_cu = paired || K > 8192 ? 1 : N > 16384 && K <= 1536 ? 4 : 2;
+      const long long budget = (long long)cu_count() * gemv_blocks_per_cu(per_cu) * 4;
       const long long waves = tiles < budget ? tiles : budget;
       int shift = 0;
       while ((16 << shift) < group) ++shift;
-      return launch(sname, dim3((unsigned)((waves + 3) / 4)), dim3(256), (unsigned)(K * 2 + K / 4), stream, words, scales,
-                    x, norm_weight, K, N, shift, bias, up_words, up_scales, eps, alpha, beta, y);
+      return launch(sname, dim3((unsigned)((waves + 3) / 4)), dim3(256), (unsigned)(K * 2 + K / 4), stream, words,
+                    scales, x, norm_weight, K, N, shift, bias, up_words, up_scales, eps, alpha, beta, y);
     }
   }
   // A wave holds R rows x U chunks of 16 codes per lane in flight: U covers the
@@ -1645,8 +1650,8 @@ int aoto_hip_decode_attention(const void* q, const void* keys, const void* value
     if (has_kernel(name)) {
       if (int st = launch(name, dim3(gs, batch * query_heads / gb), dim3(256), 0, stream, q, keys, values,
                           (long long)kv_batch_stride, (long long)kv_head_stride, mask, mask_batch_stride, valid,
-                          ring_offset, capacity, query_heads, kv_heads, gb, scale, gchunk, (float*)workspace, step_state,
-                          out))
+                          ring_offset, capacity, query_heads, kv_heads, gb, scale, gchunk, (float*)workspace,
+                          step_state, out))
         return st;
       return gs > 1 ? launch_merge(batch * query_heads, gs, head_dim, workspace, out, stream) : AOTO_OK;
     }
@@ -1700,8 +1705,8 @@ int aoto_hip_decode_rope_attention(const void* row, int row_width, int query_sta
     snprintf(name, sizeof(name), "aoto_decode_rope_attention_d%d_g", head_dim);
     if (has_kernel(name)) {
       if (int st = launch(name, dim3(gs, batch * query_heads / gb), dim3(256), 0, stream, row, rope_rows, keys, values,
-                          (int)kv_head_stride, (int)kv_batch_stride, heads, starts_qk, start_v_width, capacity, gchunk, gb,
-                          valid, ring_offset, position, slot, scale, (float*)workspace, step_state, cos_table,
+                          (int)kv_head_stride, (int)kv_batch_stride, heads, starts_qk, start_v_width, capacity, gchunk,
+                          gb, valid, ring_offset, position, slot, scale, (float*)workspace, step_state, cos_table,
                           sin_table, out))
         return st;
       return gs > 1 ? launch_merge(batch * query_heads, gs, head_dim, workspace, out, stream) : AOTO_OK;
@@ -2030,8 +2035,9 @@ int collapse_dims(int ndim, long long* shape, long long* const* walks, int count
 bool fused_op(int op) {
   switch (op) {
     case AOTO_EW_CAST: case AOTO_EW_NEG: case AOTO_EW_ABS: case AOTO_EW_RSQRT: case AOTO_EW_EXP: case AOTO_EW_SIGMOID:
-    case AOTO_EW_SILU: case AOTO_EW_RELU: case AOTO_EW_TANH: case AOTO_EW_GELU: case AOTO_EW_GELU_TANH: case AOTO_EW_ADD:
-    case AOTO_EW_SUB: case AOTO_EW_MUL: case AOTO_EW_DIV: case AOTO_EW_MAXIMUM: case AOTO_EW_MINIMUM: return true;
+    case AOTO_EW_SILU: case AOTO_EW_RELU: case AOTO_EW_TANH: case AOTO_EW_GELU: case AOTO_EW_GELU_TANH:
+    case AOTO_EW_ADD: case AOTO_EW_SUB: case AOTO_EW_MUL: case AOTO_EW_DIV: case AOTO_EW_MAXIMUM:
+    case AOTO_EW_MINIMUM: return true;
     default: return false;
   }
 }
@@ -2062,8 +2068,8 @@ unsigned grid_for(long long total);
 
 // From how many elements a single node runs as vectors: below, the fused kernel's arguments and program cost
 // more than its loads save (us, general -> fused: add and silu of 8 elements 2.5 -> 3.1, 128 x 896 3.1 -> 3.6, 256 x
-// 896 3.7 -> 3.7, 384 x 896 4.2 -> 3.8; a cast, against the copy kernel, 128 x 896 2.5 -> 3.2, 512 x 896 3.3 -> 3.4, 768
-// x 896 3.9 -> 3.7). A chain is worth its launch at any size.
+// 896 3.7 -> 3.7, 384 x 896 4.2 -> 3.8; a cast, against the copy kernel, 128 x 896 2.5 -> 3.2, 512 x 896 3.3 -> 3.4,
+// 768 x 896 3.9 -> 3.7). A chain is worth its launch at any size.
 constexpr long long kFusedNode = 1 << 18, kFusedCast = 1 << 19;
 
 int launch_elementwise(aoto::EwArgs& args, void* stream) {
@@ -2554,8 +2560,8 @@ int aoto_hip_generic_attention(const aoto_tensor* out, const aoto_tensor* q, con
   if (B == 0 || H == 0 || Lq == 0 || Dv == 0) return AOTO_OK;
   // A few keys of small heads are less than the matrix kernel's prologue and combination: up to 4 keys of 16 columns
   // run one block a row (us, that -> the matrix kernel: 8 heads of 16, one query over 1 / 4 / 8 / 16 keys, bf16 7.1 /
-  // 7.7 / 8.4 / 10.0 -> 8.8, f32 6.7 / 7.2 / 8.0 / 9.6 -> 8.5; 512 rows over 4 / 8 keys 8.0 / 8.8 -> 8.4; heads of 32, one
-  // key 11.2 -> 9.0).
+  // 7.7 / 8.4 / 10.0 -> 8.8, f32 6.7 / 7.2 / 8.0 / 9.6 -> 8.5; 512 rows over 4 / 8 keys 8.0 / 8.8 -> 8.4; heads of 32,
+  // one key 11.2 -> 9.0).
   const bool few = D <= 16 && Dv <= 16 && Lk <= 4 && B * H * Lq <= 512;
   if (D <= 128 && Dv <= 128 && !few && has_kernel("aoto_generic_attention_f32_d64_a")) {
     char name[64];

@@ -390,8 +390,8 @@ __device__ __forceinline__ void decode_attention_group_body(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ row, int row_width, int query_start, int key_start,
     int value_start, const uint16_t* __restrict__ cos_table, const uint16_t* __restrict__ sin_table,
     uint16_t* __restrict__ kbase, uint16_t* __restrict__ vbase, long long kv_batch_stride, long long kv_head_stride,
-    const uint8_t* __restrict__ mask, int mask_batch_stride, int valid, int ring_offset, int position, int slot, int cap,
-    int query_heads, int kv_heads, int gb, float scale, int chunk, float* __restrict__ partials,
+    const uint8_t* __restrict__ mask, int mask_batch_stride, int valid, int ring_offset, int position, int slot,
+    int cap, int query_heads, int kv_heads, int gb, float scale, int chunk, float* __restrict__ partials,
     const int* __restrict__ step, const uint16_t* __restrict__ rope_rows, uint16_t* __restrict__ out) {
   constexpr int WAVES = 4, WK = 32, TILE = WAVES * WK;
   constexpr int DC = D / 32;           // 32-dim operand chunks of a row

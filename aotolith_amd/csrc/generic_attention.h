@@ -121,8 +121,8 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
 #pragma unroll
       for (int i = 0; i < VL; ++i) {
         const int c = lane + 64 * i, row = c / RC, d0 = (c % RC) * E;
-        vf[i] = attn_chunk<F32, VEC>(a.v, a.v_dtype, vbase + (long long)min(j0 + row, a.lk - 1) * a.vs[2] + d0 * a.vs[3],
-                                     a.vs[3], a.dv - d0);
+        const long long off = vbase + (long long)min(j0 + row, a.lk - 1) * a.vs[2] + d0 * a.vs[3];
+        vf[i] = attn_chunk<F32, VEC>(a.v, a.v_dtype, off, a.vs[3], a.dv - d0);
       }
     }
   };
@@ -164,7 +164,8 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
         const long long vrow = vbase + (long long)j * a.vs[2];
         bool any = false;
 #pragma nounroll
-        for (int d = lane; d < a.dv; d += 64) any = any || not_finite_f32(load_float(a.v, a.v_dtype, vrow + d * a.vs[3]));
+        for (int d = lane; d < a.dv; d += 64)
+          any = any || not_finite_f32(load_float(a.v, a.v_dtype, vrow + d * a.vs[3]));
         if (!__any(any)) continue;
         bool keep = !(a.causal && j > qi);
         float add = 0.f;
@@ -311,7 +312,8 @@ __device__ __forceinline__ void generic_attention_body(const AttnArgs& a) {
       for (int e = 0; e < 16; ++e)
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
-          // (rows past the keys and columns past the head repeat the last: their weight is zero, or they are not stored)
+          // (rows past the keys and columns past the head repeat the last: their weight is zero, or they are not
+          // stored)
           const bool special = not_finite_f32(vf32[e][t]);
           odd = odd || special;
           const float v = special ? 0.f : vf32[e][t];
