@@ -639,7 +639,7 @@ constexpr int kMergeRegSplits = 40;
 extern "C" __global__ __launch_bounds__(128) void aoto_decode_attention_merge(const float* __restrict__ partials,
                                                                              int splits, int D,
                                                                              uint16_t* __restrict__ out) {
-  __shared__ float s_w[kMergeMaxSplits];
+  __shared__ float s_w[kMergeMaxSplits + 16];
   __shared__ float s_red[4];
   const int bh = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -675,14 +675,19 @@ extern "C" __global__ __launch_bounds__(128) void aoto_decode_attention_merge(co
     const float t = fmaf(s_w[s], a[s], num);
     num = s < splits ? t : num;
   }
-  // the splits past the registers, 16 loads in flight (one by one, each was a round trip)
-  for (int s0 = kMergeRegSplits; s0 < splits; s0 += 16) {
+  // The splits past the registers, 16 loads in flight and no branch between them: a condition on each (64-bit
+  // address products, one load behind a wait) took longer than four loads at a time.
+  const float* past = rec + kMergeRegSplits * stride + 2 + dc;
+  for (int s0 = kMergeRegSplits; s0 < splits; s0 += 16, past += 16 * stride) {
+    const int left = splits - s0;  // uniform
     float t[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) t[i] = rec[(size_t)min(s0 + i, splits - 1) * stride + 2 + dc];
+    for (int i = 0; i < 16; ++i) t[i] = past[(unsigned)(min(i, left - 1) * (D + 2))];
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (s0 + i < splits) num = fmaf(s_w[s0 + i], t[i], num);
+    for (int i = 0; i < 16; ++i) {
+      const float u = fmaf(s_w[s0 + i], t[i], num);  // (s_w: a whole batch past the last split)
+      num = i < left ? u : num;
+    }
   }
   if (column) out[(size_t)bh * D + d] = (uint16_t)f32_to_bf16(den > 0.f ? num / den : 0.f);
 }

@@ -756,6 +756,26 @@ def test_workspaces_in_host_memory_are_refused():
         lambda: ops.w4_matmul_gate_up(x, packed, scales, packed, scales, 64, workspace=host),
         lambda: ops.matmul_residual_norm(x, packed, scales, 64, weight.expand(8, 768).contiguous(), weight, 1e-6,
                                          workspace=host),
+@pytest.mark.parametrize("splits", [39, 40, 41, 55, 56, 57, 72, 188])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_merge_of_any_number_of_splits(dim, splits):
+    """Records in registers (40), whole batches of 16 behind them and a partial last one: against 64-bit attention."""
+
+    ops = _ops()
+    gen = torch.Generator().manual_seed(splits)
+    cap, valid = 4992, 4101
+    pair = torch.randn(2, 1, 2, cap, dim, generator=gen).bfloat16().cuda()
+    q = torch.randn(1, 4, dim, generator=gen).bfloat16().cuda()
+    workspace = ops.decode_attention_workspace(1, 4, 2, cap, dim, splits, device="cuda")
+    got = ops.decode_attention(q, pair[0], pair[1], valid=valid, splits=splits, workspace=workspace)
+    query, (keys, values) = q.double().view(1, 2, 2, dim), pair.double()
+    scores = (query @ keys.transpose(-1, -2)) * dim ** -0.5
+    scores[..., : cap - valid] = float("-inf")
+    want = (torch.softmax(scores, -1) @ values).view(1, 4, dim)
+    # f32 sums of the kept keys, then one bf16 rounding (2^-8)
+    assert bool(((got.double() - want).abs() <= 1e-5 + 2.0 ** -8 * want.abs() + 2e-4 * want.abs().amax()).all())
+
+
         lambda: ops.matmul_qkv_rope(x, packed, scales, 64, torch.arange(8, device="cuda"), table, table,
                                     kv[:, :, :4], query_heads=4, kv_heads=4, head_dim=64, slot0=0, workspace=host),
     ]
