@@ -1607,6 +1607,12 @@ int grouped_decode(int batch, int query_heads, int kv_heads, int capacity, int h
                    int* chunk) {
   if (requested > 0 || *splits <= 1 || capacity < (head_dim == 64 ? 2048 : 4096)) return 0;
   const int group = query_heads / kv_heads;
+// Beyond that line too the one-head form stays where its merge reads up to 48 records a head and its blocks have few
+// keys, or the shared form's blocks are 64 or fewer (plain form, us, one head -> shared: 8 heads over 1 of 64, batch 4,
+// 2304 / 3500 / 4096 keys 7.6 / 8.5 / 8.8 -> 8.4 / 9.8 / 9.8; 4 over 2, batch 8, 2304 keys 8.0 -> 9.9; 28 over 4, 4096
+// keys 9.1 -> 9.7; 32 over 2 of 128, 4096 keys 10.7 -> 12.3; with blocks of more keys, 28 over 4, batch 2, 2700 keys
+// 11.2 -> 9.7). Over 584 shapes of 1 to 8 windows and 2 to 64 heads the choice takes 0.3% more than the better form
+// in the mean, 9% at worst.
   int gb = group < 16 ? group : 16;
   while (group % gb != 0) --gb;
   if (gb < 2) return 0;
@@ -1619,6 +1625,7 @@ int grouped_decode(int batch, int query_heads, int kv_heads, int capacity, int h
   *splits = (capacity + *chunk - 1) / *chunk;
   return gb;
 }
+  if (*splits <= 48 && (*chunk < (head_dim == 64 ? 176 : 112) || rows * s <= 64) && present_rules()) return 0;
 
 int launch_merge(int rows, int splits, int head_dim, void* workspace, void* out, void* stream) {
   return launch("aoto_decode_attention_merge", dim3(rows), dim3(128), 0, stream, (const float*)workspace, splits,

@@ -191,7 +191,8 @@ def test_decode_gemvs_over_an_earlier_code_object_keep_its_kernels():
 
 def test_plan_rules_are_those_of_the_code_object():
     """Paired GEMVs of short int4 rows and of the widest int8 layout leave the staged layouts for wide outputs, and a
-    modelled GEMM has to promise a fifth - with a code object of this build; one whose mark is missing (its name changed
+    modelled GEMM has to promise a fifth, and 16 query heads over 2048 keys keep a block each - with a code object of
+    this build; one whose mark is missing (its name changed
     in the symbol tables) keeps the earlier lines, as the selections stored with it say."""
 
     from aotolith_amd import _lib, ops
@@ -215,19 +216,24 @@ def test_plan_rules_are_those_of_the_code_object():
         with ops.recording_launches() as take:
             take()
             ops.w4_matmul(x, packed, scales, 64)
-            return out, take()[0]
+            gemm = take()[0]
+            q, keys = (torch.zeros(1, *shape, dtype=torch.bfloat16, device="cuda") for shape in ((16, 64), (2, 2048, 64)))
+            ops.decode_attention(q, keys, keys, valid=2048,
+                                 workspace=ops.decode_attention_workspace(1, 16, 2, 2048, 64, device="cuda"))
+            return out, gemm, take()[0]
 
     image = _lib.default_code_object()
     mark = b"aoto_plan_rules_3"
     assert mark in image
-    now, gemm = names()
+    now, gemm, attention = names()
     assert [n[5:12] for n in now] == ["w4_gemv"] * 4 + ["w8_gemv"] * 3
     assert [n[13] for n in now] == ["x", "l", "l", "l", "x", "r", "x"], now  # (448 is an odd count of groups)
     _lib.install_code_object(image.replace(mark, mark[:-1] + b"Z"))
     try:
-        before, earlier = names()
+        before, earlier, shared = names()
         torch.cuda.synchronize()
     finally:
         _lib.install_code_object(image)
     assert [n[13] for n in before] == ["x", "x", "l", "x", "x", "x", "x"], before
+    assert not attention.endswith("_g") and shared.endswith("_g"), (attention, shared)
     assert re.match(r"aoto_w4_gemm_n\d_m\d", gemm) and not re.match(r"aoto_w4_gemm_n\d_m\d", earlier), (gemm, earlier)

@@ -634,7 +634,8 @@ def test_argmax_at_chunk_edges_with_ties_signs_and_nans(n):
 
 @pytest.mark.parametrize("hq,hkv,dim,cap,valid,batch", [
     (14, 2, 64, 2048, 2048, 1), (7, 1, 64, 2049, 1500, 1), (4, 2, 64, 5003, 5003, 2), (40, 2, 64, 2300, 9, 1),
-    (32, 8, 128, 4096, 4000, 1), (8, 4, 128, 4131, 4131, 2), (16, 1, 128, 9000, 7777, 1), (34, 2, 64, 2500, 2500, 1)])
+    (32, 8, 128, 4096, 4000, 1), (8, 4, 128, 4131, 4131, 2), (16, 1, 128, 9000, 7777, 1), (34, 2, 64, 2500, 2500, 1),
+    (40, 2, 64, 4200, 9, 1), (8, 4, 128, 7001, 7001, 2)])
 @pytest.mark.parametrize("form", ["ring", "rows", "step", "plain", "mask"])
 def test_long_windows_share_a_pass_over_the_kv_head(hq, hkv, dim, cap, valid, batch, form):
     """Windows from the length where query heads share a block (groups of 2 to 17 heads: 17 stays one head a block),
@@ -693,6 +694,24 @@ def test_long_windows_share_a_pass_over_the_kv_head(hq, hkv, dim, cap, valid, ba
     room = 1e-5 + 2.0 ** -8 * want.abs() + 2e-4 * want.abs().amax()
     assert bool(((got.double() - want).abs() <= room).all())
     assert bool(((got.double() - other.double()).abs() <= 2.0 ** -7 * want.abs() + 2e-4 * want.abs().amax()).all())
+
+
+@pytest.mark.parametrize("hq,hkv,dim,cap,batch,shared", [
+    (4, 1, 64, 2047, 1, False), (4, 1, 64, 2048, 1, True), (16, 2, 64, 2048, 1, False), (15, 3, 64, 2048, 1, True),
+    (28, 4, 64, 4900, 1, False), (28, 4, 64, 4901, 1, True), (32, 2, 128, 4096, 1, False), (32, 4, 128, 4096, 1, True),
+    (16, 2, 128, 5300, 1, False), (4, 4, 64, 16384, 1, False)])
+def test_query_heads_share_a_block_where_that_is_faster(hq, hkv, dim, cap, batch, shared):
+    """Either side of the lines: the shortest window, 48 records in the one-head form's merge, 176 (112 at D = 128) keys
+    in its blocks, 64 blocks in the shared form's, groups of one head."""
+
+    ops = _ops()
+    pair = torch.zeros(2, batch, hkv, cap, dim, dtype=torch.bfloat16, device="cuda")
+    q = torch.zeros(batch, hq, dim, dtype=torch.bfloat16, device="cuda")
+    with ops.recording_launches() as take:
+        take()
+        ops.decode_attention(q, pair[0], pair[1], valid=cap,
+                             workspace=ops.decode_attention_workspace(batch, hq, hkv, cap, dim, device="cuda"))
+        assert take()[0].endswith("_g") == shared
 
 
 @pytest.mark.parametrize("hq,hkv,dim,cap", [(14, 2, 64, 2304), (7, 1, 64, 2051), (32, 8, 128, 4131), (16, 1, 128, 9000)])
