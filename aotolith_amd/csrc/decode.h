@@ -718,6 +718,10 @@ extern "C" __global__ __launch_bounds__(256) void aoto_embedding(
 // per 16-byte load when the row is 16-byte aligned, scalar otherwise. Writes
 // int64 token ids; with `history` non-null also appends the token at
 // history[*history_len] and bumps the length (the decode loop's token record).
+// Rows of up to 16384 make a key of every element: they are one or two loads a thread, and the long form's last
+// load of its winner waits once more (us, short -> long form: 8 elements 2.5 -> 2.6, 8192 2.9 -> 3.4, 16384 3.5 ->
+// 3.6, 18432 3.7 -> 3.6, 32768 4.9 -> 4.0).
+constexpr int kArgmaxShortRow = 16384;
 extern "C" __global__ __launch_bounds__(1024) void aoto_argmax(const uint16_t* __restrict__ logits, int n,
                                                                long long row_stride, long long* __restrict__ out,
                                                                long long* __restrict__ history,
@@ -726,13 +730,23 @@ extern "C" __global__ __launch_bounds__(1024) void aoto_argmax(const uint16_t* _
   const uint16_t* row = logits + (size_t)blockIdx.x * row_stride;
   unsigned long long best = 0;
   const bool vec = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0) && (n % 8 == 0);
-  if (vec) {
+  const uint4* rv = reinterpret_cast<const uint4*>(row);
+  auto take = [&](const uint4& r, int c) {
+    const uint32_t raw[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      best = max_u64(best, argmax_key(raw[j] & 0xFFFFu, c * 8 + 2 * j));
+      best = max_u64(best, argmax_key(raw[j] >> 16, c * 8 + 2 * j + 1));
+    }
+  };
+  if (vec && n <= kArgmaxShortRow) {
+    for (int c = threadIdx.x; c < n / 8; c += 1024) take(rv[c], c);
+  } else if (vec) {
     // One CU reads the row, so the arithmetic per 8-element chunk is kept short: order-preserving 16-bit
     // integers two to a register, the chunk's maximum against the thread's best chunk so far (an earlier
     // chunk keeps a tie), and the element only for the winner. A 64-bit key per element took 17 us for
     // 151936 logits, four chunk loads in flight and packed maxima 9 us. Chunks with a NaN (which never
     // wins) take the keys.
-    const uint4* rv = reinterpret_cast<const uint4*>(row);
     const int chunks = n / 8;
     int best_chunk = -1, best_value = -32769;
     for (int c0 = threadIdx.x; c0 < chunks; c0 += 4096) {
@@ -752,11 +766,7 @@ extern "C" __global__ __launch_bounds__(1024) void aoto_argmax(const uint16_t* _
           size = __builtin_elementwise_max(size, v & low);
         }
         if (max((int)size.x, (int)size.y) > 0x7F80) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            best = max_u64(best, argmax_key(raw[j] & 0xFFFFu, c * 8 + 2 * j));
-            best = max_u64(best, argmax_key(raw[j] >> 16, c * 8 + 2 * j + 1));
-          }
+          take(r[u], c);
         } else {
           const int value = max((int)top.x, (int)top.y);
           if (value > best_value) {
@@ -766,15 +776,7 @@ extern "C" __global__ __launch_bounds__(1024) void aoto_argmax(const uint16_t* _
         }
       }
     }
-    if (best_chunk >= 0) {
-      const uint4 r = rv[best_chunk];
-      const uint32_t raw[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        best = max_u64(best, argmax_key(raw[j] & 0xFFFFu, best_chunk * 8 + 2 * j));
-        best = max_u64(best, argmax_key(raw[j] >> 16, best_chunk * 8 + 2 * j + 1));
-      }
-    }
+    if (best_chunk >= 0) take(rv[best_chunk], best_chunk);
   } else {
     for (int i = threadIdx.x; i < n; i += 1024) best = max_u64(best, argmax_key(row[i], i));
   }

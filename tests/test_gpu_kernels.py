@@ -606,7 +606,7 @@ def test_matmul_qkv_rope_equals_matmul_then_rope(m, hq, hkv, dim, k, splits, bia
         m, hq + 2 * hkv, dim).transpose(1, 0, 2)[None, hq + hkv:])
 
 
-@pytest.mark.parametrize("n", [8, 56, 8192, 32768, 32776, 151936])
+@pytest.mark.parametrize("n", [8, 56, 8192, 16384, 16392, 32768, 32776, 151936])
 def test_argmax_at_chunk_edges_with_ties_signs_and_nans(n):
     """Rows around the loop's 8, 8192 and 32768 elements: ties go to the first index, +0 beats -0, NaN never wins,
     an all-NaN row gives index 0; a row start that is not 16-byte aligned gives the same indices."""
