@@ -504,11 +504,15 @@ namespace {
 // The packers' kernel: the coalesced form where a group is a power-of-two count of
 // 8-weight units that fits one wave (groups of 8 to 512) and the base allows 16-byte
 // loads and whole-word stores; other groups and bases keep one thread per group.
+// Groups of 8, which a thread reads as whole 16-byte loads there too, from 2^20 bf16 or 2^18 f32 weights on (us, one
+// thread per group -> coalesced: bf16 64 x 512 3.8 -> 4.9, 1024 x 1024 4.6 -> 5.1, 2048 x 1024 6.4 -> 5.3; f32 64 x 512
+// 4.1 -> 4.3, 512 x 512 4.2 -> 4.4, 896 x 896 5.8 -> 4.5).
 int launch_quantize(int bits, const void* weight, int weight_is_f32, int rows, int inner, int group,
                     int32_t* packed, void* scales_bf16, float* scales_f32, void* stream) {
   const char* wide = bits == 4 ? "aoto_w4_quantize_units" : "aoto_w8_quantize_units";
   const int lanes = group / 8;
-  if (group % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && aligned16(weight) && aligned8(packed) &&
+  const bool few = lanes == 1 && (long long)rows * inner <= (weight_is_f32 ? 1 << 18 : 1 << 20);
+  if (!few && group % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && aligned16(weight) && aligned8(packed) &&
       has_kernel(wide)) {
     const long long units = (long long)rows * (inner / 8);
     int shift = 0;
@@ -1603,16 +1607,16 @@ int decode_attention_plan(const char* what, int batch, int query_heads, int kv_h
 // 14 over 2 heads of 64, 1536 / 2304 / 4096 keys 9.1 / 10.1 / 11.4 -> 8.9 / 9.0 / 9.3; 28 over 4, 1536 / 4096 /
 // 16384 8.6 / 10.5 / 20.7 -> 9.0 / 10.6 / 14.3; 32 over 8 heads of 128, 2304 / 4096 / 8192 / 16384 10.3 / 13.7 /
 // 23.5 / 44.0 -> 12.0 / 13.3 / 15.9 / 22.2. Two blocks per CU's worth of splits run in two rounds (24.1 us at 8192).
-int grouped_decode(int batch, int query_heads, int kv_heads, int capacity, int head_dim, int requested, int* splits,
-                   int* chunk) {
-  if (requested > 0 || *splits <= 1 || capacity < (head_dim == 64 ? 2048 : 4096)) return 0;
-  const int group = query_heads / kv_heads;
 // Beyond that line too the one-head form stays where its merge reads up to 48 records a head and its blocks have few
 // keys, or the shared form's blocks are 64 or fewer (plain form, us, one head -> shared: 8 heads over 1 of 64, batch 4,
 // 2304 / 3500 / 4096 keys 7.6 / 8.5 / 8.8 -> 8.4 / 9.8 / 9.8; 4 over 2, batch 8, 2304 keys 8.0 -> 9.9; 28 over 4, 4096
 // keys 9.1 -> 9.7; 32 over 2 of 128, 4096 keys 10.7 -> 12.3; with blocks of more keys, 28 over 4, batch 2, 2700 keys
 // 11.2 -> 9.7). Over 584 shapes of 1 to 8 windows and 2 to 64 heads the choice takes 0.3% more than the better form
 // in the mean, 9% at worst.
+int grouped_decode(int batch, int query_heads, int kv_heads, int capacity, int head_dim, int requested, int* splits,
+                   int* chunk) {
+  if (requested > 0 || *splits <= 1 || capacity < (head_dim == 64 ? 2048 : 4096)) return 0;
+  const int group = query_heads / kv_heads;
   int gb = group < 16 ? group : 16;
   while (group % gb != 0) --gb;
   if (gb < 2) return 0;
@@ -1621,11 +1625,11 @@ int grouped_decode(int batch, int query_heads, int kv_heads, int capacity, int h
   const long long tiles = (capacity + 127) / 128;
   if (s > tiles) s = tiles;
   if (s > *splits) s = *splits;
+  if (*splits <= 48 && (*chunk < (head_dim == 64 ? 176 : 112) || rows * s <= 64) && present_rules()) return 0;
   *chunk = (int)((capacity + s - 1) / s);
   *splits = (capacity + *chunk - 1) / *chunk;
   return gb;
 }
-  if (*splits <= 48 && (*chunk < (head_dim == 64 ? 176 : 112) || rows * s <= 64) && present_rules()) return 0;
 
 int launch_merge(int rows, int splits, int head_dim, void* workspace, void* out, void* stream) {
   return launch("aoto_decode_attention_merge", dim3(rows), dim3(128), 0, stream, (const float*)workspace, splits,

@@ -756,25 +756,6 @@ def test_long_windows_keep_infinite_values(hq, hkv, dim, cap, form):
     assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-5)[~special].all())
 
 
-def test_workspaces_in_host_memory_are_refused():
-    """Refused by the wrappers before anything is launched: the kernels would store to a host address."""
-
-    from aotolith_amd import ops
-
-    host = torch.zeros(1 << 20, dtype=torch.uint8)
-    q = torch.zeros(1, 4, 64, dtype=torch.bfloat16, device="cuda")
-    kv = torch.zeros(2, 1, 4, 1024, 64, dtype=torch.bfloat16, device="cuda")
-    row, table = torch.zeros(1, 12 * 64, dtype=torch.bfloat16, device="cuda"), kv[0, 0, 0]
-    packed, scales = ops.quantize(torch.zeros(768, 256, dtype=torch.bfloat16, device="cuda"), 64, 4)
-    x, weight = table[:8, :1].expand(8, 256).contiguous(), torch.zeros(768, dtype=torch.bfloat16, device="cuda")
-    calls = [
-        lambda: ops.decode_attention(q, kv[0], kv[1], valid=1024, workspace=host),
-        lambda: ops.decode_rope_attention(row, table, table, kv, query_heads=4, query_start=0, key_start=256,
-                                          value_start=512, valid=1024, workspace=host),
-        lambda: ops.w4_matmul(x, packed, scales, 64, workspace=host),
-        lambda: ops.w4_matmul_gate_up(x, packed, scales, packed, scales, 64, workspace=host),
-        lambda: ops.matmul_residual_norm(x, packed, scales, 64, weight.expand(8, 768).contiguous(), weight, 1e-6,
-                                         workspace=host),
 @pytest.mark.parametrize("splits", [39, 40, 41, 55, 56, 57, 72, 188])
 @pytest.mark.parametrize("dim", [64, 128])
 def test_merge_of_any_number_of_splits(dim, splits):
@@ -795,6 +776,25 @@ def test_merge_of_any_number_of_splits(dim, splits):
     assert bool(((got.double() - want).abs() <= 1e-5 + 2.0 ** -8 * want.abs() + 2e-4 * want.abs().amax()).all())
 
 
+def test_workspaces_in_host_memory_are_refused():
+    """Refused by the wrappers before anything is launched: the kernels would store to a host address."""
+
+    from aotolith_amd import ops
+
+    host = torch.zeros(1 << 20, dtype=torch.uint8)
+    q = torch.zeros(1, 4, 64, dtype=torch.bfloat16, device="cuda")
+    kv = torch.zeros(2, 1, 4, 1024, 64, dtype=torch.bfloat16, device="cuda")
+    row, table = torch.zeros(1, 12 * 64, dtype=torch.bfloat16, device="cuda"), kv[0, 0, 0]
+    packed, scales = ops.quantize(torch.zeros(768, 256, dtype=torch.bfloat16, device="cuda"), 64, 4)
+    x, weight = table[:8, :1].expand(8, 256).contiguous(), torch.zeros(768, dtype=torch.bfloat16, device="cuda")
+    calls = [
+        lambda: ops.decode_attention(q, kv[0], kv[1], valid=1024, workspace=host),
+        lambda: ops.decode_rope_attention(row, table, table, kv, query_heads=4, query_start=0, key_start=256,
+                                          value_start=512, valid=1024, workspace=host),
+        lambda: ops.w4_matmul(x, packed, scales, 64, workspace=host),
+        lambda: ops.w4_matmul_gate_up(x, packed, scales, packed, scales, 64, workspace=host),
+        lambda: ops.matmul_residual_norm(x, packed, scales, 64, weight.expand(8, 768).contiguous(), weight, 1e-6,
+                                         workspace=host),
         lambda: ops.matmul_qkv_rope(x, packed, scales, 64, torch.arange(8, device="cuda"), table, table,
                                     kv[:, :, :4], query_heads=4, kv_heads=4, head_dim=64, slot0=0, workspace=host),
     ]

@@ -368,10 +368,11 @@ def test_gemv_finish_refuses_other_shapes():
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("source", ["bf16", "f32"])
 @pytest.mark.parametrize("n,k,group", [(1, 8, 8), (257, 8, 8), (129, 64, 16), (33, 96, 32), (17, 1024, 64),
-                                       (9, 1280, 256), (5, 1536, 512), (2, 4096, 1024), (7, 240, 24)])
+                                       (9, 1280, 256), (5, 1536, 512), (2, 4096, 1024), (7, 240, 24),
+                                       (512, 512, 8), (513, 512, 8), (2048, 512, 8), (2049, 512, 8)])
 def test_packers_at_the_edges_of_their_units(n, k, group, source, bits):
     """Unit counts around a block's 1024, one to 64 lanes a group, groups the coalesced form leaves out
-    (over 512, not a power of two), zero, infinite and NaN groups, and a base that is not 16-byte aligned."""
+    (over 512, not a power of two, 8 in up to 2^18 f32 or 2^20 bf16 weights), zero, infinite and NaN groups, and a base that is not 16-byte aligned."""
 
     from oracle.quant import pack_weight_bits_bf16
 
