@@ -925,14 +925,21 @@ float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits
 }
 
 // The modelled instance and split count (explicit codes), or false where the fixed plan (`tile`, `splits`
-// as it resolves, with 1 or more slices) is within the promise (a share of its time) of the model's best.
-bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail, bool gate, int head_dim, float promise,
+// as it resolves, with 1 or more slices) is within 20% (10% by the rules before the `present` ones) of the model's
+// best. Where the dequant-once forms can run, the 16x16 ones of a single projection are no candidates past 256 rows
+// and K = 2048: there the model has them at 0.7 to 0.8 of their time (64 x 64 blocks in two slices, fixed plan ->
+// those -> the dequant-once form: 300 x 4096 -> 4096 35.4 -> 37.7 -> 29.6 us, 257 x 3584 -> 4608 35.0 -> 32.8 -> 27.1;
+// at K = 896, 257 -> 8192 25.8 -> 15.5 -> 19.9). Over 72 shapes whose plan this changes, times are 0.75 of the fixed
+// plan's, 1.01 at worst; with the 16x16 candidates 0.84 and 1.07.
+bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail, bool gate, int head_dim, bool present,
                    int* tile, int* splits) {
   const bool paired = tail == kTailPaired;
+  const float promise = present ? 0.8f : 0.9f;
   const GemmCost* table = paired ? (bits == 4 ? kCostPaired4 : kCostPaired8) : (bits == 4 ? kCost4 : kCost8);
   const int count = (int)(paired ? (bits == 4 ? sizeof(kCostPaired4) : sizeof(kCostPaired8))
                                  : (bits == 4 ? sizeof(kCost4) : sizeof(kCost8))) / (int)sizeof(GemmCost);
   const bool small_offsets = (long long)M * K * 2 < (1LL << 31) && (long long)N * K / 8 * bits < (1LL << 31);
+  const bool once = pow2_even && small_offsets && !gate, long_rows = present && once && !paired && M > 256 && K > 2048;
   const GemmPlan fixed = gemm_plan(M, N, K, *tile, *splits, paired);
   float best = 0.f, now = 0.f;
   int best_tile = 0, best_splits = 0;
@@ -941,7 +948,7 @@ bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail,
     const GemmCost& c = table[i];
     if (c.code == 10 * fixed.tn + fixed.tm) now = modelled_cost(c, bits, M, N, K, fixed.splits, tail, head_dim);
     if (wide_code(c.code) && (!pow2_even || K % 128 != 0)) continue;
-    if (lds_code(c.code) && (!pow2_even || !small_offsets || gate)) continue;
+    if (lds_code(c.code) ? !once : !wide_code(c.code) && long_rows) continue;
     const int steps = K / (lds_code(c.code) ? 64 : 128);
     for (int s : slices) {
       if (s > most && (s > 1 || lds_split_code(c.code))) break;
@@ -985,7 +992,7 @@ bool automatic_model(int bits, int M, int N, int K, int group, GemmTail tail, bo
     return e.chosen;
   }
   int t = *tile, s = *splits;
-  const bool chosen = modelled_plan(bits, M, N, K, pow2_even, tail, gate, head_dim, present ? 0.8f : 0.9f, &t, &s);
+  const bool chosen = modelled_plan(bits, M, N, K, pow2_even, tail, gate, head_dim, present, &t, &s);
   if (known_head) e = {{a, b}, t, s, chosen, true};
   if (chosen) *tile = t, *splits = s;
   return chosen;

@@ -576,6 +576,32 @@ def test_automatic_codes_at_wide_outputs_of_few_rows(m, n, k, bits):
                        matmul(x, packed, scales, 64, bias=bias, tile=14, splits=1))
 
 
+@pytest.mark.parametrize("m,n,k,bits,group,once", [
+    (257, 1152, 3584, 4, 64, True), (256, 1152, 3584, 4, 64, True), (300, 4096, 4096, 4, 64, True),
+    (257, 896, 2560, 8, 64, True), (300, 8192, 1536, 4, 64, False), (300, 8192, 2048, 4, 64, False),
+    (300, 4096, 4096, 4, 4096, False)])
+def test_modelled_plans_on_both_sides_of_their_long_rows(m, n, k, bits, group, once):
+    """Past 256 rows and K = 2048 a modelled plan is a dequant-once one where such can run (not with a gate epilogue or
+    one group a row); shorter rows keep the 16x16 instance. Against the 16x16 kernel's fixed plan: an f32 sum of K
+    products in another order, then one bf16 rounding."""
+
+    from aotolith_amd import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    packed, scales = ops.quantize((torch.randn(n, k, generator=gen, device="cuda") * 0.02).bfloat16(), group, bits)
+    x = torch.randn(m, k, generator=gen, device="cuda").bfloat16()
+    matmul = ops.w4_matmul if bits == 4 else ops.w8_matmul
+    with ops.recording_launches() as take:
+        take()
+        got = matmul(x, packed, scales, group).double()
+        assert take()[0].startswith(f"aoto_w{bits}_gemm_d") == once
+        matmul(x, packed, scales, group, gate=got.bfloat16())
+        assert not take()[0].startswith(f"aoto_w{bits}_gemm_d")
+    want = matmul(x, packed, scales, group, tile=28, splits=1).double()
+    size = (x.double().abs() @ torch.full((k, 1), 0.02, dtype=torch.float64, device="cuda")).amax()
+    assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + k * 2.0 ** -24 * 4 * size).all())
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("m,n,k", [(400, 8192, 1536), (400, 8192, 3584), (511, 8192, 4096)])
 def test_automatic_codes_run_without_a_workspace_where_the_fixed_plan_needs_none(m, n, k, bits):
