@@ -843,10 +843,6 @@ GemmPlan gemm_plan(int M, int N, int K, int tile, int splits, bool paired) {
   return p;
 }
 
-}  // namespace
-
-namespace {
-
 // What follows the product in its launch or behind it.
 // (kTailNorm also without the norm: the residual + norm form and the plain one then share their plan, and
 // with it every bit of the product)
@@ -1043,10 +1039,6 @@ size_t modelled_workspace(int M, int N, int K, GemmTail tail, int head_dim) {
 
 // Plans of a code object that an earlier build stored stay that build's.
 bool models_plans() { return has_kernel("aoto_w8_gemm_d8c2w2x2_split"); }
-
-}  // namespace
-
-namespace {
 
 // Automatic codes where the scales start at an odd element: the 16x16 kernel, which reads them one by one (the
 // dequant-once and wide kernels read aligned pairs), with its own split count as far as a workspace of `room`

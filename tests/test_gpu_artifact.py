@@ -190,10 +190,10 @@ def test_decode_gemvs_over_an_earlier_code_object_keep_its_kernels():
 
 
 def test_plan_rules_are_those_of_the_code_object():
-    """Paired GEMVs of short int4 rows and of the widest int8 layout leave the staged layouts for wide outputs, and a
-    modelled GEMM has to promise a fifth, and 16 query heads over 2048 keys keep a block each - with a code object of
-    this build; one whose mark is missing (its name changed
-    in the symbol tables) keeps the earlier lines, as the selections stored with it say."""
+    """Paired GEMVs of short int4 rows and of the widest int8 layout leave the staged layouts for wide outputs, a modelled
+    GEMM has to promise a fifth, and 16 query heads over 2048 keys keep a block each - with a code object of this build;
+    one whose mark is missing (its name changed in the symbol tables) keeps the earlier lines, as the selections stored
+    with it say."""
 
     from aotolith_amd import _lib, ops
 
