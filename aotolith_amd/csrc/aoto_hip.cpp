@@ -857,8 +857,8 @@ enum GemmTail { kTailNorm, kTailRope, kTailPaired };
 // Instances whose staging leaves one block to a CU pay whole rounds of 256. The constants are least squares
 // over 370 measured shapes (7 to 14 (N, K) pairs from 896 to 14336, 10 to 15 row counts from 17 to 2048, every
 // tile and 1 to 8 slices, both widths; log error of the near-best plans 0.08 to 0.10; the measurements are not
-// kept). The model's choice replaces the fixed plan's where it promises 20% less, twice that error: at 10% some
-// plans it picked were slower (511 x 8960 -> 1536 35.4 -> 39.5 us, 1500 x 896 -> 4864 28.7 -> 31.8, kept now).
+// kept). The model's choice replaces the fixed plan's where it promises 10% less, or 20%, twice that error, where its
+// picks were slower with less (modelled_plan; 1500 x 896 -> 4864 28.7 -> 31.8 us, kept now).
 // Over 264 GEMMs of 12 (N, K) pairs and 17 to 2048 rows, both widths, times are 0.68 of the fixed plan's in the 100
 // that the model replaces, 1.03 at worst, and 1.11 of those of the best instance and split tried.
 struct GemmCost {
@@ -921,8 +921,11 @@ float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits
 }
 
 // The modelled instance and split count (explicit codes), or false where the fixed plan (`tile`, `splits`
-// as it resolves, with 1 or more slices) is within 20% (10% by the rules before the `present` ones) of the model's
-// best. Where the dequant-once forms can run, the 16x16 ones of a single projection are no candidates past 256 rows
+// as it resolves, with 1 or more slices) is near the model's best: within 10%, and without RoPE by the `present` rules
+// 20% where the model flatters its pick: a wide instance, a 16x16 one over rows longer than 2048, a dequant-once one in
+// one slice or, over rows longer than 6144, of 32 or 64 columns (260 shapes with a promise of 10 to 22%: 16x16 picks
+// up to 1.24 of the fixed plan's time, those narrow dequant-once ones up to 1.18, the 128-column ones 0.67 to 0.91,
+// RoPE 0.74 to 0.98). Where the dequant-once forms can run, the 16x16 ones of a single projection are no candidates past 256 rows
 // and K = 2048: there the model has them at 0.7 to 0.8 of their time (64 x 64 blocks in two slices, fixed plan ->
 // those -> the dequant-once form: 300 x 4096 -> 4096 35.4 -> 37.7 -> 29.6 us, 257 x 3584 -> 4608 35.0 -> 32.8 -> 27.1;
 // at K = 896, 257 -> 8192 25.8 -> 15.5 -> 19.9). Over 72 shapes whose plan this changes, times are 0.75 of the fixed
@@ -930,7 +933,6 @@ float modelled_cost(const GemmCost& c, int bits, int M, int N, int K, int splits
 bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail, bool gate, int head_dim, bool present,
                    int* tile, int* splits) {
   const bool paired = tail == kTailPaired;
-  const float promise = present ? 0.8f : 0.9f;
   const GemmCost* table = paired ? (bits == 4 ? kCostPaired4 : kCostPaired8) : (bits == 4 ? kCost4 : kCost8);
   const int count = (int)(paired ? (bits == 4 ? sizeof(kCostPaired4) : sizeof(kCostPaired8))
                                  : (bits == 4 ? sizeof(kCost4) : sizeof(kCost8))) / (int)sizeof(GemmCost);
@@ -957,6 +959,9 @@ bool modelled_plan(int bits, int M, int N, int K, bool pow2_even, GemmTail tail,
       }
     }
   }
+  const bool narrow = best_tile != 815 && best_tile != 825 && best_tile != 845;
+  const bool loose = lds_code(best_tile) ? best_splits == 1 || (narrow && K > 6144) : wide_code(best_tile) || K > 2048;
+  const float promise = present && loose && tail != kTailRope ? 0.8f : 0.9f;
   if (best_tile == 0 || now == 0.f || best >= promise * now) return false;
   *tile = best_tile;
   *splits = best_splits;

@@ -147,7 +147,7 @@ int aoto_hip_w4_gemv(const void* x, const int32_t* words, const void* scales,
  * single projection of 32-256 rows with K >= 2048 and no RoPE epilogue the split form (814
  * where that gives >= 64 column blocks, else 813), else the wide kernel from M >= 512 when
  * K % 256 == 0 (group <= 128), else the instance and split count of a cost model fitted to
- * measured times where it promises 20% less than the 16x16 kernel (not for a paired gate/up or
+ * measured times where it promises 10 to 20% less than the 16x16 kernel (not for a paired gate/up or
  * N > K at M <= 256, nor q/k/v on 32-row blocks), else the 16x16 kernel. The workspace queries
  * cover that choice for either code width and every group (at most 8 slices, 6 paired, and
  * 32 MiB); without a workspace the model's split plans are left out. splits: 0 chooses (small

@@ -579,7 +579,7 @@ def test_automatic_codes_at_wide_outputs_of_few_rows(m, n, k, bits):
 @pytest.mark.parametrize("m,n,k,bits,group,once", [
     (257, 1152, 3584, 4, 64, True), (256, 1152, 3584, 4, 64, True), (300, 4096, 4096, 4, 64, True),
     (257, 896, 2560, 8, 64, True), (300, 8192, 1536, 4, 64, False), (300, 8192, 2048, 4, 64, False),
-    (300, 4096, 4096, 4, 4096, False)])
+    (300, 4096, 4096, 4, 4096, False), (1503, 1872, 3968, 4, 32, True), (511, 1536, 8960, 4, 64, False)])
 def test_modelled_plans_on_both_sides_of_their_long_rows(m, n, k, bits, group, once):
     """Past 256 rows and K = 2048 a modelled plan is a dequant-once one where such can run (not with a gate epilogue or
     one group a row); shorter rows keep the 16x16 instance. Against the 16x16 kernel's fixed plan: an f32 sum of K
