@@ -859,8 +859,8 @@ enum GemmTail { kTailNorm, kTailRope, kTailPaired };
 // tile and 1 to 8 slices, both widths; log error of the near-best plans 0.08 to 0.10; the measurements are not
 // kept). The model's choice replaces the fixed plan's where it promises 10% less, or 20%, twice that error, where its
 // picks were slower with less (modelled_plan; 1500 x 896 -> 4864 28.7 -> 31.8 us, kept now).
-// Over 264 GEMMs of 12 (N, K) pairs and 17 to 2048 rows, both widths, times are 0.68 of the fixed plan's in the 100
-// that the model replaces, 1.03 at worst, and 1.11 of those of the best instance and split tried.
+// Over 264 GEMMs of 12 (N, K) pairs and 17 to 2048 rows, both widths, times are 0.68 of the fixed plan's in the 103
+// that the model replaces, 1.04 at worst, and 1.11 of those of the best instance and split tried.
 struct GemmCost {
   int code;
   float launch, latency, rate;
